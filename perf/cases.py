@@ -181,3 +181,81 @@ def tolerance(case):
     #             1/area of boxes a fraction of a pixel thin)
     #   float16   2.1e-4 and bfloat16 1.7e-3: one rounding of the output or the input's gradient
     return {"rel": {"float32": 6e-5, "float16": 8e-4, "bfloat16": 7e-3}[case["dtype"]]}
+
+
+def _overlap(lo, hi, n, dev):
+    # [i, k]: how much of pixel k the box [i + lo, i + hi + 1] covers
+    i = torch.arange(n, dtype=torch.float64, device=dev)[:, None]
+    k = torch.arange(n, dtype=torch.float64, device=dev)[None, :]
+    return (torch.minimum(i + hi + 1, k + 1) - torch.maximum(i + lo, k)).clamp_(min=0)
+
+
+def _edge(offset, n, dev):
+    # for each i the pixel i + offset an edge lies in, and whether there is such a pixel
+    e = torch.arange(n, device=dev) + offset
+    return e.clamp(0, n - 1), ((e >= 0) & (e < n)).double()
+
+
+def _pixel_bounds(module, clip_to):
+    """The box bounds in pixels, as float32 holds them, after the projection that a training-mode
+    forward and ``eval()`` apply to the stored bounds."""
+    bounds = []
+    min_size = 1.001 if module.exact else 2.001
+    for lo, hi, factor, size in ((module.x_min, module.x_max, module.reparametrization_h, clip_to[0]),
+                                 (module.y_min, module.y_max, module.reparametrization_w, clip_to[1])):
+        lo, hi = (p.detach().double().clamp(-(size + 1) / factor, (size - 1) / factor) for p in (lo, hi))
+        gap = (min_size - 0.9999) / factor
+        mean = (0.5 * (lo + hi)).float().double()
+        thin = lo + gap > hi
+        lo, hi = torch.where(thin, mean - 0.5 * gap, lo), torch.where(thin, mean + 0.5 * gap, hi)
+        bounds += [(p.float() * factor).double() for p in (lo, hi)]
+    return bounds
+
+
+def exact(case, seed):
+    """``run``'s outputs in float64: every box filter as two dense matrices of pixel overlaps."""
+    state = prepare(case, seed)
+    module, x = state["module"], state["x"].detach().double()
+    B, C, F, h, w = (case[k] for k in "BCFhw")
+    dev, train = x.device, state["mode"] in ("train", "first_layer")
+    bounds = _pixel_bounds(module, (h, w))
+    values = [b.cpu().tolist() for b in bounds]
+    out = torch.empty(B, C * F, h, w, dtype=torch.float64, device=dev)
+    grad_input = torch.zeros_like(x) if state["mode"] == "train" else None
+    grads = [torch.zeros(C, F, dtype=torch.float64, device=dev) for _ in range(4)]
+    for c in range(C):
+        plane = x[:, c].contiguous()
+        for f in range(F):
+            x0, x1, y0, y1 = (v[c][f] for v in values)
+            if not case["exact"]:
+                x0, x1, y0, y1 = math.ceil(x0), math.floor(x1), math.ceil(y0), math.floor(y1)
+            rows, cols = _overlap(x0, x1, h, dev), _overlap(y0, y1, w, dev)
+            scale = 1 / ((x1 - x0 + 1) * (y1 - y0 + 1)) if case["normalize"] else 1.0
+            across = torch.matmul(plane, cols.t().contiguous())
+            result = torch.matmul(rows, across) * scale
+            out[:, c * F + f] = result
+            if not train:
+                continue
+            g = state["grad"][:, c * F + f].double()
+            if grad_input is not None:
+                grad_input[:, c] += torch.matmul(rows.t().contiguous(), torch.matmul(g, cols)) * scale
+            down = torch.matmul(rows, plane)
+            total = (g * result).sum()
+            for n, (value, offset, sign, source, dim) in enumerate((
+                    (x0, math.ceil(x0) - 1, -1, across, 1), (x1, math.floor(x1) + 1, 1, across, 1),
+                    (y0, math.ceil(y0) - 1, -1, down, 2), (y1, math.floor(y1) + 1, 1, down, 2))):
+                at, there = _edge(offset, source.size(dim), dev)
+                there = there[:, None] if dim == 1 else there
+                d = sign * scale * (g * source.index_select(dim, at) * there).sum()
+                if case["normalize"]:
+                    d = d - sign * total / ((x1 - x0 + 1) if dim == 1 else (y1 - y0 + 1))
+                grads[n][c, f] = d * (module.reparametrization_h if dim == 1 else module.reparametrization_w)
+    if state["mode"] == "fused":
+        out = out * state["scale"].double().view(1, -1, 1, 1) + state["shift"].double().view(1, -1, 1, 1)
+        return (out + state["residual"].double()).clamp_(min=0)
+    if state["mode"] == "infer":
+        return out
+    result = {"out": out, "x_min": grads[0], "x_max": grads[1], "y_min": grads[2], "y_max": grads[3]}
+    if grad_input is not None:
+        result["grad_input"] = grad_input
+    return result
