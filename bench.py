@@ -40,21 +40,25 @@ PREWARM_MAX_S = 1.5 # upper bound on the untimed clock-up phase after --warmup
 RANKING_STEPS = 3   # untimed eager steps per kernel name while the per-kernel times are taken
 # every kernel a training step launches ("clip" is the parameter projection, which shares its
 # launch with the marking of the single-pass integral image's hand-over words)
-TIMED_KERNELS = ("grad_output_stream", "band_scan", "band_colsum", "forward_rows", "grad_input_cols", "clip")
+TIMED_KERNELS = ("grad_output_stream", "band_scan", "band_colsum", "forward_rows", "grad_input_cols",
+                 "grad_input_taps", "clip")
 METRIC = "BoxConv2d fwd+bwd ms/iter + effective HBM GB/s (% peak) at 2x16ch 512x1024 fp32"
 
 
-def kernel_algorithmic_bytes(ab, elem=4):
+def kernel_algorithmic_bytes(ab, elem=4, from_snapshots=False):
     """Algorithmic bytes moved by ONE launch of each kernel at a given workload: the share of the
-    step's data flow that the kernel is responsible for (each is launched once per step)."""
+    step's data flow that the kernel is responsible for (each is launched once per step).
+    from_snapshots: grad_input_taps forms the input's gradient from grad_output itself, and the
+    grad_output pass writes no integral of it."""
     return {
         "clip": 0,                                               # kilobytes of box parameters and marker words
         # read grad_output and the input's integral, write the (band-local) integral of grad_output
-        "grad_output_stream": elem * (ab["n_out"] + ab["n_int"] + ab["n_gint"]),
+        "grad_output_stream": elem * (ab["n_out"] + ab["n_int"] + (0 if from_snapshots else ab["n_gint"])),
         "band_scan": elem * (ab["n_in"] + ab["n_int"]),          # read input, write its integral
         "band_colsum": elem * ab["n_in"],                        # pre-pass over the input
         "forward_rows": elem * (ab["n_int"] + ab["n_out"]),      # read integral, write output
         "grad_input_cols": elem * (ab["n_gint"] + ab["n_in"]),   # read integral of grad_output, write grad_input
+        "grad_input_taps": elem * (ab["n_out"] + ab["n_in"]),    # read grad_output, write grad_input
     }
 
 
@@ -465,7 +469,7 @@ def main():
     # (rows wider than 2048 columns run the grad_output pass as two launches: its bytes are then
     # priced against the time of both)
     launches_per_step = max(per_kernel[dominant][1], 1)
-    bytes_per_launch = kernel_algorithmic_bytes(ab)[dominant] / launches_per_step
+    bytes_per_launch = kernel_algorithmic_bytes(ab, from_snapshots=per_kernel["grad_input_taps"][1] > 0)[dominant] / launches_per_step
     avg_launch_s = dom_ms / 1e3 / max(dom_launches, 1)
     achieved = bytes_per_launch / avg_launch_s / 1e9
 

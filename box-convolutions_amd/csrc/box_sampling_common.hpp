@@ -49,7 +49,16 @@ struct SampleArgs {
                           // band-local integral that are stored with the ordinary cache policy
     int m_bands;          // rows of M interleaved over this many bands (0: rows in their natural order)
     int m_shift;          // log2 of the rows per band of M (interleaved layout only)
+    int snap_shift;       // snapshots only: log2 of the output rows per group of grad_input_taps_kernel
+    int snap_groups;      // snapshots only: such groups per plane
+    int snap_bands;       // snapshots only: bands of the grad_output pass per plane
 };
+
+// Snapshots of the column sums of grad_output (grad_input_taps_kernel has the math): one row of w
+// zeros, then per (plane, filter) the rows for the upper edge of the mirrored box, the rows for its
+// lower edge (one per group of output rows each), and the sum of every band.
+template <class T>
+__host__ __device__ __forceinline__ int snapshot_rows(const SampleArgs<T>& a) { return 2 * a.snap_groups + a.snap_bands; }
 
 namespace {
 

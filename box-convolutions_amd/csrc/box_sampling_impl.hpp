@@ -923,6 +923,40 @@ __device__ __forceinline__ void load4_dword_aligned(const float* p, float (&v)[4
     v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
 }
 
+// LDS layout of a row pair for lanes that own 4 consecutive columns: column c is element c / 4 of
+// plane c % 4. A lane's taps are 5 adjacent columns that start anywhere; tap m of all lanes then
+// lies in one plane at lane-consecutive places, so every access of a wave is 512 contiguous bytes
+// (columns side by side, a lane's neighbour sits 32 bytes away and an access takes twice as many
+// LDS cycles: 512 x 1024, 16 x 8 planes, 150 cycles per wave and row pair, 87 of them conflicts).
+// kQuadPad elements of zeros in front of every plane and behind it stand for the columns outside.
+constexpr int kQuadPad = 2;
+__host__ __device__ constexpr int quad_plane(int nt) { return nt + 64; }   // a multiple of 64 elements: two planes per access
+// Byte offsets of the taps at columns 4 * tid + first + m, m < 4 (m = 4: one element after m = 0).
+struct TapRun {
+    unsigned at[4];
+};
+template <int PLANE>
+__device__ __forceinline__ TapRun tap_run(int tid, int first, int quads) {
+    const int plane = first & 3, place = clampi(tid + (first >> 2), -kQuadPad, quads) + kQuadPad;
+    TapRun t;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        t.at[m] = static_cast<unsigned>(((plane + m) & 3) * PLANE + ((plane + m) >> 2) + place) * static_cast<unsigned>(sizeof(RowPair<float>));
+    return t;
+}
+__device__ __forceinline__ void read_taps(const RowPair<float>* row, const TapRun& t, RowPair<float> (&v)[5]) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) v[m] = *at_bytes(row, t.at[m]);
+    v[4] = at_bytes(row, t.at[0])[1];
+}
+
+// What the kernel leaves for the gradient w.r.t. the input.
+enum StreamMode {
+    kStreamParams,      // nothing: the parameter sums alone
+    kStreamScan,        // the column workspace M
+    kStreamSnapshots,   // sums of grad_output's rows at the rows where grad_input_taps_kernel starts
+};
+
 // Two waves per SIMD on purpose, although the registers would allow three: with three, more
 // workgroups are resident per XCD than share one integral plane of the input, two planes compete
 // for its L2, and the kernel gets slower (226 against 217 us at 512 x 1024).
@@ -930,21 +964,24 @@ __device__ __forceinline__ void load4_dword_aligned(const float* p, float (&v)[4
 // share a CU, where at two per SIMD two, three or two of its eight wave slots would stay empty.
 // Measured at three waves: 480 x 640 170 -> 149 us; rows of 960 and 1000 columns, four waves with
 // idle lanes, got slower with three per SIMD like the full rows: 230 -> 235 us.)
-// SCAN = false: the parameter sums only (the input needs no gradient, as in a network's first
+// kStreamParams: the parameter sums only (the input needs no gradient, as in a network's first
 // layer): no suffix sums, no column workspace, half the registers; four waves per SIMD then (no
-// column workspace competes for the L2).
-template <class TG, int NT, bool EXACT, bool FULL, bool SCAN = true>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, !SCAN ? 4 : (NT == 192 || NT == 320 || NT == 384) ? 3 : 2)))
+// column workspace competes for the L2). kStreamSnapshots: the same plus one addition per element;
+// told to fit four waves, since left alone the compiler takes one to five registers too many for
+// them (three waves per SIMD: 168 against 140 us at 512 x 1024).
+template <class TG, int NT, bool EXACT, bool FULL, int MODE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MODE == kStreamSnapshots ? 4 : 2, MODE != kStreamScan ? 4 : (NT == 192 || NT == 320 || NT == 384) ? 3 : 2)))
 grad_output_stream_consec_kernel(SampleArgs<float> a) {
     using T = float;
+    constexpr bool SCAN = MODE == kStreamScan, SNAP = MODE == kStreamSnapshots;
     constexpr int K = 4;
-    constexpr int kPad = 8;                          // zero pairs in front of and behind a row in LDS
-    constexpr int GLEN = K * NT + 2 * kPad;
+    constexpr int PLANE = quad_plane(NT);
     constexpr int WAVES = NT / 64;
-    constexpr bool MERGED = NT <= 256;
+    constexpr bool MERGED = !SCAN || NT <= 256;
+    static_assert(MERGED || !SNAP, "the running sums are taken where the merged pass publishes its rows");
     struct alignas(16) WaveSums { T tot0, tot1, tail0, tail1; };
     struct alignas(16) LastColumn { T v, dt, db, unused; };      // V, DT, DB at column w
-    __shared__ __align__(16) RowPair<T> grow[2][GLEN];
+    __shared__ __align__(16) RowPair<T> grow[2][K][PLANE];
     __shared__ __align__(16) T delta[K * NT];
     __shared__ WaveSums wsum[2][WAVES];
     __shared__ LastColumn xw[2][2];
@@ -967,7 +1004,10 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     const int owner = FULL ? NT - 1 : w / K - 1;     // the lane whose last column is column w
 
     const BoxOfWorkgroup<T> bx = load_box(a.prm, k_par);
-    const BoxSplit<T> s = split_grad_params(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
+    BoxSplit<T> s = split_grad_params(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
+    // (the same in every lane: row addresses then are scalar arithmetic)
+    s.xlo = __builtin_amdgcn_readfirstlane(s.xlo); s.xhi = __builtin_amdgcn_readfirstlane(s.xhi);
+    s.ylo = __builtin_amdgcn_readfirstlane(s.ylo); s.yhi = __builtin_amdgcn_readfirstlane(s.yhi);
     const BoxSplit<T> sm = split_grad_input(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
     const int ylo_m = 1 - sm.yhi, yhi_m = 1 - sm.ylo;
     const bool own_w = ylo_m != s.ylo || yhi_m != s.yhi;                        // workgroup-uniform
@@ -1007,13 +1047,27 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     load_g(i0 + 1, g1);
 
     // pads of both LDS rows, row 0 of the column workspace
-    if (tid < 2 * kPad) {
-        const int e = tid < kPad ? tid : K * NT + tid;
-        grow[0][e] = RowPair<T>{T(0), T(0)};
-        grow[1][e] = RowPair<T>{T(0), T(0)};
+    if (tid < 2 * K * 2 * kQuadPad) {
+        const int plane = tid / (2 * kQuadPad), e = tid % (2 * kQuadPad);
+        grow[plane / K][plane % K][e < kQuadPad ? e : NT + e] = RowPair<T>{T(0), T(0)};
     }
     if (SCAN && band == 0)
         for (int c = tid; c < mpitch; c += NT) mrows[c] = T(0);
+    if (SNAP && vid == 0)                            // the row of zeros in front of the snapshots
+        for (int c = tid; c < w; c += NT) a.dst[c] = T(0);
+    T* const snap = a.dst + w + pf * static_cast<int64_t>(snapshot_rows(a)) * w;
+    const int snap_lo = __builtin_amdgcn_readfirstlane(sm.xlo), snap_hi = __builtin_amdgcn_readfirstlane(sm.xhi);
+    // the sum of the band's rows above integral row r, where grad_input_taps_kernel will want it
+    auto keep_snapshot = [&](int r, const T (&sum)[K]) {
+        const Quad<T> q{{sum[0], sum[1], sum[2], sum[3]}};
+        const int mask = (1 << a.snap_shift) - 1, ut = r - snap_lo, ub = r - snap_hi;
+        if ((ut & mask) == 0 && ut >= 0 && (ut >> a.snap_shift) < a.snap_groups)
+            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(ut >> a.snap_shift) * w), 4u * cl) = q;
+        if ((ub & mask) == 0 && ub >= 0 && (ub >> a.snap_shift) < a.snap_groups)
+            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(a.snap_groups + (ub >> a.snap_shift)) * w), 4u * cl) = q;
+        if (r == i1)
+            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(2 * a.snap_groups + band) * w), 4u * cl) = q;
+    };
 
     auto tail_weight = [&](int j, int ylo, int yhi, T fylo, T fyhi) {
         const T one = T(1);
@@ -1022,11 +1076,9 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
              - (EXACT ? (one - fylo) : one) * T(j > w - ylo)
              - (EXACT ? fylo : T(0)) * T(j > w - ylo + 1);
     };
-    // first element (with the front pad counted in) of the runs of 5 row pairs that hold the taps
-    // of the lane's columns: right run g[c0 - yhi ..], left run g[c0 + 1 - ylo ..]
-    auto run_start = [&](int first) { return clampi(first, -kPad, w) + kPad; };
-    const int er = run_start(c0 - s.yhi), el = run_start(c0 + 1 - s.ylo);
-    const int er_m = run_start(c0 - yhi_m), el_m = run_start(c0 + 1 - ylo_m);
+    // taps of the lane's columns: right run g[c0 - yhi ..], left run g[c0 + 1 - ylo ..]
+    const int quads = FULL ? NT : w / K;
+    const TapRun er = tap_run<PLANE>(tid, -s.yhi, quads), el = tap_run<PLANE>(tid, 1 - s.ylo, quads);
     bool wave_has_tail = false;
     {
         T d[K];
@@ -1039,8 +1091,10 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     }
     wave_has_tail = __any(wave_has_tail) != 0 || own_w;                          // wave-uniform
     const int j_ymax = w - s.yhi, j_ymin = w - s.ylo + 1;
-    const int idx_ymax = (j_ymax >= 0 && j_ymax < w) ? j_ymax + kPad : 0;        // element 0 is a zero pad
-    const int idx_ymin = (j_ymin >= 0 && j_ymin < w) ? j_ymin + kPad : 0;
+    auto place_of = [&](int j) {                     // element 0 is a zero pad
+        return j >= 0 && j < w ? (j & (K - 1)) * PLANE + j / K + kQuadPad : 0;
+    };
+    const int idx_ymax = place_of(j_ymax), idx_ymin = place_of(j_ymin);
 
     double total[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     T colacc[K];
@@ -1065,9 +1119,8 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             _Pragma("unroll")                                                                       \
             for (int k = 0; k < K; ++k) { GA[k] = T(0); GB[k] = T(0); }                             \
         }                                                                                           \
-        Quad<T>* dst = reinterpret_cast<Quad<T>*>(&grow[FL][kPad + c0]);                            \
-        dst[0] = Quad<T>{{GA[0], GB[0], GA[1], GB[1]}};                                             \
-        dst[1] = Quad<T>{{GA[2], GB[2], GA[3], GB[3]}};                                             \
+        _Pragma("unroll")                                                                           \
+        for (int k = 0; k < K; ++k) grow[FL][k][kQuadPad + tid] = RowPair<T>{GA[k], GB[k]};         \
         TL0 = T(0); TL1 = T(0);                                                                     \
         if (wave_has_tail) {                                                                        \
             const Quad<T> dq = *reinterpret_cast<const Quad<T>*>(&delta[c0]);                       \
@@ -1087,9 +1140,24 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
         }                                                                                           \
     }
 
+    // grad_output rows i, i+1 (cleared past the band) into the running column sums; done as soon as
+    // the rows are in LDS, so that their registers are free again
+    auto accumulate = [&](int i, const T (&ga)[K], const T (&gb)[K]) {
+        if (!lane_in) return;
+#pragma unroll
+        for (int k = 0; k < K; ++k) colacc[k] += ga[k];
+        keep_snapshot(i + 1, colacc);
+        if (i + 1 < i1) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) colacc[k] += gb[k];
+            keep_snapshot(i + 2, colacc);
+        }
+    };
+
     T tl0 = T(0), tl1 = T(0);
     if (MERGED) {
         BOXCONV_PUBLISH_CONSEC(0, i0, g0, g1, ta, t0, t1, bc, b1, b2, tl0, tl1)
+        if (SNAP) accumulate(i0, g0, g1);
         __syncthreads();
     }
 
@@ -1107,7 +1175,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             BOXCONV_PUBLISH_CONSEC(FLIP, i, g0, g1, ta, t0, t1, bc, b1, b2, tl0, tl1)
             __syncthreads();                                                 // rows are in LDS
         }
-        const RowPair<T>* G = grow[FLIP];
+        const RowPair<T>* G = grow[FLIP][0];
         T tail0 = tl0, tail1 = tl1;
         T tn0 = T(0), tn1 = T(0);
 
@@ -1115,8 +1183,8 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
         T wq0[K], wq1[K];
         {
             RowPair<T> R[K + 1], L[K + 1];
-#pragma unroll
-            for (int m = 0; m <= K; ++m) { R[m] = G[er + m]; L[m] = G[el + m]; }
+            read_taps(G, er, R);
+            read_taps(G, el, L);
             T sum[5] = {T(0), T(0), T(0), T(0), T(0)};
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -1170,8 +1238,8 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             // rare: the mirrored split cuts the box at other whole pixels; weights and tails of
             // the column workspace from that split
             RowPair<T> R[K + 1], L[K + 1];
-#pragma unroll
-            for (int m = 0; m <= K; ++m) { R[m] = G[er_m + m]; L[m] = G[el_m + m]; }
+            read_taps(G, tap_run<PLANE>(tid, -yhi_m, quads), R);
+            read_taps(G, tap_run<PLANE>(tid, 1 - ylo_m, quads), L);
             tail0 = T(0); tail1 = T(0);
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -1184,7 +1252,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
                 }
                 if (!FULL && !lane_in) { wq0[k] = T(0); wq1[k] = T(0); }
                 const T dlt = lane_in ? tail_weight(c0 + k, ylo_m, yhi_m, sm.fyhi, sm.fylo) : T(0);
-                const RowPair<T> own = G[kPad + c0 + k];
+                const RowPair<T> own = G[k * PLANE + kQuadPad + tid];
                 tail0 += dlt * own.r0;
                 tail1 += dlt * own.r1;
             }
@@ -1213,6 +1281,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             if (lane == 63) wsum[FLIP][wave] = WaveSums{inc0, inc1, wt0, wt1};
         }
         if (MERGED && PREFETCH) BOXCONV_PUBLISH_CONSEC(FLIP ^ 1, i + 2, m0, m1, t1, n0, n1, b2, n2, n3, tn0, tn1)
+        if (SNAP && PREFETCH) accumulate(i + 2, m0, m1);
         __syncthreads();                             // wave totals (and the next pair's rows) visible
         if (SCAN) {
 #pragma unroll
@@ -1474,25 +1543,44 @@ hipError_t grad_input_launch(const T* gint, int band_rows, BoxParams<T> prm, TO*
 // policy (the memory-side cache holds 256 MB; the grad-input kernel reads that part first).
 inline int64_t cached_tail_bytes() { return switches().keep_tail_bytes; }
 
+// Rows that grad_output_stream_consec_kernel takes: a multiple of four columns, 16-byte (16-bit
+// elements: 8-byte) aligned. The workgroup is the smallest one (whole waves) whose lanes, four
+// columns each, cover the row. Only a single wave can be left mostly idle (from two waves on, more
+// than half of the lanes are busy): rows that fill less than three eighths of it stay with the
+// other kernel (measured, 16 x 4 planes of 256 rows: 100 columns 97 -> 86 us, 128: 91 -> 91, 144:
+// 110 -> 90, 260: 138 -> 118, 300: 142 -> 121; but 64 columns 72 -> 83). Rows of exactly 128 columns
+// also stay there: they fill that kernel's two waves at one column per lane with no bounds to check
+// (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us).
+inline int consecutive_threads(int w) { return (w / 4 + 63) / 64 * 64; }
+template <class TG>
+bool stream_consecutive_applies(const TG* grad_out, int w) {
+    if (w % 4 != 0 || w > 2048 || reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) != 0) return false;
+    const RowConfig rc = stream_row_config(w, sizeof(float));
+    const int lanes = w / 4, cnt = consecutive_threads(w);
+    const bool exact_fit = lanes == cnt && (cnt == 64 || cnt == 128 || cnt == 256 || cnt == 512);
+    return switches().stream_consecutive &&
+           (exact_fit || (switches().stream_consecutive_partial && lanes * 8 >= cnt * 3 && !(rc.full && rc.K == 1)));
+}
+
 // The launches of grad_output_stream_consec_kernel (`lanes` busy lanes of a workgroup of `cnt`;
 // SCAN = false: parameter sums only). Its instantiations are translation units of their own
 // (BOXCONV_INST_PART 3 and 4): some hundred kernels that would otherwise double the compile time
 // of the unit with the other variant.
-template <class TG, bool SCAN>
+template <class TG, int MODE>
 hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lanes, int cnt, bool exact,
                                             dim3 grid, hipStream_t stream);
-#if defined(BOXCONV_INST_PART) && (BOXCONV_INST_PART == 3 || BOXCONV_INST_PART == 4)
-template <class TG, bool SCAN>
+#if defined(BOXCONV_INST_PART) && BOXCONV_INST_PART >= 3 && BOXCONV_INST_PART <= 5
+template <class TG, int MODE>
 hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lanes, int cnt, bool exact,
                                             dim3 grid, hipStream_t stream) {
     const size_t lds = 0;                              // the kernel's LDS is statically sized
 #define LAUNCH_GC(NT) \
     if (lanes == NT) { \
-        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, true, SCAN>), grid, dim3(NT), lds, stream, a); \
-        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, true, SCAN>), grid, dim3(NT), lds, stream, a); \
+        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, true, MODE>), grid, dim3(NT), lds, stream, a); \
+        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, true, MODE>), grid, dim3(NT), lds, stream, a); \
     } else { \
-        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, false, SCAN>), grid, dim3(NT), lds, stream, a); \
-        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, false, SCAN>), grid, dim3(NT), lds, stream, a); \
+        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, false, MODE>), grid, dim3(NT), lds, stream, a); \
+        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, false, MODE>), grid, dim3(NT), lds, stream, a); \
     }
     switch (cnt) {
         case 64: LAUNCH_GC(64) break;
@@ -1512,7 +1600,8 @@ hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lane
 template <class T, class TG>
 hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxParams<T> prm,
                                      double* acc, int acc_slots, T* column_workspace,
-                                     const StreamPlan& sp, Dims d, bool exact, hipStream_t stream) {
+                                     const StreamPlan& sp, const SnapshotPlan* snapshots, Dims d,
+                                     bool exact, hipStream_t stream) {
     const int64_t planes_f = d.planes * d.F;
     if (planes_f == 0 || d.hw() == 0) return hipSuccess;
     const bool params = acc != nullptr, scan = column_workspace != nullptr;
@@ -1577,25 +1666,18 @@ hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxPara
     // float rows of a multiple of four columns, the parameter sums wanted (with or without the column
     // workspace), a slot per workgroup for the sums: the kernel with four consecutive columns per lane
     if constexpr (std::is_same<T, float>::value) {
-        const bool aligned = reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) == 0 && d.w % 4 == 0;
-        // the smallest workgroup (whole waves) whose lanes, four columns each, cover the row. Only
-        // a single wave can be left mostly idle (from two waves on, more than half of the lanes
-        // are busy): rows that fill less than three eighths of it stay with the other kernel
-        // (measured, 16 x 4 planes of 256 rows: 100 columns 97 -> 86 us, 128: 91 -> 91, 144:
-        // 110 -> 90, 260: 138 -> 118, 300: 142 -> 121; but 64 columns 72 -> 83). Rows of exactly
-        // 128 columns also stay there: they fill that kernel's two waves at one column per lane
-        // with no bounds to check (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us).
         const int lanes = d.w / 4;
-        const int cnt = (lanes + 63) / 64 * 64;
-        const bool exact_fit = lanes == cnt && (cnt == 64 || cnt == 128 || cnt == 256 || cnt == 512);
-        const bool covers = d.w <= 2048 && lanes >= 1 &&
-                            (exact_fit || (switches().stream_consecutive_partial && lanes * 8 >= cnt * 3 &&
-                                           !(rc.full && rc.K == 1)));
-        if (switches().stream_consecutive && covers && params && acc_slots > 0 && aligned) {
-            if (scan) return grad_output_stream_consec_launch<TG, true>(a, lanes, cnt, exact, grid, stream);
-            return grad_output_stream_consec_launch<TG, false>(a, lanes, cnt, exact, grid, stream);
+        const int cnt = consecutive_threads(d.w);
+        if (params && acc_slots > 0 && stream_consecutive_applies(grad_out, d.w)) {
+            if (snapshots != nullptr) {
+                a.snap_shift = snapshots->shift; a.snap_groups = snapshots->groups; a.snap_bands = sp.nb;
+                return grad_output_stream_consec_launch<TG, kStreamSnapshots>(a, lanes, cnt, exact, grid, stream);
+            }
+            if (scan) return grad_output_stream_consec_launch<TG, kStreamScan>(a, lanes, cnt, exact, grid, stream);
+            return grad_output_stream_consec_launch<TG, kStreamParams>(a, lanes, cnt, exact, grid, stream);
         }
     }
+    if (snapshots != nullptr) return hipErrorInvalidValue;   // (plan_snapshots asks for that kernel only)
     // doubles, two columns per lane on four or eight waves: the kernel that does both jobs needs
     // more registers than a lane has there (512 threads: 50 to 120 of them in scratch memory);
     // either job alone fits. Measured, 16 x 8 planes of 256 rows: 512 columns 212 -> 186 us,

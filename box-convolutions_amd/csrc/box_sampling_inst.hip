@@ -4,7 +4,8 @@
 //   1: the streaming pass over grad_output
 //   2: the gradient w.r.t. the input, and (where T == TG) the gather and finalize launches.
 //   3: (T = float) the streaming pass's variant with consecutive columns per lane;
-//   4: the same variant for the parameter sums alone.
+//   4: the same variant for the parameter sums alone;
+//   5: the same variant with the snapshots that grad_input_taps_kernel reads.
 
 #include "box_sampling_impl.hpp"
 
@@ -13,13 +14,16 @@ namespace boxconv {
 #if BOXCONV_INST_PART == 1
 template hipError_t grad_output_stream_launch<BOXCONV_INST_T, BOXCONV_INST_TG>(
     const BOXCONV_INST_T*, const BOXCONV_INST_TG*, BoxParams<BOXCONV_INST_T>, double*, int, BOXCONV_INST_T*,
-    const StreamPlan&, Dims, bool, hipStream_t);
+    const StreamPlan&, const SnapshotPlan*, Dims, bool, hipStream_t);
 #elif BOXCONV_INST_PART == 3
-template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, true>(const SampleArgs<float>&, int, int, bool,
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamScan>(const SampleArgs<float>&, int, int, bool,
                                                                             dim3, hipStream_t);
 #elif BOXCONV_INST_PART == 4
-template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, false>(const SampleArgs<float>&, int, int, bool,
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamParams>(const SampleArgs<float>&, int, int, bool,
                                                                              dim3, hipStream_t);
+#elif BOXCONV_INST_PART == 5
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamSnapshots>(const SampleArgs<float>&, int, int,
+                                                                                       bool, dim3, hipStream_t);
 #else
 template hipError_t grad_input_launch<BOXCONV_INST_T, BOXCONV_INST_TG>(
     const BOXCONV_INST_T*, int, BoxParams<BOXCONV_INST_T>, BOXCONV_INST_TG*, Dims, bool, bool, hipStream_t,

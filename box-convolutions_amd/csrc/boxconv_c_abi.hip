@@ -389,11 +389,23 @@ int backward_impl(const T* integ, const T* x_min, const T* x_max, const T* y_min
         // one pass over grad_output: parameter sums + column workspace, then grad_input, whose
         // launch finishes the parameter gradients on the side
         const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, sizeof(T));
+        boxconv::SnapshotPlan snap{};
+        if constexpr (std::is_same<T, float>::value)
+            if (need_input && need_params && nout > 0)
+                snap = boxconv::plan_snapshots<TG>(grad_output, sp, d);
         if (int rc = hip_result(boxconv::grad_output_stream_launch<T, TG>(
-                integ, grad_output, prm, acc, L.acc_slots, gint, sp, d, exact != 0, s),
+                integ, grad_output, prm, acc, L.acc_slots, gint, sp, snap.use ? &snap : nullptr, d, exact != 0, s),
                 "grad_output streaming launch"))
             return rc;
-        if (need_input)
+        if constexpr (std::is_same<T, float>::value)
+            if (snap.use) {
+                if (int rc = hip_result(boxconv::grad_input_taps_launch<TG>(
+                        grad_output, gint, snap, sp, prm, grad_input, d, normalize != 0, exact != 0, s,
+                        &finish, &finished),
+                        "input-gradient launch"))
+                    return rc;
+            }
+        if (need_input && !snap.use)
             if (int rc = hip_result(boxconv::grad_input_launch<T, TG>(
                     gint, sp.R, prm, grad_input, d, normalize != 0, exact != 0, s,
                     need_params ? &finish : nullptr, &finished),

@@ -132,17 +132,34 @@ struct StreamPlan {
 };
 StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size);
 
+// Where the gradient w.r.t. the input is formed from grad_output itself (grad_input_taps_launch):
+// instead of the column workspace the pass then leaves sums of grad_output's rows at the rows
+// where the groups of 1 << shift output rows start.
+struct SnapshotPlan {
+    bool use;
+    int shift, groups;
+};
+template <class TG>
+SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d);
+template <class TG>
+hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, const SnapshotPlan& plan,
+                                  const StreamPlan& sp, BoxParams<float> prm, TG* grad_in, Dims d,
+                                  bool normalize, bool exact, hipStream_t stream,
+                                  const ParamFinish<float>* finish, bool* finish_done);
+
 // acc may be null: no parameter sums. With acc_slots == sp.nb it is [all planes*F][nb][5] doubles
 // and every workgroup stores its five partial sums in its own slot (nothing to clear, no atomics,
 // results reproducible bit for bit); with acc_slots == 0 it is [C*F*5] doubles, cleared by
 // grad_params_begin, and workgroups add atomically. grad_params_finish takes the same two values.
 // column_workspace ([planes*F] planes of column_workspace_plane(h, w) elements) may be null: no
 // workspace for the gradient w.r.t. the input. At least one of the two must be given.
+// snapshots (may be null): column_workspace receives the snapshots of that plan instead.
 // TG: element type of grad_out: T, or with T = float also f16_t / bf16_t (widened on load).
 template <class T, class TG>
 hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxParams<T> prm,
                                      double* acc, int acc_slots, T* column_workspace,
-                                     const StreamPlan& sp, Dims d, bool exact, hipStream_t stream);
+                                     const StreamPlan& sp, const SnapshotPlan* snapshots, Dims d,
+                                     bool exact, hipStream_t stream);
 
 hipError_t grad_params_begin(double* acc, int n_boxes, hipStream_t stream);
 template <class T>
@@ -201,6 +218,7 @@ struct Switches {
     bool stream_consecutive_partial;  // BOXCONV_STREAM_CONSEC=1 clears it: that variant only for rows that fill its workgroup exactly
     bool stream_narrow_double;  // BOXCONV_STREAM_F64_NARROW=0 clears it: float64 rows with three or four columns per lane and one launch like float32
     bool interleave_workspace;  // BOXCONV_M_INTERLEAVE=0 clears it: rows of the column workspace in their natural order
+    bool input_from_snapshots;  // BOXCONV_GI_SNAPSHOTS=0 clears it: grad_input from the column workspace only
     int stream_workgroups;    // BOXCONV_STREAM_WGS: workgroups the grad_output pass aims for when it cuts planes into bands (2048)
     int spin_limit;           // BOXCONV_INTEGRAL_SPIN: polls of a hand-over word before re-summing (64)
     int fwd_threads;          // BOXCONV_FWD_THREADS: 256 or 512 (512)

@@ -552,3 +552,37 @@ def test_clip_parameters_matches_oracle(hip, oracle):
             hip.clip_parameters(*t, rh, rw, mh, mw, exact)
             for a, b in zip(t, want):
                 assert np.array_equal(host(a), b)
+
+
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("planes,F,h,w", [
+    # groups of 8 output rows: one group, a ragged last one, several bands of the grad_output pass
+    (1, 2, 8, 256), (2, 1, 33, 100), (2, 3, 130, 300), (1, 4, 97, 640), (1, 2, 40, 1920), (1, 1, 50, 2048),
+    # groups of 16 rows: the smallest launch that takes them, ragged rows and columns
+    (256, 1, 113, 160), (128, 2, 129, 260), (64, 1, 250, 516), (40, 3, 210, 1024), (33, 2, 257, 1400)])
+def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact):
+    """grad_input formed from grad_output itself and the snapshots of its column sums (rows of a
+    multiple of four columns) against the oracle, and against the column workspace
+    (BOXCONV_GI_SNAPSHOTS=0): the two differ in the order of float32 additions, i.e. by a few units
+    in the last place of the largest partial sum. The boxes hang over every edge, so the rows where
+    the groups start clamp to both ends of the image. Parameter gradients keep their bits."""
+    rng = np.random.default_rng(planes + F + h + w)
+    x = rng.standard_normal((1, planes, h, w)).astype(np.float32)
+    g = (rng.standard_normal((1, planes * F, h, w)) + 0.25).astype(np.float32)
+    boxes = list(make_boxes(rng, planes, F, h, w, "hanging", away_from_integers=0.05))
+    if not exact:
+        boxes[1] = np.maximum(boxes[1], np.ceil(boxes[0]) + 1).astype(np.float32)
+        boxes[3] = np.maximum(boxes[3], np.ceil(boxes[2]) + 1).astype(np.float32)
+    results = []
+    for variant in (None, "0"):
+        switches("BOXCONV_GI_SNAPSHOTS", variant)
+        if planes <= 2:
+            cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, True, exact, g)
+            assert_parity(cpu, gpu, np.float32, "snapshots=%s %dx%d" % (variant, h, w), **sc)
+        back = hip.box_convolution_backward(hip.integral_image(dev(x)), *[dev(b) for b in boxes], dev(g), None,
+                                            3.5 * h, 2.25 * w, True, exact, True, True, True, True, True)
+        results.append([t.cpu().numpy() for t in back])
+    a, b = results
+    assert np.abs(a[0] - b[0]).max() <= 4e-6 * np.abs(b[0]).max()
+    for p, q in zip(a[1:], b[1:]):
+        assert np.array_equal(p, q)
