@@ -160,6 +160,153 @@ __global__ void __launch_bounds__(NT) forward_rows_kernel(SampleArgs<T> a, Forwa
     }
 }
 
+// The same for float rows of a multiple of four columns, up to 2048: a lane owns 4 CONSECUTIVE columns, for
+// the integral rows (one 16-byte load per row) as for the output (one 16- or 8-byte store per row), and
+// V sits in LDS by column modulo four (tap_run). The planes hold V[1..w]; the places in front of
+// them stay zero (V[0] = 0 and what clamps to it), those behind hold V[w].
+template <class TO>
+__device__ __forceinline__ void store_quad(TO* p, const Quad<TO>& q, bool stream) {
+    typedef unsigned Words __attribute__((ext_vector_type(sizeof(Quad<TO>) / 4)));
+    const Words v = __builtin_bit_cast(Words, q);
+    if (stream) __builtin_nontemporal_store(v, reinterpret_cast<Words*>(p));
+    else *reinterpret_cast<Words*>(p) = v;
+}
+
+template <class TO, int NT, bool EXACT, bool FULL, bool TAIL>
+__global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, ForwardTail<TO> tl) {
+    using T = float;
+    constexpr int K = 4, PLANE = quad_plane(NT), WAVES = NT / 64;
+    __shared__ __align__(16) RowPair<T> vrow[2][K][PLANE];
+    const unsigned vid = xcd_contiguous_id(a.per_xcd);
+    if (vid >= a.total) return;                      // whole workgroup leaves together
+    const unsigned nbands = a.nb, nfilt = a.F;
+    const unsigned inner = a.band_major ? nfilt : nbands, outer = a.band_major ? nbands : nfilt;
+    const unsigned v_in = vid % inner, v_rest = vid / inner;
+    const unsigned v_out = v_rest % outer, p32 = v_rest / outer;
+    const int band = static_cast<int>(a.band_major ? v_out : v_in);
+    const int f = static_cast<int>(a.band_major ? v_in : v_out);
+    const int64_t p = p32, pf = p * nfilt + f;
+    const int k_par = static_cast<int>(static_cast<unsigned>(a.plane0 + p) % static_cast<unsigned>(a.C)) * a.F + f;
+    const int h = a.h, w = a.w, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int quads = FULL ? NT : w / K;
+    const int c0 = K * tid;
+    const bool lane_in = FULL || tid < quads;
+    const unsigned cl = lane_in ? static_cast<unsigned>(c0) : 0u;    // idle lanes load the row's first columns and drop them
+
+    const BoxOfWorkgroup<T> bx = load_box(a.prm, k_par);
+    BoxSplit<T> s = split_forward(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
+    s.xlo = __builtin_amdgcn_readfirstlane(s.xlo); s.xhi = __builtin_amdgcn_readfirstlane(s.xhi);
+    s.ylo = __builtin_amdgcn_readfirstlane(s.ylo); s.yhi = __builtin_amdgcn_readfirstlane(s.yhi);
+    const T scale = a.normalize
+        ? inverse_extent(bx.xmin, bx.xmax, bx.ymin, bx.ymax, EXACT, true, true) : T(1);
+
+    const int64_t pitch = w + 1;
+    const T* plane = a.src + p * static_cast<int64_t>(h + 1) * pitch + 1;
+    auto load_i = [&](int r, T (&dst)[K]) {
+        load4_dword_aligned(at_bytes(plane + clampi(r, 0, h) * pitch, 4u * cl), dst);
+    };
+    const int64_t out0 = pf * static_cast<int64_t>(h) * w;
+    T ch_scale = T(1), ch_shift = T(0);
+    if (TAIL) {
+        if (tl.channel_scale != nullptr) ch_scale = tl.channel_scale[k_par];
+        if (tl.channel_shift != nullptr) ch_shift = tl.channel_shift[k_par];
+    }
+    const bool relu = TAIL && tl.relu != 0;
+    const bool has_residual = TAIL && tl.residual != nullptr;
+    const TO* residual = has_residual ? tl.residual : tl.dst;
+
+    if (tid < 2 * K * kQuadPad)
+        vrow[tid / (K * kQuadPad)][tid / kQuadPad % K][tid % kQuadPad] = RowPair<T>{T(0), T(0)};
+    const TapRun er = tap_run<PLANE>(tid, s.yhi - 1, quads), el = tap_run<PLANE>(tid, s.ylo - 2, quads);
+    const int last = (quads - 1) & 63;               // lane of the last wave that owns column w
+
+    const int i0 = band * a.R;
+    const int i1 = min(h, i0 + a.R);
+    T ta[K], bc[K];                       // I[t(i-1)], I[b(i)]
+    T t0[K], t1[K], b1[K], b2[K];         // I[t(i)], I[t(i+1)], I[b(i+1)], I[b(i+2)]
+    load_i(i0 + s.xlo - 1, ta);
+    load_i(i0 + s.xhi, bc);
+    load_i(i0 + s.xlo, t0);
+    load_i(i0 + 1 + s.xlo, t1);
+    load_i(i0 + 1 + s.xhi, b1);
+    load_i(i0 + 2 + s.xhi, b2);
+
+    auto row_pair = [&](int i, auto prefetch_tag, auto flip_tag) {
+        constexpr bool PREFETCH = decltype(prefetch_tag)::value;
+        constexpr int FLIP = decltype(flip_tag)::value;
+        T n0[K] = {}, n1[K] = {}, n2[K] = {}, n3[K] = {};
+        if (PREFETCH) {
+            load_i(i + 2 + s.xlo, n0);
+            load_i(i + 3 + s.xlo, n1);
+            load_i(i + 3 + s.xhi, n2);
+            load_i(i + 4 + s.xhi, n3);
+        }
+        const bool second = i + 1 < i1;
+        const int64_t row0 = out0 + static_cast<int64_t>(i) * w, row1 = second ? row0 + w : row0;
+        Quad<TO> res0{}, res1{};                     // (without a residual the loads read what is stored over, and are dropped)
+        if (TAIL) {
+            res0 = *reinterpret_cast<const Quad<TO>*>(residual + row0 + cl);
+            res1 = *reinterpret_cast<const Quad<TO>*>(residual + row1 + cl);
+        }
+        T v0[K], v1[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            v0[k] = blend<T, EXACT>(ta[k], t0[k], bc[k], b1[k], s.fxlo, s.fxhi);
+            v1[k] = blend<T, EXACT>(t0[k], t1[k], b1[k], b2[k], s.fxlo, s.fxhi);
+        }
+        if (lane_in) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) vrow[FLIP][k][kQuadPad + tid] = RowPair<T>{v0[k], v1[k]};
+        }
+        if (wave == WAVES - 1) {                     // (scalar)
+            const RowPair<T> end{read_lane(v0[K - 1], last), read_lane(v1[K - 1], last)};
+            const int e = tid & 63;
+            if (e < K * kQuadPad) vrow[FLIP][e / kQuadPad][kQuadPad + quads + e % kQuadPad] = end;
+        }
+        __syncthreads();
+
+        RowPair<T> R[K + 1], L[K + 1];
+        read_taps(vrow[FLIP][0], er, R);
+        read_taps(vrow[FLIP][0], el, L);
+        Quad<TO> z0, z1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            T y0 = blend<T, EXACT>(L[k].r0, L[k + 1].r0, R[k].r0, R[k + 1].r0, s.fylo, s.fyhi) * scale;
+            T y1 = blend<T, EXACT>(L[k].r1, L[k + 1].r1, R[k].r1, R[k + 1].r1, s.fylo, s.fyhi) * scale;
+            if (TAIL) {
+                y0 = y0 * ch_scale + ch_shift + (has_residual ? widen(res0.v[k]) : T(0));
+                y1 = y1 * ch_scale + ch_shift + (has_residual ? widen(res1.v[k]) : T(0));
+                if (relu) { y0 = y0 < T(0) ? T(0) : y0; y1 = y1 < T(0) ? T(0) : y1; }
+            }
+            narrow(y0, z0.v[k]);
+            narrow(y1, z1.v[k]);
+        }
+        if (lane_in) {
+            store_quad(tl.dst + row0 + cl, z0, a.stream_out != 0);
+            if (second) store_quad(tl.dst + row1 + cl, z1, a.stream_out != 0);
+        }
+        if (PREFETCH) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                ta[k] = t1[k]; bc[k] = b2[k];
+                t0[k] = n0[k]; t1[k] = n1[k]; b1[k] = n2[k]; b2[k] = n3[k];
+            }
+        }
+    };
+    int i = i0;
+    for (; i + 4 < i1; i += 4) {
+        row_pair(i, std::true_type{}, Flip0{});
+        row_pair(i + 2, std::true_type{}, Flip1{});
+    }
+    if (i + 2 < i1) {
+        row_pair(i, std::true_type{}, Flip0{});
+        row_pair(i + 2, std::false_type{}, Flip1{});
+    } else {
+        row_pair(i, std::false_type{}, Flip0{});
+    }
+}
+
 template <class T, class TO, bool EXACT, bool TAIL>
 __global__ void __launch_bounds__(256) forward_gather_kernel(SampleArgs<T> a, ForwardTail<TO> tl) {
     const int64_t hw = static_cast<int64_t>(a.h) * a.w;
@@ -233,6 +380,42 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
     const uint64_t out_bytes = static_cast<uint64_t>(planes_f) * d.hw() * sizeof(TO);
     a.stream_out = ((static_cast<uint64_t>(d.w) * sizeof(TO)) % 64 == 0 || out_bytes > (256ull << 20)) ? 1 : 0;
     const dim3 grid(static_cast<unsigned>(a.per_xcd * kXcds));
+    if constexpr (std::is_same<T, float>::value) {
+        // Four consecutive columns per lane: rows of one wave (up to 256 columns, at least three
+        // eighths of its lanes busy), and 16-bit outputs of wider rows, where the other kernel stores
+        // 2 bytes per lane. Measured, us, other kernel -> this one: float32 32 x 4 planes of
+        // 128 x 256 x 4 15.5 -> 14.8, 135 x 240 19.6 -> 16.3, with the tail 32.2 -> 25.0, 36.6 -> 25.1;
+        // bfloat16 with the tail 26.2 -> 17.4, 30.2 -> 18.9 (x 8: 51.6 -> 30.7), 16 x 8 planes of 300 x 768
+        // 74 -> 47, 1080 x 1920 380 -> 356; without it 512 x 1024 118 -> 90, 720 x 1280 97 -> 76. Not for
+        // wider float32 rows (256 x 512 54 -> 72, 720 x 1280 105 -> 111, 1080 x 1920 229 -> 373: stores of
+        // 16 bytes per lane reach the memory no better, and the loads start at odd addresses), nor
+        // without a tail beyond 1280 columns (1080 x 1920 213 -> 237) or where an eighth of the
+        // lanes idles (200 x 384 27 -> 31).
+        const int lanes = d.w / 4, cnt = consecutive_threads(d.w);
+        const bool one_wave = cnt == 64 && lanes * 8 >= cnt * 3;
+        const bool wide_half = sizeof(TO) == 2 && cnt > 64 && (TAIL || (d.w <= 1280 && lanes * 8 >= cnt * 7));
+        const size_t align = 4 * sizeof(TO);
+        if (switches().forward_quads && d.w % 4 == 0 && d.w <= 2048 && (one_wave || wide_half) &&
+            reinterpret_cast<uintptr_t>(tail.dst) % align == 0 && reinterpret_cast<uintptr_t>(tail.residual) % align == 0) {
+#define LAUNCH_FQ(NT)                                                                                                  \
+    case NT:                                                                                                           \
+        if (lanes == NT) {                                                                                             \
+            if (exact) BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, true, true, TAIL>), grid, dim3(NT), 0, stream, a, tail);   \
+            else       BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, false, true, TAIL>), grid, dim3(NT), 0, stream, a, tail);  \
+        } else {                                                                                                       \
+            if (exact) BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, true, false, TAIL>), grid, dim3(NT), 0, stream, a, tail);  \
+            else       BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, false, false, TAIL>), grid, dim3(NT), 0, stream, a, tail); \
+        }                                                                                                              \
+        break;
+            switch (cnt) {
+                LAUNCH_FQ(64) LAUNCH_FQ(128) LAUNCH_FQ(192) LAUNCH_FQ(256)
+                LAUNCH_FQ(320) LAUNCH_FQ(384) LAUNCH_FQ(448) LAUNCH_FQ(512)
+                default: return hipErrorInvalidValue;
+            }
+#undef LAUNCH_FQ
+            return hipGetLastError();
+        }
+    }
     const size_t lds = 4 * static_cast<size_t>(d.w + 3) * sizeof(T);
 #define LAUNCH_FWD(NT, KK, EX, FU) \
     BOXCONV_LAUNCH("forward_rows", (forward_rows_kernel<T, TO, NT, KK, EX, FU, TAIL>), grid, dim3(NT), lds, stream, a, tail)

@@ -36,6 +36,7 @@ Switches read_switches() {
     }
     s.stream_narrow_double = flag_unless_zero("BOXCONV_STREAM_F64_NARROW");
     s.interleave_workspace = flag_unless_zero("BOXCONV_M_INTERLEAVE");
+    s.forward_quads = flag_unless_zero("BOXCONV_FWD_QUADS");
     s.input_from_snapshots = flag_unless_zero("BOXCONV_GI_SNAPSHOTS");
     e = text("BOXCONV_STREAM_WGS");
     s.stream_workgroups = e != nullptr ? std::max(1, std::atoi(e)) : 2048;

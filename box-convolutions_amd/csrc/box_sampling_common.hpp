@@ -187,6 +187,48 @@ __device__ __forceinline__ RowPair<T> sample_columns(const RowPair<T>* __restric
             blend<T, EXACT>(la.r1, l.r1, r.r1, ra.r1, fylo, fyhi)};
 }
 
+// ---- lanes that own 4 consecutive columns ---------------------------------------------------------
+template <class T>
+struct alignas(sizeof(T) >= 4 ? 16 : 4 * sizeof(T)) Quad {
+    T v[4];
+};
+
+typedef float f4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load4_dword_aligned(const float* p, float (&v)[4]) {
+    const f4_dword_aligned q = *reinterpret_cast<const f4_dword_aligned*>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+
+// LDS layout of a row pair for lanes that own 4 consecutive columns: column c is element c / 4 of
+// plane c % 4. A lane's taps are 5 adjacent columns that start anywhere; tap m of all lanes then
+// lies in one plane at lane-consecutive places, so every access of a wave is 512 contiguous bytes
+// (columns side by side, a lane's neighbour sits 32 bytes away and an access takes twice as many
+// LDS cycles: 512 x 1024, 16 x 8 planes, 150 cycles per wave and row pair, 87 of them conflicts).
+// kQuadPad elements of zeros in front of every plane and behind it stand for the columns outside.
+constexpr int kQuadPad = 2;
+__host__ __device__ constexpr int quad_plane(int nt) { return nt + 64; }   // a multiple of 64 elements: two planes per access
+// Byte offsets of the taps at columns 4 * tid + first + m, m < 4 (m = 4: one element after m = 0).
+struct TapRun {
+    unsigned at[4];
+};
+template <int PLANE>
+__device__ __forceinline__ TapRun tap_run(int tid, int first, int quads) {
+    const int plane = first & 3, place = clampi(tid + (first >> 2), -kQuadPad, quads) + kQuadPad;
+    TapRun t;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        t.at[m] = static_cast<unsigned>(((plane + m) & 3) * PLANE + ((plane + m) >> 2) + place) * static_cast<unsigned>(sizeof(RowPair<float>));
+    return t;
+}
+__device__ __forceinline__ void read_taps(const RowPair<float>* row, const TapRun& t, RowPair<float> (&v)[5]) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) v[m] = *at_bytes(row, t.at[m]);
+    v[4] = at_bytes(row, t.at[0])[1];
+}
+
+// The smallest workgroup (whole waves) whose lanes, four columns each, cover a row.
+inline int consecutive_threads(int w) { return (w / 4 + 63) / 64 * 64; }
+
 template <class T>
 struct BoxOfWorkgroup {
     T xmin, xmax, ymin, ymax;

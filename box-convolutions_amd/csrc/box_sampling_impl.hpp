@@ -173,11 +173,6 @@ param_grad_finalize_kernel(FinalizeArgs<T> fa, BoxParams<T> prm) {
 // filters g, g + FS, ... and the FS partial sums are added in that order through LDS at the end.
 // A small launch cannot fill the chip with workgroups, and a workgroup that walks through all F
 // filters alone is one chain of F memory round trips.
-template <class T>
-struct alignas(sizeof(T) >= 4 ? 16 : 4 * sizeof(T)) Quad {
-    T v[4];
-};
-
 // TO: element type of grad_input (T, or a 16-bit type when T is float: a.dst then points at
 // elements of TO and the sums are rounded to it in the store).
 template <class T, class TO, int LQ, int RB, bool EXACT, int FS>
@@ -917,38 +912,6 @@ grad_output_stream_kernel(SampleArgs<T> a) {
 // !FULL: the lanes past the row's end (whole lanes, since w is a multiple of four) load from the
 // row's first columns and drop what they loaded where it would be used: they put zeros into LDS
 // (the row's right-hand padding), hold zero weights and a zero V, and store nothing.
-typedef float f4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ void load4_dword_aligned(const float* p, float (&v)[4]) {
-    const f4_dword_aligned q = *reinterpret_cast<const f4_dword_aligned*>(p);
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-}
-
-// LDS layout of a row pair for lanes that own 4 consecutive columns: column c is element c / 4 of
-// plane c % 4. A lane's taps are 5 adjacent columns that start anywhere; tap m of all lanes then
-// lies in one plane at lane-consecutive places, so every access of a wave is 512 contiguous bytes
-// (columns side by side, a lane's neighbour sits 32 bytes away and an access takes twice as many
-// LDS cycles: 512 x 1024, 16 x 8 planes, 150 cycles per wave and row pair, 87 of them conflicts).
-// kQuadPad elements of zeros in front of every plane and behind it stand for the columns outside.
-constexpr int kQuadPad = 2;
-__host__ __device__ constexpr int quad_plane(int nt) { return nt + 64; }   // a multiple of 64 elements: two planes per access
-// Byte offsets of the taps at columns 4 * tid + first + m, m < 4 (m = 4: one element after m = 0).
-struct TapRun {
-    unsigned at[4];
-};
-template <int PLANE>
-__device__ __forceinline__ TapRun tap_run(int tid, int first, int quads) {
-    const int plane = first & 3, place = clampi(tid + (first >> 2), -kQuadPad, quads) + kQuadPad;
-    TapRun t;
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-        t.at[m] = static_cast<unsigned>(((plane + m) & 3) * PLANE + ((plane + m) >> 2) + place) * static_cast<unsigned>(sizeof(RowPair<float>));
-    return t;
-}
-__device__ __forceinline__ void read_taps(const RowPair<float>* row, const TapRun& t, RowPair<float> (&v)[5]) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) v[m] = *at_bytes(row, t.at[m]);
-    v[4] = at_bytes(row, t.at[0])[1];
-}
 
 // What the kernel leaves for the gradient w.r.t. the input.
 enum StreamMode {
@@ -1551,7 +1514,6 @@ inline int64_t cached_tail_bytes() { return switches().keep_tail_bytes; }
 // 110 -> 90, 260: 138 -> 118, 300: 142 -> 121; but 64 columns 72 -> 83). Rows of exactly 128 columns
 // also stay there: they fill that kernel's two waves at one column per lane with no bounds to check
 // (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us).
-inline int consecutive_threads(int w) { return (w / 4 + 63) / 64 * 64; }
 template <class TG>
 bool stream_consecutive_applies(const TG* grad_out, int w) {
     if (w % 4 != 0 || w > 2048 || reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) != 0) return false;

@@ -219,6 +219,7 @@ struct Switches {
     bool stream_narrow_double;  // BOXCONV_STREAM_F64_NARROW=0 clears it: float64 rows with three or four columns per lane and one launch like float32
     bool interleave_workspace;  // BOXCONV_M_INTERLEAVE=0 clears it: rows of the column workspace in their natural order
     bool input_from_snapshots;  // BOXCONV_GI_SNAPSHOTS=0 clears it: grad_input from the column workspace only
+    bool forward_quads;       // BOXCONV_FWD_QUADS=0 clears it: no forward kernel with four consecutive columns per lane
     int stream_workgroups;    // BOXCONV_STREAM_WGS: workgroups the grad_output pass aims for when it cuts planes into bands (2048)
     int spin_limit;           // BOXCONV_INTEGRAL_SPIN: polls of a hand-over word before re-summing (64)
     int fwd_threads;          // BOXCONV_FWD_THREADS: 256 or 512 (512)

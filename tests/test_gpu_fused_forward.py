@@ -278,3 +278,43 @@ def test_forward_fused_modes_and_double_input():
         got = m.forward_fused(x.double(), output_dtype=torch.float32)
         assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
     assert not m.forward_fused(x).requires_grad
+
+
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("tail", [False, True])
+@pytest.mark.parametrize("dtype,h,w", [
+    # one wave: three eighths of the lanes, an odd number of rows, all lanes
+    (torch.float32, 9, 96), (torch.float32, 35, 100), (torch.float32, 40, 252), (torch.float32, 12, 256),
+    (torch.bfloat16, 17, 132), (torch.float16, 8, 256),
+    # 16-bit rows of several waves
+    (torch.float16, 21, 512), (torch.bfloat16, 11, 1000), (torch.float16, 10, 1280), (torch.bfloat16, 7, 1284),
+    (torch.float16, 9, 2048)])
+def test_forward_with_consecutive_columns(switches, dtype, h, w, tail, exact):
+    """The forward kernel with four consecutive columns per lane against the one with wave-strided
+    columns (BOXCONV_FWD_QUADS=0): the same expressions per pixel, so at most the contraction of a
+    product and a sum differs, a unit in the last place of float32 or one rounding to 16 bits.
+    Boxes hang over every edge; without a residual the output's memory holds NaN beforehand."""
+    from box_convolution import _native as hip
+    gen = torch.Generator().manual_seed(h * w)
+    B, C, F = 2, 2, 3
+    x = torch.randn(B, C, h, w, generator=gen).cuda().to(dtype)
+    lo_x, lo_y = ((torch.rand(C, F, generator=gen) * 2 - 1.2) * n for n in (h, w))
+    boxes = [t.cuda() for t in (lo_x, lo_x + 2.2 + torch.rand(C, F, generator=gen) * h,
+                                lo_y, lo_y + 2.2 + torch.rand(C, F, generator=gen) * w)]
+    integ = hip.integral_image(x)
+    variants = [(None, None, None, False)]
+    if tail:
+        scale, shift = torch.rand(C * F, generator=gen).cuda(), torch.randn(C * F, generator=gen).cuda()
+        residual = torch.randn(B, C * F, h, w, generator=gen).cuda().to(dtype)
+        variants = [(scale, shift, residual, True), (scale, None, None, True)]
+    for args in variants:
+        results = []
+        for variant in (None, "0"):
+            switches("BOXCONV_FWD_QUADS", variant)
+            filler = torch.full((B, C * F, h, w), float("nan"), device="cuda", dtype=dtype)
+            del filler                                   # (the allocator hands this block out next)
+            results.append(hip.box_convolution_forward_fused(integ, *boxes, True, exact, dtype, *args).float())
+        a, b = results
+        assert torch.isfinite(a).all()
+        unit = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+        assert ((a - b).abs() <= unit * b.abs() + 1e-6 * b.abs().max()).all()
