@@ -13,7 +13,7 @@
 //                            input row, then a row-direction prefix of the accumulators.
 // With a single band (tall enough grid without cutting) only launch 3 runs. Rows of at most 4096
 // columns use band_scan_rows_kernel for launch 3, which adds up the bands above itself (no launch
-// 2). For float rows that fill a workgroup exactly and planes of at most 16 bands of 32 rows, one
+// 2). For float rows of 256 to 2048 columns and planes of at most 32 bands of 32 rows, one
 // kernel does everything in a single pass over the input (band_scan_lookback_kernel): workgroups
 // hand their column sums to the ones below them, with a bounded wait. Planes of at most 192 rows
 // and 256 columns take plane_scan_kernel: the bands of a plane are the waves of one workgroup,
@@ -402,7 +402,16 @@ clip_and_fill_marker_kernel(ClipArgs<T> clip, int clip_blocks, unsigned long lon
     if (i < n) dst[i] = kNotPublished;
 }
 
-template <class TI, int WAVES, int RB, bool VEC, bool FULL>
+// How band_scan_lookback_kernel reads a row.
+enum RowLoads {
+    kElements,      // element by element (16-bit rows that are not aligned; rows of fewer than 4 columns)
+    kAlignedQuads,  // rows of a multiple of four columns, 16-byte (8-byte) aligned: one load per lane
+    kShiftedQuads,  // any other float row: one 16-byte load per lane from a dword-aligned address. The lane
+                    // whose four columns straddle the row's end reads the row's last four columns
+                    // and shifts them; nothing outside the row is touched
+};
+
+template <class TI, int WAVES, int RB, int LOADS, bool FULL>
 __global__ void __launch_bounds__(WAVES * 64)
 band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, double* aux,
                           int h, int w, int nb, int R, int64_t planes, int64_t per_xcd,
@@ -441,17 +450,34 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
     // Loads are unconditional (a clamped address, the value dropped afterwards) so that all rows
     // of the band are in flight together; the row address is wave-uniform, the lane part 32 bits.
     const bool lane_in = c0 < w;
-    const unsigned lane_col = lane_in ? static_cast<unsigned>(c0) : 0u;
+    const unsigned lane_col = LOADS == kShiftedQuads ? static_cast<unsigned>(min(c0, w - 4)) : lane_in ? static_cast<unsigned>(c0) : 0u;
+    const int shift = c0 - static_cast<int>(lane_col);   // kShiftedQuads: 0 but for the last lanes; 4 and more: nothing left
     auto load_row = [&](int row, bool exists, T (&x)[4]) {
-        if (VEC) {
+        if (LOADS == kAlignedQuads) {
             const TI* rowp = src + static_cast<int64_t>(min(row, h - 1)) * w;
             load_quad(rowp + lane_col, x);
             if (!(exists && lane_in)) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) x[v] = T(0);
             }
+        } else if constexpr (LOADS == kShiftedQuads) {
+            typedef float f4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
+            const f4_dword_aligned q = __builtin_nontemporal_load(reinterpret_cast<const f4_dword_aligned*>(
+                src + static_cast<int64_t>(min(row, h - 1)) * w + lane_col));
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x[v] = exists ? q[v] : T(0);
         } else {
             buffer_load_run_as<kCacheStream, TI>(x, irows.row(min(row, h - 1), exists), in_off);
+        }
+    };
+    // kShiftedQuads: what the last wave's lanes loaded, moved to the columns they own
+    auto shift_row = [&](T (&x)[4]) {
+        const T q[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            x[v] = T(0);
+#pragma unroll
+            for (int u = v; u < 4; ++u) x[v] = shift == u - v ? q[u] : x[v];
         }
     };
 
@@ -459,6 +485,10 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
     T x[RMAX][4];
 #pragma unroll
     for (int r = 0; r < RMAX; ++r) load_row(r0 + r, r < R && r0 + r < r1, x[r]);
+    if (LOADS == kShiftedQuads && wave == WAVES - 1) {   // (scalar; the launch has no more waves than the row needs)
+#pragma unroll
+        for (int r = 0; r < RMAX; ++r) shift_row(x[r]);
+    }
 
     if (band == 0)
         for (int c = tid; c <= w; c += NT) dst[c] = T(0);
@@ -528,6 +558,7 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
                 for (int r = b * R; r < (b + 1) * R; ++r) {      // bands above are complete bands
                     T t[4];
                     load_row(r, true, t);
+                    if (LOADS == kShiftedQuads && wave == WAVES - 1) shift_row(t);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) part[v] += static_cast<double>(t[v]);
                 }
@@ -859,13 +890,20 @@ hipError_t launch_lookback(const TI* in, float* out, double* aux, int64_t planes
     const dim3 grid(static_cast<unsigned>(per_xcd * kXcds));
     const dim3 block(WAVES * 64);
     // full: every lane holds four columns of the row or none (rows of a multiple of four columns)
-    const bool vec = aligned_for_vec4(in, w), full = vec;
-#define LAUNCH_LOOKBACK(VEC, FULL)                                                                 \
-    BOXCONV_LAUNCH("band_scan", (band_scan_lookback_kernel<TI, WAVES, 4, VEC, FULL>), grid, block, 0,  \
+#define LAUNCH_LOOKBACK(LOADS, FULL)                                                               \
+    BOXCONV_LAUNCH("band_scan", (band_scan_lookback_kernel<TI, WAVES, 4, LOADS, FULL>), grid, block, 0,  \
                    stream, in, out, aux, h, w, nb, R, planes, per_xcd, rev, spin)
-    if (vec && full) LAUNCH_LOOKBACK(true, true);
-    else if (vec)    LAUNCH_LOOKBACK(true, false);
-    else             LAUNCH_LOOKBACK(false, false);
+    if (aligned_for_vec4(in, w)) {
+        LAUNCH_LOOKBACK(kAlignedQuads, true);
+    } else {
+        if constexpr (std::is_same<TI, float>::value) {
+            if (w >= 4 && reinterpret_cast<uintptr_t>(in) % sizeof(float) == 0) {
+                LAUNCH_LOOKBACK(kShiftedQuads, false);
+                return hipGetLastError();
+            }
+        }
+        LAUNCH_LOOKBACK(kElements, false);
+    }
 #undef LAUNCH_LOOKBACK
     return hipGetLastError();
 }
@@ -998,9 +1036,16 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // against 44, 256 x 1536 26 against 37, 512 x 1000 40 against 50, 480 x 640 35 against 41;
     // but 540 x 960, one workgroup in sixteen too many to be resident, 63 against 51, and
     // 1080 x 1920, 34 bands per plane, 117 against 80.)
+    // Rows of other widths (kShiftedQuads), only where all workgroups are resident, which also bounds
+    // the workspace: 64 planes of 270 x 481 39 -> 25 us, 16 of 301 x 767 33 -> 20, 16 of 500 x 1001
+    // 38 -> 27, 8 of 1000 x 2001 65 -> 40, 32 of 200 x 257 20 -> 16; in bfloat16 (element loads) 35 -> 28,
+    // 27 -> 20, 34 -> 27, 55 -> 42, 19 -> 18, and 12 of 700 x 1401 50 -> 56, of which a training or eval
+    // forward gets a launch back (the clip's launch also marks the hand-over words).
     // Narrower rows leave most of a wave idle in either kernel; the two passes are faster there
     // (64 x 128: 20 against 24 us, 135 x 240: 21 against 25).
-    const bool measured_faster = w % 4 == 0 && w >= 256 && ((groups <= resident && bands32 <= 32) || groups >= 4096);
+    const bool all_resident = groups <= resident && bands32 <= 32;
+    const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096
+                                                         : all_resident && !switches().lookback_quads_only);
     const bool single_pass = wanted >= 2 && h > kLookbackRows && w <= 2048 && scan_by_rows(h, w, sizeof(float)) &&
                              bands32 <= kLookbackBands && (lookback_any_shape() || measured_faster);
     if (single_pass) nb = (h + kLookbackRows - 1) / kLookbackRows;

@@ -586,3 +586,25 @@ def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact
     assert np.abs(a[0] - b[0]).max() <= 4e-6 * np.abs(b[0]).max()
     for p, q in zip(a[1:], b[1:]):
         assert np.array_equal(p, q)
+
+
+@pytest.mark.parametrize("spin", [None, "0"])
+@pytest.mark.parametrize("planes,h,w", [(3, 40, 257), (2, 33, 258), (5, 70, 259), (16, 301, 767), (64, 65, 481),
+                                        (1, 97, 1021), (2, 100, 1537), (1, 64, 2047)])
+def test_integral_image_single_pass_of_odd_rows(hip, switches, planes, h, w, spin):
+    """Rows of 256 columns and more that are not a multiple of four columns: the single pass reads
+    them with 16-byte loads that start anywhere, the lane at the row's end from the row's last four
+    columns. The two passes (BOXCONV_INTEGRAL_LOOKBACK=1) may cut the planes into other bands, i.e.
+    associate the double sums differently; spin = 0 sums every band above again."""
+    x = torch.randn(1, planes, h, w, generator=torch.Generator().manual_seed(h * w)).cuda()
+    switches("BOXCONV_INTEGRAL_LOOKBACK", "1")
+    two = hip.integral_image(x).clone()
+    switches("BOXCONV_INTEGRAL_LOOKBACK", None)
+    switches("BOXCONV_INTEGRAL_SPIN", spin)
+    one = hip.integral_image(x)
+    assert torch.allclose(one, two, rtol=2e-7, atol=0)
+    want = np.cumsum(np.cumsum(x.cpu().numpy().astype(np.float64), axis=2), axis=3)
+    got = one.cpu().numpy()
+    assert not got[:, :, 0].any() and not got[..., 0].any()
+    # a float32 rounding of a double sum: half a unit in the last place of the largest entry
+    assert np.abs(got[:, :, 1:, 1:] - want).max() <= 2.0 ** -24 * 1.01 * np.abs(want).max()
