@@ -105,12 +105,18 @@ hipError_t grad_params_begin(double* acc, int n_boxes, hipStream_t stream) {
     return hipGetLastError();
 }
 
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size) {
+StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool params) {
     StreamPlan sp{};
     const RowConfig rc = stream_row_config(std::max(w, 1), elem_size);
     sp.usable = row_kernels_apply(h, w, elem_size) &&
                 stream_lds_bytes(rc.K, rc.nt, elem_size) <= kMaxDynamicLds;
-    int nb = bands_for(std::max<int64_t>(planes_f, 1), h, 32, switches().stream_workgroups);
+    // Parameter sums of rows that one wave covers at four columns per lane: four such workgroups
+    // fit every SIMD and the band's chain of row pairs is what they wait for, so twice as many
+    // (256 x 4 planes of 128 x 256 in bfloat16, bands of 64 -> 32 rows: 40 -> 30 us, and 28 -> 29 in
+    // the grad-input pass, which adds up more bands). Wider rows lose there what they gain
+    // (512 x 1024: 136 -> 133 and 129 -> 138 us).
+    const bool one_wave = params && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64;
+    int nb = bands_for(std::max<int64_t>(planes_f, 1), h, 32, switches().stream_workgroups * (one_wave ? 2 : 1));
     int R = (h + nb - 1) / nb;
     R += R & 1;                                        // rows are handled in pairs
     sp.R = std::max(R, 2);

@@ -1514,14 +1514,17 @@ inline int64_t cached_tail_bytes() { return switches().keep_tail_bytes; }
 // 110 -> 90, 260: 138 -> 118, 300: 142 -> 121; but 64 columns 72 -> 83). Rows of exactly 128 columns
 // also stay there: they fill that kernel's two waves at one column per lane with no bounds to check
 // (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us).
-template <class TG>
-bool stream_consecutive_applies(const TG* grad_out, int w) {
-    if (w % 4 != 0 || w > 2048 || reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) != 0) return false;
+inline bool consecutive_rows(int w) {
+    if (w % 4 != 0 || w > 2048) return false;
     const RowConfig rc = stream_row_config(w, sizeof(float));
     const int lanes = w / 4, cnt = consecutive_threads(w);
     const bool exact_fit = lanes == cnt && (cnt == 64 || cnt == 128 || cnt == 256 || cnt == 512);
     return switches().stream_consecutive &&
            (exact_fit || (switches().stream_consecutive_partial && lanes * 8 >= cnt * 3 && !(rc.full && rc.K == 1)));
+}
+template <class TG>
+bool stream_consecutive_applies(const TG* grad_out, int w) {
+    return consecutive_rows(w) && reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) == 0;
 }
 
 // The launches of grad_output_stream_consec_kernel (`lanes` busy lanes of a workgroup of `cnt`;

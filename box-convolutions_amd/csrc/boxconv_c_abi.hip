@@ -109,7 +109,7 @@ BackwardLayout backward_layout(int batch, int in_planes, int num_filters, int h,
                                int elem_size, bool need_input, bool need_params) {
     BackwardLayout L{};
     const int64_t planes = std::max<int64_t>(static_cast<int64_t>(batch) * in_planes, 1);
-    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, elem_size);
+    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, elem_size, need_params);
     L.streaming = sp.usable;
     size_t off = 0;
     L.gint_off = off;
@@ -388,7 +388,7 @@ int backward_impl(const T* integ, const T* x_min, const T* x_max, const T* y_min
     if (L.streaming) {
         // one pass over grad_output: parameter sums + column workspace, then grad_input, whose
         // launch finishes the parameter gradients on the side
-        const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, sizeof(T));
+        const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, sizeof(T), need_params);
         boxconv::SnapshotPlan snap{};
         if constexpr (std::is_same<T, float>::value)
             if (need_input && need_params && nout > 0)

@@ -130,7 +130,8 @@ struct StreamPlan {
     int parts;               // workgroups that share a band for the parameter sums (1, or 2 for rows
                              // wider than 2048 columns): accumulation slots per (plane, filter) = nb * parts
 };
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size);
+// params: the parameter sums are wanted (the bands, i.e. the slots per (plane, filter), depend on it)
+StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool params);
 
 // Where the gradient w.r.t. the input is formed from grad_output itself (grad_input_taps_launch):
 // instead of the column workspace the pass then leaves sums of grad_output's rows at the rows
