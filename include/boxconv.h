@@ -256,7 +256,8 @@ int boxconv_forward_fused_f32(const float* input_integrated, const float* x_min,
  * workspace: boxconv_backward_workspace_bytes(...) bytes, 256-byte aligned. It receives the
  * backward's one intermediate per (plane, filter) - h+1 rows of grad_output filtered along the
  * row and summed down the rows of a band (the bulk; for rows wider than 4096 columns, 2048 in
- * float64, a true integral image of grad_output instead) - and the per-box accumulators. */
+ * float64, a true integral image of grad_output instead; for most rows of a multiple of four columns
+ * only column sums at every 8th or 16th row, in the same place) - and the per-box accumulators. */
 size_t boxconv_backward_workspace_bytes(int batch, int in_planes, int num_filters, int h, int w,
                                         int elem_size, int input_needs_grad,
                                         int params_need_grad);
