@@ -39,6 +39,8 @@ Switches read_switches() {
     s.interleave_workspace = flag_unless_zero("BOXCONV_M_INTERLEAVE");
     s.forward_quads = flag_unless_zero("BOXCONV_FWD_QUADS");
     s.input_from_snapshots = flag_unless_zero("BOXCONV_GI_SNAPSHOTS");
+    e = text("BOXCONV_GI_SNAPSHOTS");
+    s.snapshots_any_shape = e != nullptr && std::atoi(e) == 2;
     e = text("BOXCONV_STREAM_WGS");
     s.stream_workgroups = e != nullptr ? std::max(1, std::atoi(e)) : 2048;
     e = text("BOXCONV_INTEGRAL_SPIN");
@@ -105,7 +107,7 @@ hipError_t grad_params_begin(double* acc, int n_boxes, hipStream_t stream) {
     return hipGetLastError();
 }
 
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool params) {
+StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool sums_only) {
     StreamPlan sp{};
     const RowConfig rc = stream_row_config(std::max(w, 1), elem_size);
     sp.usable = row_kernels_apply(h, w, elem_size) &&
@@ -114,8 +116,9 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
     // fit every SIMD and the band's chain of row pairs is what they wait for, so twice as many
     // (256 x 4 planes of 128 x 256 in bfloat16, bands of 64 -> 32 rows: 40 -> 30 us, and 28 -> 29 in
     // the grad-input pass, which adds up more bands). Wider rows lose there what they gain
-    // (512 x 1024: 136 -> 133 and 129 -> 138 us).
-    const bool one_wave = params && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64;
+    // (512 x 1024: 136 -> 133 and 129 -> 138 us), and so does the pass that also leaves the column
+    // workspace (64 x 8 planes of 200 x 252, both kernels: 70 -> 82 us).
+    const bool one_wave = sums_only && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64;
     int nb = bands_for(std::max<int64_t>(planes_f, 1), h, 32, switches().stream_workgroups * (one_wave ? 2 : 1));
     int R = (h + nb - 1) / nb;
     R += R & 1;                                        // rows are handled in pairs
@@ -123,6 +126,31 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
     sp.nb = (h + sp.R - 1) / sp.R;
     sp.parts = (rc.nt == 1024 || stream_double_wide_split(w, elem_size)) ? 2 : 1;
     return sp;
+}
+
+// grad_input_taps_kernel walks through a plane's filters one after the other, 1.5 to 2.5 us each
+// however few the planes are, where grad_input_cols_kernel spreads filters and rows over more waves.
+// Both backward kernels together were timed against the column workspace on 5600 shapes (1 to 512
+// planes, 1 to 40 filters, 16 to 1100 rows, 96 to 2048 columns, float32 and bfloat16):
+//  * input pixels over filters (eight at most): below 2^17.5 the chain is all there is (8 planes of
+//    17 x 100 with 40 filters 22 us by the workspace, 104 by snapshots; 1 of 96 x 256 with 8, 23
+//    against 35; 16 of 200 x 252 with 8, 36 against 44), above it the workspace's bytes count
+//    (8 of 300 x 700 with 16 filters, 101 against 83);
+//  * fewer than 24 rows leave too much of a group's 8 rows empty (86 of 17 x 1212 with 8: 62 against 83);
+//  * a last round of workgroups that is nearly empty costs what the workspace does while rounds times
+//    filters is small (15 of 552 x 1124 with one filter 46 against 63, 479 of 69 x 100 with two 37
+//    against 46, 99 of 186 x 96 with four 40 against 50): one round, or four over all filters.
+// By this rule 2.5 % of the shapes are more than 3 % slower than by the workspace; without it 44 % were.
+bool snapshots_pay(int64_t planes, int F, int h, int w) {
+    if (!switches().input_from_snapshots || F < 1 || !consecutive_rows(w)) return false;
+    if (switches().snapshots_any_shape) return true;
+    const int64_t pixels = planes * h * w;
+    if (h < 24 || pixels < 180000 * static_cast<int64_t>(std::min(F, 8))) return false;
+    // resident: three waves per SIMD, ten workgroups of one wave by their LDS. Of two workgroups of five or
+    // six waves on a CU the second slows the first by as much as it brings: they count as two rounds
+    const int waves = consecutive_threads(w) / 64;
+    const int64_t workgroups = planes * ((h + 7) / 8), resident = 256 * (waves == 1 ? 10 : 12 / waves);
+    return workgroups <= (waves > 4 ? 256 : resident) || workgroups * F >= 4 * resident;
 }
 
 }  // namespace boxconv

@@ -1522,10 +1522,6 @@ inline bool consecutive_rows(int w) {
     return switches().stream_consecutive &&
            (exact_fit || (switches().stream_consecutive_partial && lanes * 8 >= cnt * 3 && !(rc.full && rc.K == 1)));
 }
-template <class TG>
-bool stream_consecutive_applies(const TG* grad_out, int w) {
-    return consecutive_rows(w) && reinterpret_cast<uintptr_t>(grad_out) % (4 * sizeof(TG)) == 0;
-}
 
 // The launches of grad_output_stream_consec_kernel (`lanes` busy lanes of a workgroup of `cnt`;
 // SCAN = false: parameter sums only). Its instantiations are translation units of their own
@@ -1633,7 +1629,7 @@ hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxPara
     if constexpr (std::is_same<T, float>::value) {
         const int lanes = d.w / 4;
         const int cnt = consecutive_threads(d.w);
-        if (params && acc_slots > 0 && stream_consecutive_applies(grad_out, d.w)) {
+        if (params && acc_slots > 0 && consecutive_rows(d.w) && quads_aligned(grad_out, sizeof(TG))) {
             if (snapshots != nullptr) {
                 a.snap_shift = snapshots->shift; a.snap_groups = snapshots->groups; a.snap_bands = sp.nb;
                 return grad_output_stream_consec_launch<TG, kStreamSnapshots>(a, lanes, cnt, exact, grid, stream);

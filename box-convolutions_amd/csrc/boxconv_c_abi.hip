@@ -101,7 +101,8 @@ bool reverse_second_pass() { return boxconv::switches().bwd_reverse; }
 //                                                              only if parameter gradients are wanted
 struct BackwardLayout {
     size_t gint_off, aux_off, acc_off, total;
-    int acc_slots;        // > 0: per-workgroup accumulation slots per (plane, filter), see grad_output_stream_launch
+    int acc_slots;        // > 0: per-workgroup accumulation slots per (plane, filter), see
+                          // grad_output_stream_launch (room for; a grad_output that is not aligned takes fewer)
     bool streaming;       // grad_output_stream_kernel usable for this shape
 };
 
@@ -109,7 +110,8 @@ BackwardLayout backward_layout(int batch, int in_planes, int num_filters, int h,
                                int elem_size, bool need_input, bool need_params) {
     BackwardLayout L{};
     const int64_t planes = std::max<int64_t>(static_cast<int64_t>(batch) * in_planes, 1);
-    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, elem_size, need_params);
+    const bool sums_only = need_params && (!need_input || boxconv::snapshots_pay(planes, num_filters, h, w));
+    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, elem_size, sums_only);
     L.streaming = sp.usable;
     size_t off = 0;
     L.gint_off = off;
@@ -378,23 +380,27 @@ int backward_impl(const T* integ, const T* x_min, const T* x_max, const T* y_min
         if (int rc = hip_result(boxconv::grad_params_begin(acc, n_boxes, s), "accumulator clear"))
             return rc;
 
+    const int64_t planes = static_cast<int64_t>(batch) * in_planes;
+    const boxconv::Dims d{in_planes, num_filters, h, w, planes, 0};
+    const bool sums_only = need_params && boxconv::quads_aligned(grad_output, kSameType ? sizeof(T) : 2) &&
+                           (!need_input || boxconv::snapshots_pay(planes, num_filters, h, w));
+    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(std::max<int64_t>(planes, 1) * num_filters, h, w,
+                                                                    sizeof(T), sums_only);
+    const int acc_slots = L.acc_slots > 0 ? sp.nb * sp.parts : 0;
     const int grad_dtype = std::is_same<TG, T>::value ? 0 : std::is_same<TG, boxconv::f16_t>::value ? 1 : 2;
-    const boxconv::ParamFinish<T> finish{acc, batch, L.acc_slots, {gx_min, gx_max, gy_min, gy_max},
+    const boxconv::ParamFinish<T> finish{acc, batch, acc_slots, {gx_min, gx_max, gy_min, gy_max},
                                          n_boxes, reparam_h, reparam_w, normalize != 0, exact != 0,
                                          integ, grad_output, grad_dtype, h, w, num_filters};
     bool finished = false;
-    const int64_t planes = static_cast<int64_t>(batch) * in_planes;
-    const boxconv::Dims d{in_planes, num_filters, h, w, planes, 0};
     if (L.streaming) {
         // one pass over grad_output: parameter sums + column workspace, then grad_input, whose
         // launch finishes the parameter gradients on the side
-        const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, sizeof(T), need_params);
         boxconv::SnapshotPlan snap{};
         if constexpr (std::is_same<T, float>::value)
             if (need_input && need_params && nout > 0)
                 snap = boxconv::plan_snapshots<TG>(grad_output, sp, d);
         if (int rc = hip_result(boxconv::grad_output_stream_launch<T, TG>(
-                integ, grad_output, prm, acc, L.acc_slots, gint, sp, snap.use ? &snap : nullptr, d, exact != 0, s),
+                integ, grad_output, prm, acc, acc_slots, gint, sp, snap.use ? &snap : nullptr, d, exact != 0, s),
                 "grad_output streaming launch"))
             return rc;
         if constexpr (std::is_same<T, float>::value)

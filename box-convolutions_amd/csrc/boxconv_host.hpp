@@ -130,8 +130,13 @@ struct StreamPlan {
     int parts;               // workgroups that share a band for the parameter sums (1, or 2 for rows
                              // wider than 2048 columns): accumulation slots per (plane, filter) = nb * parts
 };
-// params: the parameter sums are wanted (the bands, i.e. the slots per (plane, filter), depend on it)
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool params);
+// sums_only: the parameter sums are wanted and no column workspace (at most snapshots): the bands,
+// i.e. the slots per (plane, filter), depend on it, and are then at least as many as otherwise.
+StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool sums_only);
+// Whether a grad_output is aligned for the kernels whose lanes read 4 consecutive columns.
+inline bool quads_aligned(const void* grad_out, size_t elem_size) {
+    return reinterpret_cast<uintptr_t>(grad_out) % (4 * elem_size) == 0;
+}
 
 // Where the gradient w.r.t. the input is formed from grad_output itself (grad_input_taps_launch):
 // instead of the column workspace the pass then leaves sums of grad_output's rows at the rows
@@ -140,6 +145,8 @@ struct SnapshotPlan {
     bool use;
     int shift, groups;
 };
+// Whether that is the faster way for float sums of an image of this size (both gradients wanted).
+bool snapshots_pay(int64_t planes, int F, int h, int w);
 template <class TG>
 SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d);
 template <class TG>
@@ -221,6 +228,7 @@ struct Switches {
     bool stream_narrow_double;  // BOXCONV_STREAM_F64_NARROW=0 clears it: float64 rows with three or four columns per lane and one launch like float32
     bool interleave_workspace;  // BOXCONV_M_INTERLEAVE=0 clears it: rows of the column workspace in their natural order
     bool input_from_snapshots;  // BOXCONV_GI_SNAPSHOTS=0 clears it: grad_input from the column workspace only
+    bool snapshots_any_shape;   // BOXCONV_GI_SNAPSHOTS=2: from snapshots for every shape that way covers
     bool forward_quads;       // BOXCONV_FWD_QUADS=0 clears it: no forward kernel with four consecutive columns per lane
     int stream_workgroups;    // BOXCONV_STREAM_WGS: workgroups the grad_output pass aims for when it cuts planes into bands (2048)
     int spin_limit;           // BOXCONV_INTEGRAL_SPIN: polls of a hand-over word before re-summing (64)

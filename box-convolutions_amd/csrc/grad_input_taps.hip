@@ -324,8 +324,8 @@ SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d) {
     plan.shift = waves16 >= 2048 ? 4 : 3;
     plan.groups = (d.h + (1 << plan.shift) - 1) >> plan.shift;
     // (the last condition: the snapshots fit where the column workspace would be)
-    plan.use = switches().input_from_snapshots && sp.usable && sp.parts == 1 && d.F > 0 &&
-               stream_consecutive_applies(grad_out, d.w) && 2 * plan.groups + sp.nb + 1 <= d.h + 1;
+    plan.use = snapshots_pay(d.planes, d.F, d.h, d.w) && sp.usable && sp.parts == 1 &&
+               quads_aligned(grad_out, sizeof(TG)) && 2 * plan.groups + sp.nb + 1 <= d.h + 1;
     return plan;
 }
 

@@ -562,8 +562,8 @@ def test_clip_parameters_matches_oracle(hip, oracle):
     (256, 1, 113, 160), (128, 2, 129, 260), (64, 1, 250, 516), (40, 3, 210, 1024), (33, 2, 257, 1400)])
 def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact):
     """grad_input formed from grad_output itself and the snapshots of its column sums (rows of a
-    multiple of four columns) against the oracle, and against the column workspace
-    (BOXCONV_GI_SNAPSHOTS=0): the two differ in the order of float32 additions, i.e. by a few units
+    multiple of four columns; BOXCONV_GI_SNAPSHOTS=2: launches of any size) against the oracle, and
+    against the column workspace (BOXCONV_GI_SNAPSHOTS=0): the two differ in the order of float32 additions, i.e. by a few units
     in the last place of the largest partial sum. The boxes hang over every edge, so the rows where
     the groups start clamp to both ends of the image. Parameter gradients keep their bits."""
     rng = np.random.default_rng(planes + F + h + w)
@@ -574,7 +574,7 @@ def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact
         boxes[1] = np.maximum(boxes[1], np.ceil(boxes[0]) + 1).astype(np.float32)
         boxes[3] = np.maximum(boxes[3], np.ceil(boxes[2]) + 1).astype(np.float32)
     results = []
-    for variant in (None, "0"):
+    for variant in ("2", "0"):
         switches("BOXCONV_GI_SNAPSHOTS", variant)
         if planes <= 2:
             cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, True, exact, g)
@@ -586,6 +586,37 @@ def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact
     assert np.abs(a[0] - b[0]).max() <= 4e-6 * np.abs(b[0]).max()
     for p, q in zip(a[1:], b[1:]):
         assert np.array_equal(p, q)
+
+
+def launches(hip, kernel, call):
+    """How often `kernel` is launched by `call`."""
+    hip.profile_arm(kernel)
+    call()
+    return hip.profile_collect()[1]
+
+
+@pytest.mark.parametrize("snapshots,planes,F,h,w", [
+    (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
+    # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
+    (False, 8, 40, 17, 100), (False, 1, 8, 96, 256), (False, 16, 8, 200, 252), (False, 2, 1, 64, 1024),
+    (False, 86, 8, 17, 1212), (False, 15, 1, 552, 1124), (False, 479, 2, 69, 100), (False, 16, 8, 512, 514)])
+def test_snapshots_only_where_they_pay(hip, switches, snapshots, planes, F, h, w):
+    """The launches for which snapshots are the slower way keep the column workspace, and then
+    return what BOXCONV_GI_SNAPSHOTS=0 returns, bit for bit."""
+    rng = np.random.default_rng(h + w)
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    g = torch.randn(1, planes * F, h, w, device="cuda")
+    boxes = [dev(b) for b in make_boxes(rng, planes, F, h, w, "inside")]
+
+    def backward():
+        return hip.box_convolution_backward(integ, *boxes, g, None, 1.0, 1.0, True, True, True, True, True, True, True)
+    assert launches(hip, "grad_input_taps", backward) == snapshots
+    assert launches(hip, "grad_input_cols", backward) == (not snapshots)
+    if not snapshots:
+        got = backward()
+        switches("BOXCONV_GI_SNAPSHOTS", "0")
+        for a, b in zip(got, backward()):
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("spin", [None, "0"])
