@@ -112,14 +112,17 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
     const RowConfig rc = stream_row_config(std::max(w, 1), elem_size);
     sp.usable = row_kernels_apply(h, w, elem_size) &&
                 stream_lds_bytes(rc.K, rc.nt, elem_size) <= kMaxDynamicLds;
+    int nb = bands_for(std::max<int64_t>(planes_f, 1), h, 32, switches().stream_workgroups);
     // Parameter sums of rows that one wave covers at four columns per lane: four such workgroups
-    // fit every SIMD and the band's chain of row pairs is what they wait for, so twice as many
-    // (256 x 4 planes of 128 x 256 in bfloat16, bands of 64 -> 32 rows: 40 -> 30 us, and 28 -> 29 in
-    // the grad-input pass, which adds up more bands). Wider rows lose there what they gain
-    // (512 x 1024: 136 -> 133 and 129 -> 138 us), and so does the pass that also leaves the column
-    // workspace (64 x 8 planes of 200 x 252, both kernels: 70 -> 82 us).
-    const bool one_wave = sums_only && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64;
-    int nb = bands_for(std::max<int64_t>(planes_f, 1), h, 32, switches().stream_workgroups * (one_wave ? 2 : 1));
+    // fit every SIMD and the band's chain of row pairs is what they wait for, so up to twice as many,
+    // but no more than fit (256 x 4 planes of 128 x 256 in bfloat16, bands of 64 -> 32 rows: 40 -> 30 us,
+    // and 28 -> 29 in the grad-input pass, which adds up more bands; but 416 planes of 661 x 204,
+    // parameter sums alone, 77 us with 5 bands, 80 with 9, 91 with 10, which are 4160 workgroups). Wider
+    // rows lose there what they gain (512 x 1024: 136 -> 133 and 129 -> 138 us), and so does the pass
+    // that also leaves the column workspace (64 x 8 planes of 200 x 252, both kernels: 70 -> 82 us).
+    if (sums_only && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64)
+        nb = std::max(nb, static_cast<int>(std::min<int64_t>(2 * switches().stream_workgroups / std::max<int64_t>(planes_f, 1),
+                                                             std::max(1, h / 32))));
     int R = (h + nb - 1) / nb;
     R += R & 1;                                        // rows are handled in pairs
     sp.R = std::max(R, 2);

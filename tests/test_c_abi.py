@@ -153,3 +153,15 @@ def test_workspace_sizes(lib):
     assert f32_4097 >= 65 * 4098 * 4
     assert 65 * 2048 * 8 <= f64_2048 < 65 * 2049 * 8
     assert f64_2049 >= 65 * 2050 * 8
+
+
+@pytest.mark.parametrize("w", [96, 204, 256])
+@pytest.mark.parametrize("planes,h", [(1, 1000), (3, 64), (64, 300), (100, 450), (416, 661), (511, 940), (1024, 128),
+                                      (1025, 512), (2100, 64), (5000, 40)])
+def test_bands_of_one_wave_rows_are_all_resident(lib, planes, h, w):
+    """Parameter sums of rows that one wave covers: four workgroups per SIMD fit the chip, 4096 in
+    all, and planes are not cut into more bands than that (a last round with a few of them cost a
+    sixth of the time). There is one slot of five doubles per (plane, band)."""
+    room = lib.boxconv_backward_workspace_bytes(1, planes, 1, h, w, 4, 0, 1)
+    bands = room // (planes * 5 * 8)
+    assert bands * planes <= max(4096, planes)
