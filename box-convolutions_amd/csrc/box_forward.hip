@@ -164,6 +164,16 @@ __global__ void __launch_bounds__(NT) forward_rows_kernel(SampleArgs<T> a, Forwa
 // the integral rows (one 16-byte load per row) as for the output (one 16- or 8-byte store per row), and
 // V sits in LDS by column modulo four (tap_run). The planes hold V[1..w]; the places in front of
 // them stay zero (V[0] = 0 and what clamps to it), those behind hold V[w].
+// The tail's residual: none, or loaded with the ordinary or the streaming cache policy.
+enum ResidualLoads { kNoResidual, kResidualCached, kResidualStreamed };
+template <bool STREAM, class TO>
+__device__ __forceinline__ Quad<TO> load_quad(const TO* p) {
+    typedef unsigned Words __attribute__((ext_vector_type(sizeof(Quad<TO>) / 4)));
+    Words v;
+    if constexpr (STREAM) v = __builtin_nontemporal_load(reinterpret_cast<const Words*>(p));
+    else v = *reinterpret_cast<const Words*>(p);     // (one expression for both would drop the policy)
+    return __builtin_bit_cast(Quad<TO>, v);
+}
 template <class TO>
 __device__ __forceinline__ void store_quad(TO* p, const Quad<TO>& q, bool stream) {
     typedef unsigned Words __attribute__((ext_vector_type(sizeof(Quad<TO>) / 4)));
@@ -172,13 +182,17 @@ __device__ __forceinline__ void store_quad(TO* p, const Quad<TO>& q, bool stream
     else *reinterpret_cast<Words*>(p) = v;
 }
 
-// RESIDUAL: the tail adds one. Without one nothing is loaded for it (loads of the output in its place,
-// dropped, cost a read as large as the output: 16 x 8 planes of 512 x 1024 in float16 153 -> 91 us, 256 x 4
-// of 128 x 256 in bfloat16, output not in any cache, 42 -> 26).
-template <class TO, int NT, bool EXACT, bool FULL, bool TAIL, bool RESIDUAL>
+// Without a residual nothing is loaded for it (loads of the output in its place, dropped, cost a read as
+// large as the output: 16 x 8 planes of 512 x 1024 in float16 153 -> 91 us, 256 x 4 of 128 x 256 in
+// bfloat16, output not in any cache, 42 -> 26). With one, the rows of the next pair are requested
+// with its integral rows: workgroups of few waves otherwise wait for memory right before the barrier
+// (residual not in any cache, 46 planes of 398 x 140 in float32 12.1 -> 10.0 us, 128 x 4 of 135 x 240
+// in bfloat16 27.7 -> 26.3); with two waves, and from five on, the registers cost more than that brings. Its cache policy: see forward_launch_any.
+template <class TO, int NT, bool EXACT, bool FULL, bool TAIL, int RESIDUAL>
 __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, ForwardTail<TO> tl) {
     using T = float;
     constexpr int K = 4, PLANE = quad_plane(NT), WAVES = NT / 64;
+    constexpr bool EARLY = RESIDUAL != kNoResidual && WAVES <= 4 && WAVES != 2;   // residual rows a pair ahead
     __shared__ __align__(16) RowPair<T> vrow[2][K][PLANE];
     const unsigned vid = xcd_contiguous_id(a.per_xcd);
     if (vid >= a.total) return;                      // whole workgroup leaves together
@@ -232,12 +246,21 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
     load_i(i0 + 1 + s.xlo, t1);
     load_i(i0 + 1 + s.xhi, b1);
     load_i(i0 + 2 + s.xhi, b2);
+    auto load_residual = [&](int i, Quad<TO>& q0, Quad<TO>& q1) {
+        const int64_t row = out0 + static_cast<int64_t>(i) * w;
+        q0 = load_quad<RESIDUAL == kResidualStreamed>(tl.residual + row + cl);
+        q1 = load_quad<RESIDUAL == kResidualStreamed>(tl.residual + (i + 1 < i1 ? row + w : row) + cl);
+    };
+    Quad<TO> res0{}, res1{};
+    if (EARLY) load_residual(i0, res0, res1);
 
     auto row_pair = [&](int i, auto prefetch_tag, auto flip_tag) {
         constexpr bool PREFETCH = decltype(prefetch_tag)::value;
         constexpr int FLIP = decltype(flip_tag)::value;
         T n0[K] = {}, n1[K] = {}, n2[K] = {}, n3[K] = {};
+        Quad<TO> m0{}, m1{};
         if (PREFETCH) {
+            if (EARLY) load_residual(i + 2, m0, m1);
             load_i(i + 2 + s.xlo, n0);
             load_i(i + 3 + s.xlo, n1);
             load_i(i + 3 + s.xhi, n2);
@@ -245,11 +268,7 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
         }
         const bool second = i + 1 < i1;
         const int64_t row0 = out0 + static_cast<int64_t>(i) * w, row1 = second ? row0 + w : row0;
-        Quad<TO> res0{}, res1{};
-        if (RESIDUAL) {
-            res0 = *reinterpret_cast<const Quad<TO>*>(tl.residual + row0 + cl);
-            res1 = *reinterpret_cast<const Quad<TO>*>(tl.residual + row1 + cl);
-        }
+        if (RESIDUAL != kNoResidual && !EARLY) load_residual(i, res0, res1);
         T v0[K], v1[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -276,8 +295,8 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
             T y0 = blend<T, EXACT>(L[k].r0, L[k + 1].r0, R[k].r0, R[k + 1].r0, s.fylo, s.fyhi) * scale;
             T y1 = blend<T, EXACT>(L[k].r1, L[k + 1].r1, R[k].r1, R[k + 1].r1, s.fylo, s.fyhi) * scale;
             if (TAIL) {
-                y0 = y0 * ch_scale + ch_shift + (RESIDUAL ? widen(res0.v[k]) : T(0));
-                y1 = y1 * ch_scale + ch_shift + (RESIDUAL ? widen(res1.v[k]) : T(0));
+                y0 = y0 * ch_scale + ch_shift + (RESIDUAL != kNoResidual ? widen(res0.v[k]) : T(0));
+                y1 = y1 * ch_scale + ch_shift + (RESIDUAL != kNoResidual ? widen(res1.v[k]) : T(0));
                 if (relu) { y0 = y0 < T(0) ? T(0) : y0; y1 = y1 < T(0) ? T(0) : y1; }
             }
             narrow(y0, z0.v[k]);
@@ -293,6 +312,7 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
                 ta[k] = t1[k]; bc[k] = b2[k];
                 t0[k] = n0[k]; t1[k] = n1[k]; b1[k] = n2[k]; b2[k] = n3[k];
             }
+            if (EARLY) { res0 = m0; res1 = m1; }
         }
     };
     int i = i0;
@@ -398,14 +418,23 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
         const size_t align = 4 * sizeof(TO);
         if (switches().forward_quads && d.w % 4 == 0 && d.w <= 2048 && (one_wave || wide_half) &&
             reinterpret_cast<uintptr_t>(tail.dst) % align == 0 && reinterpret_cast<uintptr_t>(tail.residual) % align == 0) {
+            // A residual that an earlier layer has just left in the memory-side cache is worth reading from
+            // there (256 x 4 planes of 128 x 256 in bfloat16 30 us, 40 with the streaming policy); one that
+            // does not fit it beside the output would only push that out (16-bit outputs, 16 x 8 planes of
+            // 512 x 1024 153 -> 150 us, of 720 x 1280 158 -> 149, of 1080 x 1920 335 -> 321; float32 of 128 MB
+            // and more 0.9 of the time).
+            const bool stream_residual = out_bytes > (128ull << 20);
 #define LAUNCH_FQ_TAIL(NT, EX, FU)                                                                                     \
     do {                                                                                                               \
         if constexpr (TAIL)                                                                                            \
             if (tail.residual != nullptr) {                                                                            \
-                BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, true, true>), grid, dim3(NT), 0, stream, a, tail); \
+                if (stream_residual)                                                                                   \
+                    BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualStreamed>), grid, dim3(NT), 0, stream, a, tail); \
+                else                                                                                                   \
+                    BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualCached>), grid, dim3(NT), 0, stream, a, tail); \
                 break;                                                                                                 \
             }                                                                                                          \
-        BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, TAIL, false>), grid, dim3(NT), 0, stream, a, tail); \
+        BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, TAIL, kNoResidual>), grid, dim3(NT), 0, stream, a, tail); \
     } while (0)
 #define LAUNCH_FQ(NT)                                                                                                  \
     case NT:                                                                                                           \

@@ -339,3 +339,26 @@ def test_tail_without_residual_loads_none():
         assert launches == 5
         times[name] = min(times.get(name, ms), ms)
     assert times["without"] < 0.85 * times["with"]
+
+
+@pytest.mark.parametrize("dtype,planes,F,h,w", [
+    # a residual of 128 MB and more is read with the streaming policy: one, two, four, five waves per row
+    (torch.float32, 140, 1, 1001, 244), (torch.bfloat16, 37, 4, 900, 508), (torch.float16, 9, 8, 923, 1020),
+    (torch.bfloat16, 7, 8, 955, 1276)])
+def test_large_residual(switches, dtype, planes, F, h, w):
+    from box_convolution import _native as hip
+    gen = torch.Generator(device="cuda").manual_seed(w)
+    integ = hip.integral_image(torch.randn(1, planes, h, w, generator=gen, device="cuda"))
+    lo_x, lo_y = (-torch.rand(planes, F, generator=gen, device="cuda") * n for n in (h, w))
+    boxes = (lo_x, lo_x + 3 + h // 3, lo_y, lo_y + 3 + w // 3)
+    scale, shift = (torch.randn(planes * F, generator=gen, device="cuda") for _ in range(2))
+    residual = torch.randn(1, planes * F, h, w, generator=gen, device="cuda").to(dtype)
+    assert residual.numel() * residual.element_size() > 128 << 20
+    results = []
+    for variant in (None, "0"):
+        switches("BOXCONV_FWD_QUADS", variant)
+        results.append(hip.box_convolution_forward_fused(integ, *boxes, True, True, dtype, scale, shift, residual, True))
+    a, b = (r.float() for r in results)
+    # the same expressions per pixel: one contraction of a product and a sum, or one rounding to 16 bits
+    unit = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    assert ((a - b).abs() <= unit * b.abs() + 1e-6 * b.abs().max()).all()
