@@ -356,6 +356,38 @@ __global__ void __launch_bounds__(256) forward_gather_kernel(SampleArgs<T> a, Fo
 
 }  // namespace
 
+namespace {
+
+// Rows that one wave covers: where four consecutive columns per lane (forward_quads_kernel) are
+// faster than columns 64 apart (forward_rows_kernel), by columns, output pixels and element size.
+// Both were timed on 8000 shapes, output buffers reused and in no cache; time of the first over the
+// second:
+//  * fewer than 96 columns leave too many lanes idle; exactly 128 fill the other kernel's two waves
+//    (0.96 to 1.25);
+//  * 96 to 127 are two waves at one column per lane there, a shorter chain: 1.1 to 1.3 below 2^21
+//    pixels, 0.85 to 0.93 above;
+//  * 129 to 192 are three columns per lane there and leave fewer lanes idle: 0.87 to 0.97 below 2^22
+//    pixels, 1.0 to 1.25 above; with a residual 0.8 and 1.0 (in no cache) there too;
+//  * 193 to 256: 0.70 to 0.97. But float32 rows that start on 64-byte boundaries, which the other
+//    kernel stores best: no tail 1.0 to 1.17 from 2^22 pixels (208 to 240 columns), and 256 columns
+//    0.92 to 1.02 below 2^25 pixels, 1.0 to 1.1 above;
+//  * output and integral images that do not fit the memory-side cache together: 1.2 to 1.9 (408 x 4
+//    planes of 330 x 160 70 against 130 us, 308 x 2 of 794 x 112 62 against 101), except with a residual
+//    and for 129 columns and more that do not start on 64-byte boundaries (0.8 to 0.9).
+bool one_wave_quads_pay(int w, uint64_t pixels, uint64_t integral_bytes, size_t elem_size, bool tail, bool residual) {
+    if (w < 96) return false;
+    if (switches().quads_any_size) return true;
+    if (w == 128) return false;
+    const bool whole_sectors = static_cast<size_t>(w) * elem_size % 64 == 0;
+    if (!residual && pixels * elem_size + integral_bytes >= (256ull << 20)) return w > 128 && !whole_sectors;
+    if (w < 128) return pixels >= (1ull << 21);
+    if (w <= 192) return residual || pixels < (1ull << 22);
+    if (elem_size == 4 && whole_sectors) return w == 256 ? pixels < (1ull << 25) : tail || pixels < (1ull << 22);
+    return true;
+}
+
+}  // namespace
+
 // TAIL selects the kernels with the fused tail; without it only tail.dst is used.
 template <class T, class TO, bool TAIL>
 hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> tail, Dims d,
@@ -402,18 +434,17 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
     a.stream_out = ((static_cast<uint64_t>(d.w) * sizeof(TO)) % 64 == 0 || out_bytes > (256ull << 20)) ? 1 : 0;
     const dim3 grid(static_cast<unsigned>(a.per_xcd * kXcds));
     if constexpr (std::is_same<T, float>::value) {
-        // Four consecutive columns per lane: rows of one wave (up to 256 columns, at least three
-        // eighths of its lanes busy), and 16-bit outputs of wider rows, where the other kernel stores
-        // 2 bytes per lane. Measured, us, other kernel -> this one: float32 32 x 4 planes of
-        // 128 x 256 x 4 15.5 -> 14.8, 135 x 240 19.6 -> 16.3, with the tail 32.2 -> 25.0, 36.6 -> 25.1;
-        // bfloat16 with the tail 26.2 -> 17.4, 30.2 -> 18.9 (x 8: 51.6 -> 30.7), 16 x 8 planes of 300 x 768
-        // 74 -> 47, 1080 x 1920 380 -> 356; without it 512 x 1024 118 -> 90, 720 x 1280 97 -> 76. Not for
-        // wider float32 rows (256 x 512 54 -> 72, 720 x 1280 105 -> 111, 1080 x 1920 229 -> 373: stores of
-        // 16 bytes per lane reach the memory no better, and the loads start at odd addresses), nor
-        // without a tail beyond 1280 columns (1080 x 1920 213 -> 237) or where an eighth of the
-        // lanes idles (200 x 384 27 -> 31).
+        // Four consecutive columns per lane: rows of one wave where one_wave_quads_pay says so, and
+        // 16-bit outputs of wider rows, where the other kernel stores 2 bytes per lane. Measured, us, other
+        // kernel -> this one: bfloat16 16 x 8 planes of 300 x 768 with the tail 74 -> 50, 1080 x 1920 380 -> 321;
+        // without it 512 x 1024 118 -> 90, 720 x 1280 97 -> 76. Not for wider float32 rows (256 x 512 54 -> 72,
+        // 720 x 1280 105 -> 111, 1080 x 1920 229 -> 373: stores of 16 bytes per lane reach the memory no
+        // better, and the loads start at odd addresses), nor without a tail beyond 1280 columns
+        // (1080 x 1920 213 -> 237) or where an eighth of the lanes idles (200 x 384 27 -> 31).
         const int lanes = d.w / 4, cnt = consecutive_threads(d.w);
-        const bool one_wave = cnt == 64 && lanes * 8 >= cnt * 3;
+        const uint64_t integral_bytes = static_cast<uint64_t>(d.planes) * (d.h + 1) * (d.w + 1) * sizeof(T);
+        const bool one_wave = cnt == 64 && one_wave_quads_pay(d.w, static_cast<uint64_t>(planes_f) * d.hw(), integral_bytes,
+                                                              sizeof(TO), TAIL, tail.residual != nullptr);
         const bool wide_half = sizeof(TO) == 2 && cnt > 64 && (TAIL || (d.w <= 1280 && lanes * 8 >= cnt * 7));
         const size_t align = 4 * sizeof(TO);
         if (switches().forward_quads && d.w % 4 == 0 && d.w <= 2048 && (one_wave || wide_half) &&
@@ -429,12 +460,12 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
         if constexpr (TAIL)                                                                                            \
             if (tail.residual != nullptr) {                                                                            \
                 if (stream_residual)                                                                                   \
-                    BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualStreamed>), grid, dim3(NT), 0, stream, a, tail); \
+                    BOXCONV_LAUNCH("forward_quads", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualStreamed>), grid, dim3(NT), 0, stream, a, tail); \
                 else                                                                                                   \
-                    BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualCached>), grid, dim3(NT), 0, stream, a, tail); \
+                    BOXCONV_LAUNCH("forward_quads", (forward_quads_kernel<TO, NT, EX, FU, true, kResidualCached>), grid, dim3(NT), 0, stream, a, tail); \
                 break;                                                                                                 \
             }                                                                                                          \
-        BOXCONV_LAUNCH("forward_rows", (forward_quads_kernel<TO, NT, EX, FU, TAIL, kNoResidual>), grid, dim3(NT), 0, stream, a, tail); \
+        BOXCONV_LAUNCH("forward_quads", (forward_quads_kernel<TO, NT, EX, FU, TAIL, kNoResidual>), grid, dim3(NT), 0, stream, a, tail); \
     } while (0)
 #define LAUNCH_FQ(NT)                                                                                                  \
     case NT:                                                                                                           \

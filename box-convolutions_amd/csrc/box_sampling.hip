@@ -38,6 +38,8 @@ Switches read_switches() {
     s.stream_narrow_double = flag_unless_zero("BOXCONV_STREAM_F64_NARROW");
     s.interleave_workspace = flag_unless_zero("BOXCONV_M_INTERLEAVE");
     s.forward_quads = flag_unless_zero("BOXCONV_FWD_QUADS");
+    e = text("BOXCONV_FWD_QUADS");
+    s.quads_any_size = e != nullptr && std::atoi(e) == 2;
     s.input_from_snapshots = flag_unless_zero("BOXCONV_GI_SNAPSHOTS");
     e = text("BOXCONV_GI_SNAPSHOTS");
     s.snapshots_any_shape = e != nullptr && std::atoi(e) == 2;

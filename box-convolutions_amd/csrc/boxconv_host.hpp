@@ -230,6 +230,7 @@ struct Switches {
     bool input_from_snapshots;  // BOXCONV_GI_SNAPSHOTS=0 clears it: grad_input from the column workspace only
     bool snapshots_any_shape;   // BOXCONV_GI_SNAPSHOTS=2: from snapshots for every shape that way covers
     bool forward_quads;       // BOXCONV_FWD_QUADS=0 clears it: no forward kernel with four consecutive columns per lane
+    bool quads_any_size;      // BOXCONV_FWD_QUADS=2: that kernel for rows of one wave in launches of any size
     int stream_workgroups;    // BOXCONV_STREAM_WGS: workgroups the grad_output pass aims for when it cuts planes into bands (2048)
     int spin_limit;           // BOXCONV_INTEGRAL_SPIN: polls of a hand-over word before re-summing (64)
     int fwd_threads;          // BOXCONV_FWD_THREADS: 256 or 512 (512)

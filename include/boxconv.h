@@ -54,7 +54,7 @@ void boxconv_reload_env(void);
  * boxconv_profile_arm(name): from now on every launch of the kernel called `name` is bracketed by
  * a pair of HIP events recorded on the stream it is launched on (so the time is that kernel's
  * alone, whatever else the entry point launches). Names: "band_colsum", "band_prefix",
- * "band_scan", "forward_rows", "grad_output_stream", "grad_input_cols",
+ * "band_scan", "forward_rows", "forward_quads", "grad_output_stream", "grad_input_cols",
  * "param_grad_finalize", "fill_zero", "fill_marker", "clip", "forward_gather", "grad_input_gather",
  * "int_row_prefix", "int_col_prefix", "probe_copy_bands", "probe_grad_input_pattern",
  * "grad_params_gather".

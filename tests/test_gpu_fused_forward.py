@@ -291,7 +291,7 @@ def test_forward_fused_modes_and_double_input():
     (torch.float16, 9, 2048)])
 def test_forward_with_consecutive_columns(switches, dtype, h, w, tail, exact):
     """The forward kernel with four consecutive columns per lane against the one with wave-strided
-    columns (BOXCONV_FWD_QUADS=0): the same expressions per pixel, so at most the contraction of a
+    columns (BOXCONV_FWD_QUADS=2, whatever the size, and =0): the same expressions per pixel, so at most the contraction of a
     product and a sum differs, a unit in the last place of float32 or one rounding to 16 bits.
     Boxes hang over every edge; without a residual the output's memory holds NaN beforehand."""
     from box_convolution import _native as hip
@@ -309,11 +309,13 @@ def test_forward_with_consecutive_columns(switches, dtype, h, w, tail, exact):
         variants = [(scale, shift, residual, True), (scale, None, None, True)]
     for args in variants:
         results = []
-        for variant in (None, "0"):
+        for variant in ("2", "0"):
             switches("BOXCONV_FWD_QUADS", variant)
             filler = torch.full((B, C * F, h, w), float("nan"), device="cuda", dtype=dtype)
             del filler                                   # (the allocator hands this block out next)
+            hip.profile_arm("forward_quads")
             results.append(hip.box_convolution_forward_fused(integ, *boxes, True, exact, dtype, *args).float())
+            assert hip.profile_collect()[1] == (variant == "2" and (tail or w != 1284 and w != 2048))
         a, b = results
         assert torch.isfinite(a).all()
         unit = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
@@ -332,7 +334,7 @@ def test_tail_without_residual_loads_none():
     residual = torch.randn(B, C * F, h, w, device="cuda").half()
     times = {}
     for name, res in (("with", residual), ("without", None), ("with", residual), ("without", None)):
-        hip.profile_arm("forward_rows")
+        hip.profile_arm("forward_quads")
         for _ in range(5):
             hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, torch.float16, scale, shift, res, True)
         ms, launches = hip.profile_collect()
@@ -362,3 +364,27 @@ def test_large_residual(switches, dtype, planes, F, h, w):
     # the same expressions per pixel: one contraction of a product and a sum, or one rounding to 16 bits
     unit = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
     assert ((a - b).abs() <= unit * b.abs() + 1e-6 * b.abs().max()).all()
+
+
+@pytest.mark.parametrize("quads,dtype,planes,h,w,tail", [
+    # 96 to 127 columns from 2^21 pixels on, never 128; 129 to 192 below 2^22; above with a residual
+    (False, torch.float32, 19, 59, 96, None), (True, torch.float32, 219, 100, 96, None),
+    (False, torch.float32, 219, 100, 128, None), (True, torch.float32, 100, 200, 192, None),
+    (False, torch.float32, 150, 200, 160, None), (True, torch.float32, 150, 200, 160, "residual"),
+    (False, torch.bfloat16, 150, 200, 160, None),
+    # float32 rows that start on 64-byte boundaries, and others
+    (True, torch.float32, 90, 200, 224, None), (False, torch.float32, 110, 200, 224, None),
+    (True, torch.float32, 110, 200, 224, "relu"), (True, torch.float32, 110, 200, 220, None),
+    (True, torch.bfloat16, 110, 200, 224, None), (True, torch.float32, 512, 128, 256, None),
+    # 256 MB and more of output and integral images
+    (False, torch.float32, 140, 1000, 256, None), (False, torch.float32, 262, 1000, 256, None), (False, torch.float32, 600, 1000, 112, None),
+    (True, torch.float32, 320, 1000, 212, None)])
+def test_consecutive_columns_only_where_they_pay(quads, dtype, planes, h, w, tail):
+    """Rows of one wave: which forward kernel takes them, by columns and output pixels."""
+    from box_convolution import _native as hip
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    lo = torch.full((planes, 1), -3.25, device="cuda")
+    residual = torch.randn(1, planes, h, w, device="cuda").to(dtype) if tail == "residual" else None
+    hip.profile_arm("forward_quads")
+    hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, dtype, None, None, residual, tail == "relu")
+    assert hip.profile_collect()[1] == quads
