@@ -404,12 +404,29 @@ clip_and_fill_marker_kernel(ClipArgs<T> clip, int clip_blocks, unsigned long lon
 
 // How band_scan_lookback_kernel reads a row.
 enum RowLoads {
-    kElements,      // element by element (16-bit rows that are not aligned; rows of fewer than 4 columns)
+    kElements,      // element by element (elements that are not aligned; rows of fewer than 4 columns)
     kAlignedQuads,  // rows of a multiple of four columns, 16-byte (8-byte) aligned: one load per lane
-    kShiftedQuads,  // any other float row: one 16-byte load per lane from a dword-aligned address. The lane
+    kShiftedQuads,  // any other row: one load per lane from an address that is aligned to the element. The lane
                     // whose four columns straddle the row's end reads the row's last four columns
                     // and shifts them; nothing outside the row is touched
 };
+
+// Four consecutive elements from an address that is aligned to the element only, one load (16 or 8
+// bytes; a global load need not be aligned here).
+__device__ __forceinline__ void load_quad_unaligned(const float* p, float (&v)[4]) {
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    const f4 q = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+template <class H>
+__device__ __forceinline__ void load_quad_unaligned(const H* p, float (&v)[4]) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2), aligned(2)));
+    const u2 q = __builtin_nontemporal_load(reinterpret_cast<const u2*>(p));
+    f16_t raw[4];
+    unpack_quad(q.x, q.y, raw);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = widen(H{raw[k].bits});
+}
 
 template <class TI, int WAVES, int RB, int LOADS, bool FULL>
 __global__ void __launch_bounds__(WAVES * 64)
@@ -461,11 +478,9 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
                 for (int v = 0; v < 4; ++v) x[v] = T(0);
             }
         } else if constexpr (LOADS == kShiftedQuads) {
-            typedef float f4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
-            const f4_dword_aligned q = __builtin_nontemporal_load(reinterpret_cast<const f4_dword_aligned*>(
-                src + static_cast<int64_t>(min(row, h - 1)) * w + lane_col));
+            load_quad_unaligned(src + static_cast<int64_t>(min(row, h - 1)) * w + lane_col, x);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) x[v] = exists ? q[v] : T(0);
+            for (int v = 0; v < 4; ++v) x[v] = exists ? x[v] : T(0);
         } else {
             buffer_load_run_as<kCacheStream, TI>(x, irows.row(min(row, h - 1), exists), in_off);
         }
@@ -896,13 +911,8 @@ hipError_t launch_lookback(const TI* in, float* out, double* aux, int64_t planes
     if (aligned_for_vec4(in, w)) {
         LAUNCH_LOOKBACK(kAlignedQuads, true);
     } else {
-        if constexpr (std::is_same<TI, float>::value) {
-            if (w >= 4 && reinterpret_cast<uintptr_t>(in) % sizeof(float) == 0) {
-                LAUNCH_LOOKBACK(kShiftedQuads, false);
-                return hipGetLastError();
-            }
-        }
-        LAUNCH_LOOKBACK(kElements, false);
+        if (w >= 4 && reinterpret_cast<uintptr_t>(in) % sizeof(TI) == 0) LAUNCH_LOOKBACK(kShiftedQuads, false);
+        else LAUNCH_LOOKBACK(kElements, false);
     }
 #undef LAUNCH_LOOKBACK
     return hipGetLastError();
@@ -1038,9 +1048,8 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // 1080 x 1920, 34 bands per plane, 117 against 80.)
     // Rows of other widths (kShiftedQuads), only where all workgroups are resident, which also bounds
     // the workspace: 64 planes of 270 x 481 39 -> 25 us, 16 of 301 x 767 33 -> 20, 16 of 500 x 1001
-    // 38 -> 27, 8 of 1000 x 2001 65 -> 40, 32 of 200 x 257 20 -> 16; in bfloat16 (element loads) 35 -> 28,
-    // 27 -> 20, 34 -> 27, 55 -> 42, 19 -> 18, and 12 of 700 x 1401 50 -> 56, of which a training or eval
-    // forward gets a launch back (the clip's launch also marks the hand-over words).
+    // 38 -> 27, 8 of 1000 x 2001 65 -> 41, 12 of 700 x 1401 57 -> 49; in bfloat16 35 -> 25, 27 -> 21, 34 -> 26,
+    // 56 -> 37, 50 -> 49 (28, 21, 27, 43 and 56 with element loads).
     // Narrower rows leave most of a wave idle in either kernel; the two passes are faster there
     // (64 x 128: 20 against 24 us, 135 x 240: 21 against 25).
     const bool all_resident = groups <= resident && bands32 <= 32;

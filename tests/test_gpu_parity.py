@@ -620,21 +620,25 @@ def test_snapshots_only_where_they_pay(hip, switches, snapshots, planes, F, h, w
 
 
 @pytest.mark.parametrize("spin", [None, "0"])
-@pytest.mark.parametrize("planes,h,w", [(3, 40, 257), (2, 33, 258), (5, 70, 259), (16, 301, 767), (64, 65, 481),
-                                        (1, 97, 1021), (2, 100, 1537), (1, 64, 2047)])
-def test_integral_image_single_pass_of_odd_rows(hip, switches, planes, h, w, spin):
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("planes,h,w,single", [
+    (3, 40, 257, True), (2, 33, 258, True), (16, 301, 767, True), (64, 65, 481, True), (1, 97, 1021, True),
+    (2, 100, 1537, True), (1, 64, 2047, True)])
+def test_integral_image_single_pass_of_odd_rows(hip, switches, dtype, planes, h, w, single, spin):
     """Rows of 256 columns and more that are not a multiple of four columns: the single pass reads
-    them with 16-byte loads that start anywhere, the lane at the row's end from the row's last four
-    columns. The two passes (BOXCONV_INTEGRAL_LOOKBACK=1) may cut the planes into other bands, i.e.
-    associate the double sums differently; spin = 0 sums every band above again."""
-    x = torch.randn(1, planes, h, w, generator=torch.Generator().manual_seed(h * w)).cuda()
+    them with loads of four elements that start anywhere, the lane at the row's end from the row's
+    last four columns. Against the two passes (BOXCONV_INTEGRAL_LOOKBACK=1), which may cut
+    the planes into other bands, i.e. associate the double sums differently; spin = 0 sums every band above again."""
+    x = torch.randn(1, planes, h, w, generator=torch.Generator().manual_seed(h * w)).cuda().to(dtype)
     switches("BOXCONV_INTEGRAL_LOOKBACK", "1")
     two = hip.integral_image(x).clone()
     switches("BOXCONV_INTEGRAL_LOOKBACK", None)
     switches("BOXCONV_INTEGRAL_SPIN", spin)
     one = hip.integral_image(x)
+    assert launches(hip, "band_colsum", lambda: hip.integral_image(x)) == (not single)
+    assert launches(hip, "fill_marker", lambda: hip.integral_image(x)) == single
     assert torch.allclose(one, two, rtol=2e-7, atol=0)
-    want = np.cumsum(np.cumsum(x.cpu().numpy().astype(np.float64), axis=2), axis=3)
+    want = np.cumsum(np.cumsum(x.double().cpu().numpy(), axis=2), axis=3)
     got = one.cpu().numpy()
     assert not got[:, :, 0].any() and not got[..., 0].any()
     # a float32 rounding of a double sum: half a unit in the last place of the largest entry
