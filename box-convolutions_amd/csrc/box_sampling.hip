@@ -28,7 +28,6 @@ Switches read_switches() {
     e = text("BOXCONV_INTEGRAL_LOOKBACK");
     s.lookback = e == nullptr || std::atoi(e) != 0;
     s.lookback_any_shape = e != nullptr && std::atoi(e) == 2;
-    s.lookback_quads_only = e != nullptr && std::atoi(e) == 1;
     s.plane_integral = flag_unless_zero("BOXCONV_INTEGRAL_PLANE");
     s.stream_consecutive = flag_unless_zero("BOXCONV_STREAM_CONSEC");
     {

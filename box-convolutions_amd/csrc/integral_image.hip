@@ -1053,8 +1053,7 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // Narrower rows leave most of a wave idle in either kernel; the two passes are faster there
     // (64 x 128: 20 against 24 us, 135 x 240: 21 against 25).
     const bool all_resident = groups <= resident && bands32 <= 32;
-    const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096
-                                                         : all_resident && !switches().lookback_quads_only);
+    const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096 : all_resident);
     const bool single_pass = wanted >= 2 && h > kLookbackRows && w <= 2048 && scan_by_rows(h, w, sizeof(float)) &&
                              bands32 <= kLookbackBands && (lookback_any_shape() || measured_faster);
     if (single_pass) nb = (h + kLookbackRows - 1) / kLookbackRows;

@@ -627,10 +627,10 @@ def test_snapshots_only_where_they_pay(hip, switches, snapshots, planes, F, h, w
 def test_integral_image_single_pass_of_odd_rows(hip, switches, dtype, planes, h, w, single, spin):
     """Rows of 256 columns and more that are not a multiple of four columns: the single pass reads
     them with loads of four elements that start anywhere, the lane at the row's end from the row's
-    last four columns. Against the two passes (BOXCONV_INTEGRAL_LOOKBACK=1), which may cut
-    the planes into other bands, i.e. associate the double sums differently; spin = 0 sums every band above again."""
+    last four columns. Against the two passes on the same bands (BOXCONV_INTEGRAL_LOOKBACK=0), which
+    associate the double sums differently; spin = 0 sums every band above again."""
     x = torch.randn(1, planes, h, w, generator=torch.Generator().manual_seed(h * w)).cuda().to(dtype)
-    switches("BOXCONV_INTEGRAL_LOOKBACK", "1")
+    switches("BOXCONV_INTEGRAL_LOOKBACK", "0")
     two = hip.integral_image(x).clone()
     switches("BOXCONV_INTEGRAL_LOOKBACK", None)
     switches("BOXCONV_INTEGRAL_SPIN", spin)
@@ -643,3 +643,10 @@ def test_integral_image_single_pass_of_odd_rows(hip, switches, dtype, planes, h,
     assert not got[:, :, 0].any() and not got[..., 0].any()
     # a float32 rounding of a double sum: half a unit in the last place of the largest entry
     assert np.abs(got[:, :, 1:, 1:] - want).max() <= 2.0 ** -24 * 1.01 * np.abs(want).max()
+
+
+def test_integral_image_switch_one_is_the_default(hip, switches):
+    """BOXCONV_INTEGRAL_LOOKBACK=1 takes the single pass where the default does, odd widths included."""
+    x = torch.randn(1, 16, 301, 767, device="cuda")
+    switches("BOXCONV_INTEGRAL_LOOKBACK", "1")
+    assert launches(hip, "fill_marker", lambda: hip.integral_image(x)) == 1
