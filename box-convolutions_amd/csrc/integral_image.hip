@@ -1049,11 +1049,16 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // Rows of other widths (kShiftedQuads), only where all workgroups are resident, which also bounds
     // the workspace: 64 planes of 270 x 481 39 -> 25 us, 16 of 301 x 767 33 -> 20, 16 of 500 x 1001
     // 38 -> 27, 8 of 1000 x 2001 65 -> 41, 12 of 700 x 1401 57 -> 49; in bfloat16 35 -> 25, 27 -> 21, 34 -> 26,
-    // 56 -> 37, 50 -> 49 (28, 21, 27, 43 and 56 with element loads).
+    // 56 -> 37, 50 -> 49 (28, 21, 27, 43 and 56 with element loads). Not below 3 << 19 pixels for images of 64 to
+    // 256 rows and up to 512 columns, which the two passes cut into bands of 16 rows (single pass
+    // against two, alone and in a training forward, where the clip's launch also marks the hand-over
+    // words: 6 planes of 64 x 505 in bfloat16 14.6 against 11.3 and 20.3 against 18.5 us, 4 of 144 x 402 in
+    // float32 15.4 against 13.2 and 21.2 against 20.4; but 32 of 200 x 257 17 against 20).
     // Narrower rows leave most of a wave idle in either kernel; the two passes are faster there
     // (64 x 128: 20 against 24 us, 135 x 240: 21 against 25).
     const bool all_resident = groups <= resident && bands32 <= 32;
-    const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096 : all_resident);
+    const bool short_bands = min_rows == 16 && w <= 512 && planes * h * w < (3 << 19);
+    const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096 : all_resident && !short_bands);
     const bool single_pass = wanted >= 2 && h > kLookbackRows && w <= 2048 && scan_by_rows(h, w, sizeof(float)) &&
                              bands32 <= kLookbackBands && (lookback_any_shape() || measured_faster);
     if (single_pass) nb = (h + kLookbackRows - 1) / kLookbackRows;

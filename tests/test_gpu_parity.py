@@ -623,7 +623,9 @@ def test_snapshots_only_where_they_pay(hip, switches, snapshots, planes, F, h, w
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("planes,h,w,single", [
     (3, 40, 257, True), (2, 33, 258, True), (16, 301, 767, True), (64, 65, 481, True), (1, 97, 1021, True),
-    (2, 100, 1537, True), (1, 64, 2047, True)])
+    (2, 100, 1537, True), (1, 64, 2047, True),
+    # few pixels of 64 to 256 rows and up to 512 columns: two passes; the first size that takes the single pass
+    (5, 70, 259, False), (9, 256, 511, False), (47, 65, 511, False), (48, 65, 511, True), (1, 64, 513, True)])
 def test_integral_image_single_pass_of_odd_rows(hip, switches, dtype, planes, h, w, single, spin):
     """Rows of 256 columns and more that are not a multiple of four columns: the single pass reads
     them with loads of four elements that start anywhere, the lane at the row's end from the row's
