@@ -388,3 +388,27 @@ def test_consecutive_columns_only_where_they_pay(quads, dtype, planes, h, w, tai
     hip.profile_arm("forward_quads")
     hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, dtype, None, None, residual, tail == "relu")
     assert hip.profile_collect()[1] == quads
+
+
+@pytest.mark.parametrize("dtype,h,w", [(torch.float32, 130, 252), (torch.bfloat16, 40, 512)])
+def test_residual_at_any_offset(switches, dtype, h, w):
+    """A residual that does not start on four elements takes the kernel with wave-strided columns and
+    returns what that kernel returns for an aligned copy, bit for bit."""
+    from box_convolution import _native as hip
+    planes = 8
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    lo = torch.full((planes, 1), -3.25, device="cuda")
+    aligned = torch.randn(1, planes, h, w, device="cuda").to(dtype)
+    shifted = torch.empty(aligned.numel() + 1, device="cuda", dtype=dtype)[1:].view_as(aligned).copy_(aligned)
+    assert shifted.data_ptr() % (4 * shifted.element_size()) != 0
+
+    def forward(residual):
+        return hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, dtype, None, None, residual, True)
+    hip.profile_arm("forward_quads")
+    got = forward(shifted)
+    assert hip.profile_collect()[1] == 0
+    hip.profile_arm("forward_quads")
+    forward(aligned)
+    assert hip.profile_collect()[1] == 1
+    switches("BOXCONV_FWD_QUADS", "0")
+    assert torch.equal(got, forward(aligned))

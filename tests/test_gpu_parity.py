@@ -554,18 +554,29 @@ def test_clip_parameters_matches_oracle(hip, oracle):
                 assert np.array_equal(host(a), b)
 
 
-@pytest.mark.parametrize("exact", [True, False])
-@pytest.mark.parametrize("planes,F,h,w", [
+def launches(hip, kernel, call):
+    """How often `kernel` is launched by `call`."""
+    hip.profile_arm(kernel)
+    call()
+    return hip.profile_collect()[1]
+
+
+SNAPSHOT_SHAPES = [
     # groups of 8 output rows: one group, a ragged last one, several bands of the grad_output pass
     (1, 2, 8, 256), (2, 1, 33, 100), (2, 3, 130, 300), (1, 4, 97, 640), (1, 2, 40, 1920), (1, 1, 50, 2048),
     # groups of 16 rows: the smallest launch that takes them, ragged rows and columns
-    (256, 1, 113, 160), (128, 2, 129, 260), (64, 1, 250, 516), (40, 3, 210, 1024), (33, 2, 257, 1400)])
-def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact):
+    (256, 1, 113, 160), (128, 2, 129, 260), (64, 1, 250, 516), (40, 3, 210, 1024), (33, 2, 257, 1400)]
+
+
+@pytest.mark.parametrize("exact,normalize", [(True, True), (False, True), (True, False)])
+@pytest.mark.parametrize("planes,F,h,w", SNAPSHOT_SHAPES)
+def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact, normalize):
     """grad_input formed from grad_output itself and the snapshots of its column sums (rows of a
-    multiple of four columns; BOXCONV_GI_SNAPSHOTS=2: launches of any size) against the oracle, and
-    against the column workspace (BOXCONV_GI_SNAPSHOTS=0): the two differ in the order of float32 additions, i.e. by a few units
-    in the last place of the largest partial sum. The boxes hang over every edge, so the rows where
-    the groups start clamp to both ends of the image. Parameter gradients keep their bits."""
+    multiple of four columns; BOXCONV_GI_SNAPSHOTS=2: launches of any size) against the oracle (the
+    groups of 8 rows up to two planes, those of 16 at their smallest launch), and against the column
+    workspace (BOXCONV_GI_SNAPSHOTS=0): the two differ in the order of float32 additions, i.e. by a few
+    units in the last place of the largest partial sum. The boxes hang over every edge, so the rows
+    where the groups start clamp to both ends of the image. Parameter gradients keep their bits."""
     rng = np.random.default_rng(planes + F + h + w)
     x = rng.standard_normal((1, planes, h, w)).astype(np.float32)
     g = (rng.standard_normal((1, planes * F, h, w)) + 0.25).astype(np.float32)
@@ -573,26 +584,50 @@ def test_grad_input_from_snapshots(hip, oracle, switches, planes, F, h, w, exact
     if not exact:
         boxes[1] = np.maximum(boxes[1], np.ceil(boxes[0]) + 1).astype(np.float32)
         boxes[3] = np.maximum(boxes[3], np.ceil(boxes[2]) + 1).astype(np.float32)
+    integ, dg, db = hip.integral_image(dev(x)), dev(g), [dev(b) for b in boxes]
     results = []
     for variant in ("2", "0"):
         switches("BOXCONV_GI_SNAPSHOTS", variant)
-        if planes <= 2:
-            cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, True, exact, g)
+
+        def backward():
+            return hip.box_convolution_backward(integ, *db, dg, None, 3.5 * h, 2.25 * w, normalize, exact,
+                                                True, True, True, True, True)
+        if planes <= 2 or planes == 256:
+            cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, normalize, exact, g)
             assert_parity(cpu, gpu, np.float32, "snapshots=%s %dx%d" % (variant, h, w), **sc)
-        back = hip.box_convolution_backward(hip.integral_image(dev(x)), *[dev(b) for b in boxes], dev(g), None,
-                                            3.5 * h, 2.25 * w, True, exact, True, True, True, True, True)
-        results.append([t.cpu().numpy() for t in back])
+        assert launches(hip, "grad_input_taps", backward) == (variant == "2")
+        results.append([t.cpu().numpy() for t in backward()])
     a, b = results
     assert np.abs(a[0] - b[0]).max() <= 4e-6 * np.abs(b[0]).max()
     for p, q in zip(a[1:], b[1:]):
         assert np.array_equal(p, q)
 
 
-def launches(hip, kernel, call):
-    """How often `kernel` is launched by `call`."""
-    hip.profile_arm(kernel)
-    call()
-    return hip.profile_collect()[1]
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("planes,F,h,w", SNAPSHOT_SHAPES)
+def test_grad_input_from_snapshots_half(hip, switches, planes, F, h, w, dtype):
+    """The same with a 16-bit grad_output against its float32 copy through the column workspace:
+    grad_input is rounded once more, parameter gradients see the same float32 values."""
+    rng = np.random.default_rng(planes + F + h + w)
+    integ = hip.integral_image(dev(rng.standard_normal((1, planes, h, w)).astype(np.float32)))
+    g = dev((rng.standard_normal((1, planes * F, h, w)) + 0.25).astype(np.float32)).to(dtype)
+    boxes = [dev(b) for b in make_boxes(rng, planes, F, h, w, "hanging", away_from_integers=0.05)]
+
+    def backward(grad):
+        return hip.box_convolution_backward(integ, *boxes, grad, None, 3.5 * h, 2.25 * w, True, True,
+                                            True, True, True, True, True)
+    switches("BOXCONV_GI_SNAPSHOTS", "2")
+    assert launches(hip, "grad_input_taps", lambda: backward(g)) == 1
+    a = backward(g)
+    switches("BOXCONV_GI_SNAPSHOTS", "0")
+    b = backward(g.float())
+    assert a[0].dtype == dtype
+    # half a unit in the last place of the 16-bit type, and of denormals of float16, beside the float32
+    # difference of the test above
+    unit, least = {torch.float16: (2.0 ** -11, 2.0 ** -25), torch.bfloat16: (2.0 ** -8, 0.0)}[dtype]
+    assert ((a[0].float() - b[0]).abs() <= unit * b[0].abs() + 4.1e-6 * b[0].abs().max() + least).all()
+    for p, q in zip(a[1:], b[1:]):
+        assert torch.equal(p, q)
 
 
 @pytest.mark.parametrize("snapshots,planes,F,h,w", [
