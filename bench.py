@@ -79,6 +79,18 @@ def load_measured_traffic(kernel, workload_name):
     return None
 
 
+def load_measured_step_traffic(workload_name):
+    """HBM bytes of one step, every kernel's recorded bytes per launch added up (same file as
+    load_measured_traffic; each kernel runs once per step); None if there is none."""
+    path = os.path.join(ROOT, "profiles", "hbm_traffic_%s.txt" % workload_name)
+    try:
+        with open(path) as fh:
+            rows = [line.split() for line in fh if line.strip() and not line.startswith("#")]
+        return sum(int(parts[3]) for parts in rows if "calibration" not in parts[0])
+    except (OSError, ValueError, IndexError):
+        return None
+
+
 def cpu_baseline(k, ab_full):
     """The reference's CPU kernels (oracle/_ref, built from the reference's own sources) or, where
     that library does not exist, the C++ restatement, timed on this host: whole steps of the same
@@ -474,6 +486,8 @@ def main():
     avg_launch_s = dom_ms / 1e3 / max(dom_launches, 1)
     achieved = bytes_per_launch / avg_launch_s / 1e9
 
+    whole_step = not (args.forward_only or args.shape)
+    step_traffic = load_measured_step_traffic(wl.name) if whole_step else None
     result = {
         "metric": METRIC if not args.forward_only else
                   "BoxConv2d inference forward ms/iter + effective HBM GB/s (% peak) at 2x16ch 512x1024 fp32",
@@ -502,7 +516,12 @@ def main():
             "mode": ("inference forward, eval mode, %s box bounds" % ("rounded" if args.rounded else "exact")
                      if args.forward_only else
                      "captured HIP graph of the step's native calls" if args.graph else "eager module step"),
+            # the data flow of the integral-image algorithm, the backward's intermediate written and read
+            # among it, whichever way the backward takes; beside it what the recorded counters say
+            # really crossed the memory interface
             "algorithmic_bytes_per_step": ab["alg"],
+            "recorded_hbm_bytes_per_step": step_traffic,
+            "recorded_hbm_GBps": round(step_traffic / (elapsed / args.steps) / 1e9, 2) if step_traffic else None,
             "io_bytes_per_step": ab["io"],
             "frac_of_hbm_peak": round(value / HBM_PEAK_GBS, 4),
             "io_GBps": round(ab["io"] / (elapsed / args.steps) / 1e9, 2),
