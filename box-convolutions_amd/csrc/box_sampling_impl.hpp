@@ -1524,9 +1524,9 @@ inline bool consecutive_rows(int w) {
 }
 
 // The launches of grad_output_stream_consec_kernel (`lanes` busy lanes of a workgroup of `cnt`;
-// SCAN = false: parameter sums only). Its instantiations are translation units of their own
-// (BOXCONV_INST_PART 3 and 4): some hundred kernels that would otherwise double the compile time
-// of the unit with the other variant.
+// MODE: a StreamMode). Its instantiations are translation units of their own (BOXCONV_INST_PART 3 to
+// 5): some hundred kernels that would otherwise double the compile time of the unit with the other
+// variant.
 template <class TG, int MODE>
 hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lanes, int cnt, bool exact,
                                             dim3 grid, hipStream_t stream);

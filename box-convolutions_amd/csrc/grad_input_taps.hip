@@ -24,12 +24,14 @@
 // the sum of each band.
 //
 // It replaces the column workspace, which is written whole and read twice (grad_input_cols_kernel),
-// by a second read of grad_output and snapshots of 1/8 or 1/16 of that size. Both backward kernels
-// together, 16 x 8 planes: 512 x 1024 x 2 346 -> 271 us, 720 x 1280 372 -> 318 us; 32 x 4 planes of
-// 128 x 256 x 4 46 -> 44 us (x 8 in bfloat16 82 -> 71); 128 x 2 planes of 1024 x 2048 1607 -> 1458 us.
-// Bound (512 x 1024, 132 us): the vector ALU issues 45 % of the time and the LDS pipe is busy for a
-// quarter at two waves per SIMD; 2.2 reads of grad_output at the L2, the second of which misses it
-// where the planes in flight outgrow 4 MB.
+// by a second read of grad_output and snapshots of 1/4 or 1/8 of that size (two rows per group of 8 or 16
+// output rows) and one row per band. Both backward kernels together, 16 x 8 planes: 512 x 1024 x 2 346 ->
+// 266 us, 720 x 1280 357 -> 304 us; 32 x 4 planes of 128 x 256 x 4 44 -> 41 us (x 8 in bfloat16 79 -> 57); 128 x 2
+// planes of 1024 x 2048 1632 -> 1520 us. Not every launch gains: snapshots_pay (box_sampling.hip).
+// Bound (512 x 1024, 131 us): latency and issue at 6.6 resident waves per CU; the vector ALU issues a third
+// of the time, the LDS pipe is busy for 15 % of it with no bank conflicts; 578 MB are fetched for 537 MB of
+// grad_output and 54 of snapshots, so its second read hits the L2 for the most part (at 1024 x 2048, with
+// planes of 8 MB, 2.5 GB for 2.1).
 // Groups of 16 rows where that leaves two waves per SIMD, else of 8: against 8 rows, 16 take 132 against
 // 137 us at 512 x 1024, 159 against 191 at 720 x 1280, 687 against 774 at 1024 x 2048 (half the
 // snapshots), but 25 against 19 us at 128 planes of 128 x 256, where they leave half of the SIMDs idle.

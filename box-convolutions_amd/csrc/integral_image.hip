@@ -13,9 +13,11 @@
 //                            input row, then a row-direction prefix of the accumulators.
 // With a single band (tall enough grid without cutting) only launch 3 runs. Rows of at most 4096
 // columns use band_scan_rows_kernel for launch 3, which adds up the bands above itself (no launch
-// 2). For float rows of 256 to 2048 columns and planes of at most 32 bands of 32 rows, one
-// kernel does everything in a single pass over the input (band_scan_lookback_kernel): workgroups
-// hand their column sums to the ones below them, with a bounded wait. Planes of at most 192 rows
+// 2). For float output rows of 256 to 2048 columns one kernel does everything in a single pass over
+// the input (band_scan_lookback_kernel): workgroups hand their column sums to the ones below them,
+// with a bounded wait; where all workgroups are resident (planes of at most 32 bands of 32 rows), and
+// for rows of a multiple of four columns also where there are several times as many (up to 64
+// bands; plan_integral has the rule). Planes of at most 192 rows
 // and 256 columns take plane_scan_kernel: the bands of a plane are the waves of one workgroup,
 // which hand their sums over through LDS.
 //

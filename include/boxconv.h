@@ -55,7 +55,7 @@ void boxconv_reload_env(void);
  * a pair of HIP events recorded on the stream it is launched on (so the time is that kernel's
  * alone, whatever else the entry point launches). Names: "band_colsum", "band_prefix",
  * "band_scan", "forward_rows", "forward_quads", "grad_output_stream", "grad_input_cols",
- * "param_grad_finalize", "fill_zero", "fill_marker", "clip", "forward_gather", "grad_input_gather",
+ * "grad_input_taps", "param_grad_finalize", "fill_zero", "fill_marker", "clip", "forward_gather", "grad_input_gather",
  * "int_row_prefix", "int_col_prefix", "probe_copy_bands", "probe_grad_input_pattern",
  * "grad_params_gather".
  * NULL or "" disarms. Arming discards earlier measurements.
@@ -256,8 +256,9 @@ int boxconv_forward_fused_f32(const float* input_integrated, const float* x_min,
  * workspace: boxconv_backward_workspace_bytes(...) bytes, 256-byte aligned. It receives the
  * backward's one intermediate per (plane, filter) - h+1 rows of grad_output filtered along the
  * row and summed down the rows of a band (the bulk; for rows wider than 4096 columns, 2048 in
- * float64, a true integral image of grad_output instead; for most rows of a multiple of four columns
- * only column sums at every 8th or 16th row, in the same place) - and the per-box accumulators. */
+ * float64, a true integral image of grad_output instead; for most large launches with rows of a
+ * multiple of four columns only column sums at every 8th or 16th row, in the same place) - and the
+ * per-box accumulators. */
 size_t boxconv_backward_workspace_bytes(int batch, int in_planes, int num_filters, int h, int w,
                                         int elem_size, int input_needs_grad,
                                         int params_need_grad);
