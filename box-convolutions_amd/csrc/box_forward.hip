@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
 
     if (tid < 2 * K * kQuadPad)
         vrow[tid / (K * kQuadPad)][tid / kQuadPad % K][tid % kQuadPad] = RowPair<T>{T(0), T(0)};
-    const TapRun er = tap_run<PLANE>(tid, s.yhi - 1, quads), el = tap_run<PLANE>(tid, s.ylo - 2, quads);
+    const TapRun er = tap_run<PLANE>(c0, s.yhi - 1, quads), el = tap_run<PLANE>(c0, s.ylo - 2, quads);
     const int last = (quads - 1) & 63;               // lane of the last wave that owns column w
 
     const int i0 = band * a.R;

@@ -29,10 +29,14 @@ Switches read_switches() {
     s.lookback = e == nullptr || std::atoi(e) != 0;
     s.lookback_any_shape = e != nullptr && std::atoi(e) == 2;
     s.plane_integral = flag_unless_zero("BOXCONV_INTEGRAL_PLANE");
+    e = text("BOXCONV_INTEGRAL_PLANE");
+    s.plane_integral_tall = e == nullptr || (e[0] != '0' && e[0] != '1');
     s.stream_consecutive = flag_unless_zero("BOXCONV_STREAM_CONSEC");
     {
         const char* e = text("BOXCONV_STREAM_CONSEC");
         s.stream_consecutive_partial = e == nullptr || (e[0] != '0' && e[0] != '1');
+        s.odd_rows_any_size = e != nullptr && e[0] == '3';
+        s.stream_ragged = e == nullptr || s.odd_rows_any_size;
     }
     s.stream_narrow_double = flag_unless_zero("BOXCONV_STREAM_F64_NARROW");
     s.interleave_workspace = flag_unless_zero("BOXCONV_M_INTERLEAVE");
@@ -145,6 +149,13 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
 //    filters is small (15 of 552 x 1124 with one filter 46 against 63, 479 of 69 x 100 with two 37
 //    against 46, 99 of 186 x 96 with four 40 against 50): one round, or four over all filters.
 // By this rule 2.5 % of the shapes are more than 3 % slower than by the workspace; without it 44 % were.
+// Rows that are no multiple of four columns were timed on 2300 shapes against the workspace of
+// grad_output_stream_kernel (0.70 to 0.85 of its time from 2^24 output pixels on, 0.88 to 1.0 below); in addition
+//  * fewer than 40 rows (487 x 4 planes of 33 x 151 47 against 56 us, 90 x 8 of 34 x 506 46 against 54), or
+//    up to 192 columns and fewer than 2^24 output pixels (5 x 4 of 1055 x 171 45 against 51), are up to 1.2;
+//  * three waves and more whose last one has a single lane in use keep the workspace (16 x 8 planes of
+//    512 x 514 128 us that way, 115 by snapshots, 162 before this kernel took such rows: what a launch of
+//    that size returns is fixed bit for bit).
 bool snapshots_pay(int64_t planes, int F, int h, int w) {
     if (!switches().input_from_snapshots || F < 1 || !consecutive_rows(w)) return false;
     if (switches().snapshots_any_shape) return true;
@@ -153,6 +164,7 @@ bool snapshots_pay(int64_t planes, int F, int h, int w) {
     // resident: three waves per SIMD, ten workgroups of one wave by their LDS. Of two workgroups of five or
     // six waves on a CU the second slows the first by as much as it brings: they count as two rounds
     const int waves = consecutive_threads(w) / 64;
+    if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) || (waves > 2 && (w + 3) / 4 % 64 == 1))) return false;
     const int64_t workgroups = planes * ((h + 7) / 8), resident = 256 * (waves == 1 ? 10 : 12 / waves);
     return workgroups <= (waves > 4 ? 256 : resident) || workgroups * F >= 4 * resident;
 }

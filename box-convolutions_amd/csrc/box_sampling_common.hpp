@@ -207,13 +207,13 @@ __device__ __forceinline__ void load4_dword_aligned(const float* p, float (&v)[4
 // kQuadPad elements of zeros in front of every plane and behind it stand for the columns outside.
 constexpr int kQuadPad = 2;
 __host__ __device__ constexpr int quad_plane(int nt) { return nt + 64; }   // a multiple of 64 elements: two planes per access
-// Byte offsets of the taps at columns 4 * tid + first + m, m < 4 (m = 4: one element after m = 0).
+// Byte offsets of the taps at columns c0 + first + m, m < 4 (m = 4: one element after m = 0).
 struct TapRun {
     unsigned at[4];
 };
 template <int PLANE>
-__device__ __forceinline__ TapRun tap_run(int tid, int first, int quads) {
-    const int plane = first & 3, place = clampi(tid + (first >> 2), -kQuadPad, quads) + kQuadPad;
+__device__ __forceinline__ TapRun tap_run(int c0, int first, int quads) {
+    const int plane = (c0 + first) & 3, place = clampi((c0 + first) >> 2, -kQuadPad, quads) + kQuadPad;
     TapRun t;
 #pragma unroll
     for (int m = 0; m < 4; ++m)
@@ -226,8 +226,95 @@ __device__ __forceinline__ void read_taps(const RowPair<float>* row, const TapRu
     v[4] = at_bytes(row, t.at[0])[1];
 }
 
+// The four consecutive columns of lane `tid` in a row of w <= 4 * NT columns. The lanes behind the row's
+// end are idle (they load the row's first columns and drop what they loaded). FIT: kRowQuads, a multiple
+// of four columns (a kernel of its own for rows that fill the workgroup has the same loop and is no
+// faster: both backward kernels, 16 x 8 planes of 720 x 1280, 308 against 312 us); kRowAny: the last lane takes the row's last four columns, and
+// its first `twice` columns are its neighbour's too, which owns them. So no lane reads or writes past
+// the row, and no value has to be shifted between lanes.
+enum RowFit { kRowQuads, kRowAny };
+template <int NT, int FIT>
+struct RowLane {
+    int c0, cl;          // first column; the same or, for an idle lane, 0
+    int quads, twice;    // lanes in use; columns of this lane that the lane in front of it owns
+    bool in;
+    __device__ __forceinline__ RowLane(int tid, int w)
+        : c0(FIT == kRowAny ? min(4 * tid, max(w - 4, 0)) : 4 * tid), quads((w + 3) / 4), in(4 * tid < w) {
+        cl = in ? c0 : 0;
+        twice = FIT == kRowAny && in ? 4 * tid - c0 : 0;
+    }
+    __device__ __forceinline__ bool owns(int k) const { return in && !shares(k); }
+    // (known to be false at compile time for most k and fits)
+    __device__ __forceinline__ bool shares(int k) const { return FIT == kRowAny && k < 3 && k < twice; }
+    // What lies behind the row in the LDS layout above, in ROWS rows one after the other: the rest of
+    // the last quad and the idle lanes' places, which no lane writes later on.
+    template <int PLANE, int ROWS>
+    __device__ __forceinline__ void clear_behind(RowPair<float>* row, int w) const {
+        const int c = 4 * static_cast<int>(threadIdx.x);
+        for (int k = 0; k < 4; ++k)
+            if (c + k >= w)
+                for (int r = 0; r < ROWS; ++r)
+                    row[(4 * r + k) * PLANE + kQuadPad + threadIdx.x] = RowPair<float>{0.0f, 0.0f};
+    }
+};
+// The taps of the lane's columns (an idle lane's: the zeros in front of the row).
+template <int PLANE, int NT, int FIT>
+__device__ __forceinline__ TapRun lane_taps(const RowLane<NT, FIT>& ln, int first) {
+    TapRun t = tap_run<PLANE>(ln.c0, first, ln.quads);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) t.at[m] = ln.in ? t.at[m] : 0u;
+    return t;
+}
+
+// Where the lane's own columns lie in that layout. Idle lanes write what they loaded to places that
+// nobody reads, behind the zeros that follow the longest row: clearing it first, or a branch around
+// the stores, costs all lanes of a wave more.
+template <int PLANE, int FIT>
+struct QuadPlace {
+    unsigned first[FIT == kRowAny ? 4 : 1];
+    template <int NT>
+    __device__ __forceinline__ explicit QuadPlace(const RowLane<NT, FIT>& ln) {
+        const int unread = NT + 2 * kQuadPad + min(static_cast<int>(threadIdx.x) - ln.quads, PLANE - NT - 2 * kQuadPad - 1);
+#pragma unroll
+        for (int k = 0; k < (FIT == kRowAny ? 4 : 1); ++k) {
+            const int c = ln.c0 + k, own = (c & 3) * PLANE + (c >> 2) + kQuadPad;
+            first[k] = static_cast<unsigned>(ln.in ? own : k * PLANE + unread) *
+                       static_cast<unsigned>(sizeof(RowPair<float>));
+        }
+    }
+    template <class P>
+    __device__ __forceinline__ P* at(P* row, int k) const {
+        return FIT == kRowAny ? at_bytes(row, first[FIT == kRowAny ? k : 0]) : at_bytes(row + k * PLANE, first[0]);
+    }
+};
+
+// A quad as one access of 16 or 8 bytes at an address that is aligned to them, or (!ALIGNED) to its
+// elements only, which global memory allows.
+typedef unsigned w4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned w2_half_aligned __attribute__((ext_vector_type(2), aligned(2)));
+template <bool ALIGNED, class TG>
+__device__ __forceinline__ void load_row_quad(const TG* p, float (&v)[4]) {
+    if constexpr (ALIGNED) {
+        load_quad(p, v);
+    } else {
+        Quad<TG> q;
+        if constexpr (sizeof(TG) == 4)
+            q = __builtin_bit_cast(Quad<TG>, __builtin_nontemporal_load(reinterpret_cast<const w4_dword_aligned*>(p)));
+        else
+            q = __builtin_bit_cast(Quad<TG>, __builtin_nontemporal_load(reinterpret_cast<const w2_half_aligned*>(p)));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = widen(q.v[k]);
+    }
+}
+template <bool ALIGNED, class TG>
+__device__ __forceinline__ void store_row_quad(TG* p, const Quad<TG>& q) {
+    if constexpr (ALIGNED) *reinterpret_cast<Quad<TG>*>(p) = q;
+    else if constexpr (sizeof(TG) == 4) *reinterpret_cast<w4_dword_aligned*>(p) = __builtin_bit_cast(w4_dword_aligned, q);
+    else *reinterpret_cast<w2_half_aligned*>(p) = __builtin_bit_cast(w2_half_aligned, q);
+}
+
 // The smallest workgroup (whole waves) whose lanes, four columns each, cover a row.
-inline int consecutive_threads(int w) { return (w / 4 + 63) / 64 * 64; }
+inline int consecutive_threads(int w) { return ((w + 3) / 4 + 63) / 64 * 64; }
 
 template <class T>
 struct BoxOfWorkgroup {

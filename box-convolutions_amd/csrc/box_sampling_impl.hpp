@@ -895,8 +895,7 @@ grad_output_stream_kernel(SampleArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same pass for float rows of a multiple of four columns (w <= 4 * NT; FULL: w == 4 * NT), both
-// products at once: a lane owns 4 CONSECUTIVE columns for everything, where
+// The same pass for float rows (w <= 4 * NT), both products at once: a lane owns 4 CONSECUTIVE columns for everything, where
 // grad_output_stream_kernel gives it the columns lane, lane + 64, ... of its wave and moves the
 // weights W through LDS to get consecutive ones for the suffix sum. With consecutive columns
 //   * the taps of a lane's 4 columns are two runs of 5 adjacent row pairs in LDS (3 instructions
@@ -909,9 +908,8 @@ grad_output_stream_kernel(SampleArgs<T> a) {
 // Same arithmetic, same order of additions inside a lane's row pair; the sums differ from the
 // other kernel's only in which columns share a lane. Everything said there about the math, the
 // two splits, the single barrier per row pair (MERGED) and the cache policy of the stores applies.
-// !FULL: the lanes past the row's end (whole lanes, since w is a multiple of four) load from the
-// row's first columns and drop what they loaded where it would be used: they put zeros into LDS
-// (the row's right-hand padding), hold zero weights and a zero V, and store nothing.
+// FIT: see RowLane. Idle lanes take their taps from the zeros in front of the row, so their weights are
+// zero; the columns that the last lane shares with its neighbour have their weights and V cleared.
 
 // What the kernel leaves for the gradient w.r.t. the input.
 enum StreamMode {
@@ -932,7 +930,7 @@ enum StreamMode {
 // column workspace competes for the L2). kStreamSnapshots: the same plus one addition per element;
 // told to fit four waves, since left alone the compiler takes one to five registers too many for
 // them (three waves per SIMD: 168 against 140 us at 512 x 1024).
-template <class TG, int NT, bool EXACT, bool FULL, int MODE>
+template <class TG, int NT, bool EXACT, int FIT, int MODE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MODE == kStreamSnapshots ? 4 : 2, MODE != kStreamScan ? 4 : (NT == 192 || NT == 320 || NT == 384) ? 3 : 2)))
 grad_output_stream_consec_kernel(SampleArgs<float> a) {
     using T = float;
@@ -961,10 +959,10 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     const int h = a.h, w = a.w, tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c0 = K * tid;                          // the lane's first pixel column
-    const bool lane_in = FULL || c0 < w;             // (w is a multiple of K: a lane is in or out as a whole)
-    const int cl = lane_in ? c0 : 0;                 // idle lanes load the row's first columns
-    const int owner = FULL ? NT - 1 : w / K - 1;     // the lane whose last column is column w
+    const RowLane<NT, FIT> ln(tid, w);
+    const int c0 = ln.c0, cl = ln.cl;
+    const bool lane_in = ln.in;
+    const int owner = ln.quads - 1;                  // the lane whose last column is column w
 
     const BoxOfWorkgroup<T> bx = load_box(a.prm, k_par);
     BoxSplit<T> s = split_grad_params(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
@@ -977,6 +975,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
 
     const int64_t pitch = w + 1;
     const int64_t mpitch = a.mpitch;
+    const int spitch = FIT == kRowAny ? (w + 3) / 4 * 4 : w;                    // of the snapshots: the same
     const T* iplane = a.src + p * static_cast<int64_t>(h + 1) * pitch;        // integral of the input
     const TG* gplane = reinterpret_cast<const TG*>(a.grad_out) + pf * static_cast<int64_t>(h) * w;
     T* mrows = a.dst + pf * static_cast<int64_t>(h + 1) * mpitch;
@@ -996,7 +995,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
         load4_dword_aligned(iplane + static_cast<int64_t>(r) * pitch + 1 + cl, dst);
     };
     auto load_g = [&](int i, T (&dst)[K]) {
-        load_quad(gplane + static_cast<int64_t>(min(i, h - 1)) * w + cl, dst);
+        load_row_quad<FIT != kRowAny>(gplane + static_cast<int64_t>(min(i, h - 1)) * w + cl, dst);
     };
     auto load_window = [&](int i, T (&t0)[K], T (&t1)[K], T (&b1)[K], T (&b2)[K]) {
         load_i(clampi(i + s.xlo, 0, h), t0);
@@ -1014,22 +1013,23 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
         const int plane = tid / (2 * kQuadPad), e = tid % (2 * kQuadPad);
         grow[plane / K][plane % K][e < kQuadPad ? e : NT + e] = RowPair<T>{T(0), T(0)};
     }
+    ln.template clear_behind<PLANE, 2>(grow[0][0], w);
     if (SCAN && band == 0)
         for (int c = tid; c < mpitch; c += NT) mrows[c] = T(0);
     if (SNAP && vid == 0)                            // the row of zeros in front of the snapshots
-        for (int c = tid; c < w; c += NT) a.dst[c] = T(0);
-    T* const snap = a.dst + w + pf * static_cast<int64_t>(snapshot_rows(a)) * w;
+        for (int c = tid; c < spitch; c += NT) a.dst[c] = T(0);
+    T* const snap = a.dst + spitch + pf * static_cast<int64_t>(snapshot_rows(a)) * spitch;
     const int snap_lo = __builtin_amdgcn_readfirstlane(sm.xlo), snap_hi = __builtin_amdgcn_readfirstlane(sm.xhi);
     // the sum of the band's rows above integral row r, where grad_input_taps_kernel will want it
     auto keep_snapshot = [&](int r, const T (&sum)[K]) {
         const Quad<T> q{{sum[0], sum[1], sum[2], sum[3]}};
         const int mask = (1 << a.snap_shift) - 1, ut = r - snap_lo, ub = r - snap_hi;
         if ((ut & mask) == 0 && ut >= 0 && (ut >> a.snap_shift) < a.snap_groups)
-            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(ut >> a.snap_shift) * w), 4u * cl) = q;
+            store_row_quad<FIT != kRowAny>(at_bytes(snap + static_cast<int64_t>(ut >> a.snap_shift) * spitch, 4u * cl), q);
         if ((ub & mask) == 0 && ub >= 0 && (ub >> a.snap_shift) < a.snap_groups)
-            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(a.snap_groups + (ub >> a.snap_shift)) * w), 4u * cl) = q;
+            store_row_quad<FIT != kRowAny>(at_bytes(snap + static_cast<int64_t>(a.snap_groups + (ub >> a.snap_shift)) * spitch, 4u * cl), q);
         if (r == i1)
-            *at_bytes(reinterpret_cast<Quad<T>*>(snap + static_cast<int64_t>(2 * a.snap_groups + band) * w), 4u * cl) = q;
+            store_row_quad<FIT != kRowAny>(at_bytes(snap + static_cast<int64_t>(2 * a.snap_groups + band) * spitch, 4u * cl), q);
     };
 
     auto tail_weight = [&](int j, int ylo, int yhi, T fylo, T fyhi) {
@@ -1040,17 +1040,17 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
              - (EXACT ? fylo : T(0)) * T(j > w - ylo + 1);
     };
     // taps of the lane's columns: right run g[c0 - yhi ..], left run g[c0 + 1 - ylo ..]
-    const int quads = FULL ? NT : w / K;
-    const TapRun er = tap_run<PLANE>(tid, -s.yhi, quads), el = tap_run<PLANE>(tid, 1 - s.ylo, quads);
+    const TapRun er = lane_taps<PLANE>(ln, -s.yhi), el = lane_taps<PLANE>(ln, 1 - s.ylo);
+    const QuadPlace<PLANE, FIT> place(ln);
     bool wave_has_tail = false;
     {
         T d[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            d[k] = lane_in ? tail_weight(c0 + k, s.ylo, s.yhi, s.fylo, s.fyhi) : T(0);
+            d[k] = ln.owns(k) ? tail_weight(c0 + k, s.ylo, s.yhi, s.fylo, s.fyhi) : T(0);
             wave_has_tail = wave_has_tail || d[k] != T(0);
         }
-        *reinterpret_cast<Quad<T>*>(&delta[c0]) = Quad<T>{{d[0], d[1], d[2], d[3]}};
+        *reinterpret_cast<Quad<T>*>(&delta[K * tid]) = Quad<T>{{d[0], d[1], d[2], d[3]}};
     }
     wave_has_tail = __any(wave_has_tail) != 0 || own_w;                          // wave-uniform
     const int j_ymax = w - s.yhi, j_ymin = w - s.ylo + 1;
@@ -1078,15 +1078,11 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             _Pragma("unroll")                                                                       \
             for (int k = 0; k < K; ++k) GB[k] = T(0);                                               \
         }                                                                                           \
-        if (!FULL && !lane_in) {                                                                    \
-            _Pragma("unroll")                                                                       \
-            for (int k = 0; k < K; ++k) { GA[k] = T(0); GB[k] = T(0); }                             \
-        }                                                                                           \
         _Pragma("unroll")                                                                           \
-        for (int k = 0; k < K; ++k) grow[FL][k][kQuadPad + tid] = RowPair<T>{GA[k], GB[k]};         \
+        for (int k = 0; k < K; ++k) *place.at(grow[FL][0], k) = RowPair<T>{GA[k], GB[k]};           \
         TL0 = T(0); TL1 = T(0);                                                                     \
         if (wave_has_tail) {                                                                        \
-            const Quad<T> dq = *reinterpret_cast<const Quad<T>*>(&delta[c0]);                       \
+            const Quad<T> dq = *reinterpret_cast<const Quad<T>*>(&delta[K * tid]);                  \
             _Pragma("unroll")                                                                       \
             for (int k = 0; k < K; ++k) { TL0 += dq.v[k] * GA[k]; TL1 += dq.v[k] * GB[k]; }         \
         }                                                                                           \
@@ -1160,7 +1156,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
                     wq0[k] += s.fyhi * dr0; wq0[k] += s.fylo * dl0;
                     wq1[k] += s.fyhi * dr1; wq1[k] += s.fylo * dl1;
                 }
-                if (!FULL && !lane_in) { wq0[k] = T(0); wq1[k] = T(0); }    // (no column q > w)
+                if (ln.shares(k)) { wq0[k] = T(0); wq1[k] = T(0); }
                 const T dt0 = t0[k] - ta[k], db0 = b1[k] - bc[k];
                 const T dt1 = t1[k] - t0[k], db1 = b2[k] - b1[k];
                 T v0 = bc[k] - t0[k], v1 = b1[k] - t1[k];
@@ -1168,9 +1164,9 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
                     v0 += s.fxhi * db0; v0 += s.fxlo * dt0;
                     v1 += s.fxhi * db1; v1 += s.fxlo * dt1;
                 }
-                // (an idle lane: its weights are zero, which takes care of the products with dt and
-                // db; its V must go as well, since the taps of its columns are not zero)
-                if (!FULL && !lane_in) { v0 = T(0); v1 = T(0); }
+                // (a column that the neighbour owns: its weights are zero, which takes care of the
+                // products with dt and db; its V must go as well, since its taps are not zero)
+                if (ln.shares(k)) { v0 = T(0); v1 = T(0); }
                 sum[4] += v0 * wq0[k];
                 sum[1] += db0 * wq0[k];
                 sum[0] -= dt0 * wq0[k];
@@ -1201,8 +1197,8 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             // rare: the mirrored split cuts the box at other whole pixels; weights and tails of
             // the column workspace from that split
             RowPair<T> R[K + 1], L[K + 1];
-            read_taps(G, tap_run<PLANE>(tid, -yhi_m, quads), R);
-            read_taps(G, tap_run<PLANE>(tid, 1 - ylo_m, quads), L);
+            read_taps(G, lane_taps<PLANE>(ln, -yhi_m), R);
+            read_taps(G, lane_taps<PLANE>(ln, 1 - ylo_m), L);
             tail0 = T(0); tail1 = T(0);
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -1213,9 +1209,9 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
                     wq0[k] += sm.fylo * (grA.r0 - gr.r0); wq0[k] += sm.fyhi * (gl.r0 - glA.r0);
                     wq1[k] += sm.fylo * (grA.r1 - gr.r1); wq1[k] += sm.fyhi * (gl.r1 - glA.r1);
                 }
-                if (!FULL && !lane_in) { wq0[k] = T(0); wq1[k] = T(0); }
-                const T dlt = lane_in ? tail_weight(c0 + k, ylo_m, yhi_m, sm.fyhi, sm.fylo) : T(0);
-                const RowPair<T> own = G[k * PLANE + kQuadPad + tid];
+                if (ln.shares(k)) { wq0[k] = T(0); wq1[k] = T(0); }
+                const T dlt = ln.owns(k) ? tail_weight(c0 + k, ylo_m, yhi_m, sm.fyhi, sm.fylo) : T(0);
+                const RowPair<T> own = *place.at(G, k);
                 tail0 += dlt * own.r0;
                 tail1 += dlt * own.r1;
             }
@@ -1270,7 +1266,14 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             const int limit = static_cast<int>(mpitch * sizeof(T));
             // (the rows are addressed by offset into one descriptor for the plane: a lane past the
             // row's end must not store at all)
-            if (FULL || lane_in) {
+            if (FIT == kRowAny && ln.twice > 0) {             // its first columns are its neighbour's
+#pragma unroll
+                for (int k = 1; k < K; ++k)
+                    if (k >= ln.twice) {
+                        buffer_store<kCacheDefault>(out0[k], ob0, first + 4 * k);
+                        buffer_store<kCacheDefault>(colacc[k], ob1, first + 4 * k);
+                    }
+            } else if (lane_in) {
                 if (keep_in_cache) {
                     buffer_store_run<kCacheDefault, true>(out0, ob0, first, limit);
                     buffer_store_run<kCacheDefault, true>(colacc, ob1, first, limit);
@@ -1506,16 +1509,18 @@ hipError_t grad_input_launch(const T* gint, int band_rows, BoxParams<T> prm, TO*
 // policy (the memory-side cache holds 256 MB; the grad-input kernel reads that part first).
 inline int64_t cached_tail_bytes() { return switches().keep_tail_bytes; }
 
-// Rows that grad_output_stream_consec_kernel takes: a multiple of four columns, 16-byte (16-bit
-// elements: 8-byte) aligned. The workgroup is the smallest one (whole waves) whose lanes, four
-// columns each, cover the row. Only a single wave can be left mostly idle (from two waves on, more
-// than half of the lanes are busy): rows that fill less than three eighths of it stay with the
-// other kernel (measured, 16 x 4 planes of 256 rows: 100 columns 97 -> 86 us, 128: 91 -> 91, 144:
+// Rows that grad_output_stream_consec_kernel takes: up to 2048 columns; where they are a multiple of
+// four, 16-byte (16-bit elements: 8-byte) aligned. The workgroup is the smallest one (whole waves)
+// whose lanes, four columns each, cover the row. Only a single wave can be left mostly idle (from two
+// waves on, more than half of the lanes are busy): rows that fill less than three eighths of it stay
+// with the other kernel (measured, 16 x 4 planes of 256 rows: 100 columns 97 -> 86 us, 128: 91 -> 91, 144:
 // 110 -> 90, 260: 138 -> 118, 300: 142 -> 121; but 64 columns 72 -> 83). Rows of exactly 128 columns
 // also stay there: they fill that kernel's two waves at one column per lane with no bounds to check
-// (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us).
+// (10 to 38 x 64 planes of 64 to 256 rows: 70 against 80 us). Rows that are no multiple of four start
+// behind those: 97 to 127 columns have the shorter chain there, and take 1.0 to 1.4 of its time.
 inline bool consecutive_rows(int w) {
-    if (w % 4 != 0 || w > 2048) return false;
+    if (w > 2048) return false;
+    if (w % 4 != 0) return w > 128 && switches().stream_ragged;
     const RowConfig rc = stream_row_config(w, sizeof(float));
     const int lanes = w / 4, cnt = consecutive_threads(w);
     const bool exact_fit = lanes == cnt && (cnt == 64 || cnt == 128 || cnt == 256 || cnt == 512);
@@ -1523,26 +1528,35 @@ inline bool consecutive_rows(int w) {
            (exact_fit || (switches().stream_consecutive_partial && lanes * 8 >= cnt * 3 && !(rc.full && rc.K == 1)));
 }
 
-// The launches of grad_output_stream_consec_kernel (`lanes` busy lanes of a workgroup of `cnt`;
-// MODE: a StreamMode). Its instantiations are translation units of their own (BOXCONV_INST_PART 3 to
+// Without snapshots (those are asked for where they pay: snapshots_pay), rows that are no multiple of four
+// columns, whose last lane costs every wave a few selects, gain less. Timed on 6700 shapes, time over that of
+// grad_output_stream_kernel, both backward kernels with the column workspace / the parameter sums alone:
+//  * 129 to 192 columns 1.03 to 1.06 / 0.85 to 0.99; from 193 on 0.79 to 1.01 / 0.75 to 1.0;
+//  * but 1281 to 1536 columns, three columns per lane there, 1.0 to 1.03 / 1.1 to 1.16 below 2^24 output pixels
+//    and 0.87 above, as 1025 to 2048 columns are 1.02 to 1.11 and 0.8.
+inline bool odd_rows_pay(int w, int64_t pixels, bool workspace) {
+    if (switches().odd_rows_any_size) return true;
+    if (workspace) return w > 192 && (w <= 1280 || w > 1536);
+    return w <= 1024 || pixels >= (1ll << 24);
+}
+
+// The launches of grad_output_stream_consec_kernel (workgroups of `cnt`; MODE: a StreamMode). Its instantiations are translation units of their own (BOXCONV_INST_PART 3 to
 // 5): some hundred kernels that would otherwise double the compile time of the unit with the other
 // variant.
 template <class TG, int MODE>
-hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lanes, int cnt, bool exact,
+hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int cnt, bool exact,
                                             dim3 grid, hipStream_t stream);
 #if defined(BOXCONV_INST_PART) && BOXCONV_INST_PART >= 3 && BOXCONV_INST_PART <= 5
 template <class TG, int MODE>
-hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lanes, int cnt, bool exact,
+hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int cnt, bool exact,
                                             dim3 grid, hipStream_t stream) {
     const size_t lds = 0;                              // the kernel's LDS is statically sized
+#define LAUNCH_GC_FIT(NT, FIT) \
+    if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, FIT, MODE>), grid, dim3(NT), lds, stream, a); \
+    else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, FIT, MODE>), grid, dim3(NT), lds, stream, a)
 #define LAUNCH_GC(NT) \
-    if (lanes == NT) { \
-        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, true, MODE>), grid, dim3(NT), lds, stream, a); \
-        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, true, MODE>), grid, dim3(NT), lds, stream, a); \
-    } else { \
-        if (exact) BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, true, false, MODE>), grid, dim3(NT), lds, stream, a); \
-        else       BOXCONV_LAUNCH("grad_output_stream", (grad_output_stream_consec_kernel<TG, NT, false, false, MODE>), grid, dim3(NT), lds, stream, a); \
-    }
+    if (a.w % 4 == 0) { LAUNCH_GC_FIT(NT, kRowQuads); } \
+    else              { LAUNCH_GC_FIT(NT, kRowAny); }
     switch (cnt) {
         case 64: LAUNCH_GC(64) break;
         case 128: LAUNCH_GC(128) break;
@@ -1554,6 +1568,7 @@ hipError_t grad_output_stream_consec_launch(const SampleArgs<float>& a, int lane
         default: LAUNCH_GC(512) break;
     }
 #undef LAUNCH_GC
+#undef LAUNCH_GC_FIT
     return hipGetLastError();
 }
 #endif
@@ -1624,18 +1639,18 @@ hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxPara
             return hipGetLastError();
         }
     }
-    // float rows of a multiple of four columns, the parameter sums wanted (with or without the column
-    // workspace), a slot per workgroup for the sums: the kernel with four consecutive columns per lane
+    // float rows, the parameter sums wanted (with or without the column workspace), a slot per workgroup
+    // for the sums: the kernel with four consecutive columns per lane
     if constexpr (std::is_same<T, float>::value) {
-        const int lanes = d.w / 4;
         const int cnt = consecutive_threads(d.w);
-        if (params && acc_slots > 0 && consecutive_rows(d.w) && quads_aligned(grad_out, sizeof(TG))) {
+        if (params && acc_slots > 0 && consecutive_rows(d.w) && quads_aligned(grad_out, sizeof(TG), d.w) &&
+            (d.w % 4 == 0 || snapshots != nullptr || odd_rows_pay(d.w, planes_f * d.hw(), scan))) {
             if (snapshots != nullptr) {
                 a.snap_shift = snapshots->shift; a.snap_groups = snapshots->groups; a.snap_bands = sp.nb;
-                return grad_output_stream_consec_launch<TG, kStreamSnapshots>(a, lanes, cnt, exact, grid, stream);
+                return grad_output_stream_consec_launch<TG, kStreamSnapshots>(a, cnt, exact, grid, stream);
             }
-            if (scan) return grad_output_stream_consec_launch<TG, kStreamScan>(a, lanes, cnt, exact, grid, stream);
-            return grad_output_stream_consec_launch<TG, kStreamParams>(a, lanes, cnt, exact, grid, stream);
+            if (scan) return grad_output_stream_consec_launch<TG, kStreamScan>(a, cnt, exact, grid, stream);
+            return grad_output_stream_consec_launch<TG, kStreamParams>(a, cnt, exact, grid, stream);
         }
     }
     if (snapshots != nullptr) return hipErrorInvalidValue;   // (plan_snapshots asks for that kernel only)

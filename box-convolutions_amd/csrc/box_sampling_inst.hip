@@ -16,13 +16,13 @@ template hipError_t grad_output_stream_launch<BOXCONV_INST_T, BOXCONV_INST_TG>(
     const BOXCONV_INST_T*, const BOXCONV_INST_TG*, BoxParams<BOXCONV_INST_T>, double*, int, BOXCONV_INST_T*,
     const StreamPlan&, const SnapshotPlan*, Dims, bool, hipStream_t);
 #elif BOXCONV_INST_PART == 3
-template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamScan>(const SampleArgs<float>&, int, int, bool,
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamScan>(const SampleArgs<float>&, int, bool,
                                                                             dim3, hipStream_t);
 #elif BOXCONV_INST_PART == 4
-template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamParams>(const SampleArgs<float>&, int, int, bool,
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamParams>(const SampleArgs<float>&, int, bool,
                                                                              dim3, hipStream_t);
 #elif BOXCONV_INST_PART == 5
-template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamSnapshots>(const SampleArgs<float>&, int, int,
+template hipError_t grad_output_stream_consec_launch<BOXCONV_INST_TG, kStreamSnapshots>(const SampleArgs<float>&, int,
                                                                                        bool, dim3, hipStream_t);
 #else
 template hipError_t grad_input_launch<BOXCONV_INST_T, BOXCONV_INST_TG>(

@@ -382,7 +382,7 @@ int backward_impl(const T* integ, const T* x_min, const T* x_max, const T* y_min
 
     const int64_t planes = static_cast<int64_t>(batch) * in_planes;
     const boxconv::Dims d{in_planes, num_filters, h, w, planes, 0};
-    const bool sums_only = need_params && boxconv::quads_aligned(grad_output, kSameType ? sizeof(T) : 2) &&
+    const bool sums_only = need_params && boxconv::quads_aligned(grad_output, kSameType ? sizeof(T) : 2, w) &&
                            (!need_input || boxconv::snapshots_pay(planes, num_filters, h, w));
     const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(std::max<int64_t>(planes, 1) * num_filters, h, w,
                                                                     sizeof(T), sums_only);

@@ -133,9 +133,11 @@ struct StreamPlan {
 // sums_only: the parameter sums are wanted and no column workspace (at most snapshots): the bands,
 // i.e. the slots per (plane, filter), depend on it, and are then at least as many as otherwise.
 StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool sums_only);
-// Whether a grad_output is aligned for the kernels whose lanes read 4 consecutive columns.
-inline bool quads_aligned(const void* grad_out, size_t elem_size) {
-    return reinterpret_cast<uintptr_t>(grad_out) % (4 * elem_size) == 0;
+// Whether a tensor with rows of w elements is aligned for the kernels whose lanes read 4 consecutive columns:
+// where rows are a multiple of that many columns they have to start on addresses that are, else on
+// whole elements.
+inline bool quads_aligned(const void* tensor, size_t elem_size, int w) {
+    return reinterpret_cast<uintptr_t>(tensor) % (w % 4 == 0 ? 4 * elem_size : elem_size) == 0;
 }
 
 // Where the gradient w.r.t. the input is formed from grad_output itself (grad_input_taps_launch):
@@ -222,8 +224,11 @@ struct Switches {
     bool lookback;            // BOXCONV_INTEGRAL_LOOKBACK=0 clears it: no single-pass integral image
     bool lookback_any_shape;  // BOXCONV_INTEGRAL_LOOKBACK=2: single pass for every shape it covers
     bool plane_integral;      // BOXCONV_INTEGRAL_PLANE=0 clears it: no plane-per-workgroup integral image
+    bool plane_integral_tall; // BOXCONV_INTEGRAL_PLANE=1 clears it: that image only for planes of at most 192 rows
     bool stream_consecutive;  // BOXCONV_STREAM_CONSEC=0 clears it: no consecutive-column variant of the grad_output pass at all
     bool stream_consecutive_partial;  // BOXCONV_STREAM_CONSEC=1 clears it: that variant only for rows that fill its workgroup exactly
+    bool stream_ragged;       // BOXCONV_STREAM_CONSEC=2 clears it: that variant only for rows of a multiple of four columns
+    bool odd_rows_any_size;   // BOXCONV_STREAM_CONSEC=3: that variant for all other rows, too, in launches of any size
     bool stream_narrow_double;  // BOXCONV_STREAM_F64_NARROW=0 clears it: float64 rows with three or four columns per lane and one launch like float32
     bool interleave_workspace;  // BOXCONV_M_INTERLEAVE=0 clears it: rows of the column workspace in their natural order
     bool input_from_snapshots;  // BOXCONV_GI_SNAPSHOTS=0 clears it: grad_input from the column workspace only

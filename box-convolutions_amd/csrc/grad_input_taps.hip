@@ -50,29 +50,36 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // it is written; no instruction.
 __device__ __forceinline__ void finish_here(float& v) { asm volatile("" : "+v"(v)); }
 
-template <class TG>
+template <class TG, bool ALIGNED>
 struct GradQuad;
-template <>
-struct GradQuad<float> {
+template <bool ALIGNED>
+struct GradQuad<float, ALIGNED> {
     typedef float f4 __attribute__((ext_vector_type(4)));
     f4 q;
-    __device__ __forceinline__ void load(const float* p) { q = *reinterpret_cast<const f4*>(p); }
+    __device__ __forceinline__ void load(const float* p) {
+        if constexpr (ALIGNED) q = *reinterpret_cast<const f4*>(p);
+        else q = *reinterpret_cast<const f4_dword_aligned*>(p);
+    }
     __device__ __forceinline__ float get(int v) const { return q[v]; }
 };
-template <class H>
+template <class H, bool ALIGNED>
 struct GradQuadHalf {
     typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u2_at_any_half __attribute__((ext_vector_type(2), aligned(2)));
     u2 q;
-    __device__ __forceinline__ void load(const H* p) { q = *reinterpret_cast<const u2*>(p); }
+    __device__ __forceinline__ void load(const H* p) {
+        if constexpr (ALIGNED) q = *reinterpret_cast<const u2*>(p);
+        else q = *reinterpret_cast<const u2_at_any_half*>(p);
+    }
     __device__ __forceinline__ float get(int v) const {
         const unsigned word = v < 2 ? q.x : q.y;
         return widen(H{static_cast<unsigned short>((v & 1) ? word >> 16 : word & 0xffffu)});
     }
 };
-template <> struct GradQuad<f16_t> : GradQuadHalf<f16_t> {};
-template <> struct GradQuad<bf16_t> : GradQuadHalf<bf16_t> {};
+template <bool ALIGNED> struct GradQuad<f16_t, ALIGNED> : GradQuadHalf<f16_t, ALIGNED> {};
+template <bool ALIGNED> struct GradQuad<bf16_t, ALIGNED> : GradQuadHalf<bf16_t, ALIGNED> {};
 
-template <class TG, int NT, int RB, bool EXACT, bool FULL>
+template <class TG, int NT, int RB, bool EXACT, int FIT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, RB == 8 ? 3 : 2)))
 grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
     constexpr int K = 4, PLANE = quad_plane(NT), WAVES = NT / 64;
@@ -95,17 +102,17 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
     const int h = a.h, w = a.w, tid = threadIdx.x, lane = tid & 63;
     const int wave = uniform(tid >> 6);
     const int i0 = group * RB;
-    const int c0 = K * tid;
-    const bool lane_in = FULL || c0 < w;             // (w is a multiple of K: a lane is in or out as a whole)
-    const int cl = lane_in ? c0 : 0;                 // idle lanes load the row's first columns and drop them
+    const RowLane<NT, FIT> ln(tid, w);
+    const int c0 = ln.c0, cl = ln.cl;
+    const bool lane_in = ln.in;
+    const int64_t spitch = a.mpitch;                 // of the snapshots
 
     for (int e = tid; e < 2 * PAIRS * K * 2 * kQuadPad; e += NT) {
         const int plane = e / (2 * kQuadPad), n = e % (2 * kQuadPad);
         (&rows[0][0][0][0])[plane * PLANE + (n < kQuadPad ? n : NT + n)] = RowPair<float>{0.0f, 0.0f};
     }
-    if (!FULL && !lane_in)                           // idle lanes never write a row: their columns stay zero
-        for (int plane = 0; plane < 2 * PAIRS * K; ++plane)
-            (&rows[0][0][0][0])[plane * PLANE + kQuadPad + tid] = RowPair<float>{0.0f, 0.0f};
+    ln.template clear_behind<PLANE, 2 * PAIRS>(&rows[0][0][0][0], w);
+    const QuadPlace<PLANE, FIT> place(ln);
 
     const float* zeros = a.src;
     const int srows = snapshot_rows(a);
@@ -119,8 +126,8 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
     bool wave_any_tail = false;
 
     // what is in flight for the coming filter
-    GradQuad<TG> top[RC], bot[RC];
-    GradQuad<float> snap_t, snap_b, between[2];
+    GradQuad<TG, FIT != kRowAny> top[RC], bot[RC];
+    GradQuad<float, FIT != kRowAny> snap_t, snap_b, between[2];
     auto split_of = [&](int f, float& scale) {
         const BoxOfWorkgroup<float> bx = load_box(a.prm, c_in * a.F + f);
         BoxSplit<float> s = split_grad_input(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
@@ -138,20 +145,20 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
             return reinterpret_cast<const TG*>(static_cast<unsigned>(i) < static_cast<unsigned>(h) ? at : none);
         };
         if (chunk == 0) {
-            const float* snaps = a.src + w + (p * a.F + f) * static_cast<int64_t>(srows) * w;
+            const float* snaps = a.src + spitch + (p * a.F + f) * static_cast<int64_t>(srows) * spitch;
             auto snapshot = [&](int edge, int first) {
                 const int r = i0 + edge;
-                const uintptr_t at = reinterpret_cast<uintptr_t>(snaps + static_cast<int64_t>(r >= h ? srows - 1 : first + group) * w);
+                const uintptr_t at = reinterpret_cast<uintptr_t>(snaps + static_cast<int64_t>(r >= h ? srows - 1 : first + group) * spitch);
                 const uintptr_t none = reinterpret_cast<uintptr_t>(zeros);
                 return reinterpret_cast<const float*>(r <= 0 ? none : at);
             };
             snap_t.load(snapshot(s.xlo, 0) + cl);
             snap_b.load(snapshot(s.xhi, a.snap_groups) + cl);
             const int bt = band_of(s.xlo), bb = band_of(s.xhi), lo = min(bt, bb), hi = max(bt, bb);
-            const float* first = snaps + static_cast<int64_t>(2 * a.snap_groups + lo) * w;
+            const float* first = snaps + static_cast<int64_t>(2 * a.snap_groups + lo) * spitch;
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
-                const uintptr_t at = reinterpret_cast<uintptr_t>(first + n * w), none = reinterpret_cast<uintptr_t>(zeros);
+                const uintptr_t at = reinterpret_cast<uintptr_t>(first + n * spitch), none = reinterpret_cast<uintptr_t>(zeros);
                 between[n].load(reinterpret_cast<const float*>(lo + n < hi ? at : none) + cl);
             }
         }
@@ -173,7 +180,7 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
         float core[K];
         {
             const int bt = band_of(s.xlo), bb = band_of(s.xhi), lo = min(bt, bb), hi = max(bt, bb);
-            const float* bands = a.src + w + ((p * a.F + f) * static_cast<int64_t>(srows) + 2 * a.snap_groups) * w + cl;
+            const float* bands = a.src + spitch + ((p * a.F + f) * static_cast<int64_t>(srows) + 2 * a.snap_groups) * spitch + cl;
             double sum[K];
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -182,8 +189,8 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
                 for (int n = 0; n < 2; ++n) sum[k] += static_cast<double>(between[n].get(k));
             }
             for (int b = lo + 2; b < hi; ++b) {
-                GradQuad<float> q;
-                q.load(bands + static_cast<int64_t>(b) * w);
+                GradQuad<float, FIT != kRowAny> q;
+                q.load(bands + static_cast<int64_t>(b) * spitch);
 #pragma unroll
                 for (int k = 0; k < K; ++k) sum[k] += static_cast<double>(q.get(k));
             }
@@ -204,13 +211,12 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
                 t += q == s.yhi - 1 ? s.fyhi : 0.0f;
                 t += q == s.ylo - 2 ? s.fylo : 0.0f;
             }
-            tw[k] = lane_in ? t * scale : 0.0f;
+            tw[k] = ln.owns(k) ? t * scale : 0.0f;
             has_tail = has_tail || tw[k] != 0.0f;
         }
         has_tail = __any(has_tail) != 0;             // wave-uniform
         wave_any_tail = wave_any_tail || has_tail;
-        const int quads = FULL ? NT : w / K;
-        const TapRun er = tap_run<PLANE>(tid, s.yhi - 1, quads), el = tap_run<PLANE>(tid, s.ylo - 2, quads);
+        const TapRun er = lane_taps<PLANE>(ln, s.yhi - 1), el = lane_taps<PLANE>(ln, s.ylo - 2);
         const float fxhi = s.fxhi, fxlo = s.fxlo;
 #pragma unroll
         for (int stage = 0; stage < STAGES; ++stage) {
@@ -239,7 +245,7 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
                         finish_here(tail[r]);
                     }
 #pragma unroll
-                    for (int k = 0; k < K; ++k) rows[buf][q][k][kQuadPad + tid] = RowPair<float>{v[0][k], v[1][k]};
+                    for (int k = 0; k < K; ++k) *place.at(rows[buf][q][0], k) = RowPair<float>{v[0][k], v[1][k]};
                 }
             }
             __builtin_amdgcn_sched_barrier(0);       // (loads moved up past the stores above would spill)
@@ -280,6 +286,9 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
 #pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (ln.shares(k)) E[r][k] = 0.0f;        // (the neighbour's columns count once)
+#pragma unroll
         for (int k = 1; k < K; ++k) E[r][k] += E[r][k - 1];
         const float inc = wave_inclusive_scan(E[r][K - 1]);
         left[r] = inc - E[r][K - 1];
@@ -306,11 +315,12 @@ grad_input_taps_kernel(SampleArgs<float> a, FinalizeArgs<float> fin) {
 #pragma unroll
         for (int k = 0; k < K; ++k) narrow(base + E[r][k], q.v[k]);
         TG* orow = out + static_cast<int64_t>(i) * w;
-        if (a.vec_out) {
-            *reinterpret_cast<Quad<TG>*>(orow) = q;
+        if (a.vec_out && (FIT != kRowAny || ln.twice == 0)) {
+            store_row_quad<FIT != kRowAny>(orow, q);
         } else {
 #pragma unroll
-            for (int k = 0; k < K; ++k) orow[k] = q.v[k];
+            for (int k = 0; k < K; ++k)
+                if (ln.owns(k)) orow[k] = q.v[k];
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -327,7 +337,7 @@ SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d) {
     plan.groups = (d.h + (1 << plan.shift) - 1) >> plan.shift;
     // (the last condition: the snapshots fit where the column workspace would be)
     plan.use = snapshots_pay(d.planes, d.F, d.h, d.w) && sp.usable && sp.parts == 1 &&
-               quads_aligned(grad_out, sizeof(TG)) && 2 * plan.groups + sp.nb + 1 <= d.h + 1;
+               quads_aligned(grad_out, sizeof(TG), d.w) && 2 * plan.groups + sp.nb + 1 <= d.h + 1;
     return plan;
 }
 
@@ -344,7 +354,8 @@ hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, co
     a.normalize = normalize ? 1 : 0;
     a.off_R = sp.R;
     a.reverse = switches().gi_reverse ? 1 : 0;
-    a.vec_out = reinterpret_cast<uintptr_t>(grad_in) % (4 * sizeof(TG)) == 0 ? 1 : 0;
+    a.vec_out = quads_aligned(grad_in, sizeof(TG), d.w) ? 1 : 0;
+    a.mpitch = column_workspace_pitch(d.w);
     a.snap_shift = plan.shift; a.snap_groups = plan.groups; a.snap_bands = sp.nb;
     finish_args(a, d.planes * plan.groups);
     const dim3 grid(static_cast<unsigned>(a.per_xcd * kXcds));
@@ -353,15 +364,12 @@ hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, co
         fin = finalize_args(*finish);
         if (finish_done != nullptr) *finish_done = true;
     }
-    const int lanes = d.w / 4;
+#define LAUNCH_GT_FIT(NT, RB, FIT)                                                                                    \
+    if (exact) BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, true, FIT>), grid, dim3(NT), 0, stream, a, fin);   \
+    else       BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, false, FIT>), grid, dim3(NT), 0, stream, a, fin)
 #define LAUNCH_GT_RB(NT, RB)                                                                                          \
-    if (lanes == NT) {                                                                                              \
-        if (exact) BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, true, true>), grid, dim3(NT), 0, stream, a, fin);   \
-        else       BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, false, true>), grid, dim3(NT), 0, stream, a, fin);  \
-    } else {                                                                                                        \
-        if (exact) BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, true, false>), grid, dim3(NT), 0, stream, a, fin);  \
-        else       BOXCONV_LAUNCH("grad_input_taps", (grad_input_taps_kernel<TG, NT, RB, false, false>), grid, dim3(NT), 0, stream, a, fin); \
-    }
+    if (d.w % 4 == 0) { LAUNCH_GT_FIT(NT, RB, kRowQuads); }                                                            \
+    else              { LAUNCH_GT_FIT(NT, RB, kRowAny); }
 #define LAUNCH_GT(NT)                                                                                               \
     case NT:                                                                                                        \
         if (plan.shift == 4) { LAUNCH_GT_RB(NT, 16) } else { LAUNCH_GT_RB(NT, 8) }                                   \
@@ -379,6 +387,7 @@ hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, co
     }
 #undef LAUNCH_GT
 #undef LAUNCH_GT_RB
+#undef LAUNCH_GT_FIT
     return hipGetLastError();
 }
 

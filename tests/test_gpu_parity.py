@@ -630,6 +630,68 @@ def test_grad_input_from_snapshots_half(hip, switches, planes, F, h, w, dtype):
         assert torch.equal(p, q)
 
 
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("h,w", [
+    # remainders of one, two and three columns: the smallest rows, rows of just under, on and over a
+    # whole number of waves, lanes behind the row's end in the same wave or a wave of their own
+    (33, 129), (26, 130), (31, 191), (40, 255), (24, 257), (37, 258), (24, 301), (29, 510), (25, 513),
+    (70, 767), (24, 1021), (27, 1023), (24, 1281), (26, 2045), (25, 2047)])
+def test_grad_output_pass_of_odd_rows(hip, oracle, switches, h, w, exact):
+    """Rows that are not a multiple of four columns in the grad_output pass with consecutive columns
+    per lane, whose last lane takes the row's last four columns and shares some with its neighbour:
+    with snapshots, with the column workspace and with the parameter sums alone, against the oracle
+    (BOXCONV_STREAM_CONSEC=3: in launches of any size), and against the kernel with wave-strided
+    columns (=2). The boxes hang over both ends of the rows."""
+    rng = np.random.default_rng(h * w + int(exact))
+    B, C, F = 1, 2, 3
+    x = rng.standard_normal((B, C, h, w)).astype(np.float32)
+    g = (rng.standard_normal((B, C * F, h, w)) + 0.25).astype(np.float32)
+    boxes = list(make_boxes(rng, C, F, h, w, "hanging", away_from_integers=0.05))
+    if not exact:
+        boxes[1] = np.maximum(boxes[1], np.ceil(boxes[0]) + 1).astype(np.float32)
+        boxes[3] = np.maximum(boxes[3], np.ceil(boxes[2]) + 1).astype(np.float32)
+    results = []
+    for snapshots, consecutive in (("2", "3"), ("0", "3"), ("0", "2")):
+        switches("BOXCONV_GI_SNAPSHOTS", snapshots)
+        switches("BOXCONV_STREAM_CONSEC", consecutive)
+        cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, True, exact, g)
+        assert_parity(cpu, gpu, np.float32, "snapshots=%s consecutive=%s %dx%d" % (snapshots, consecutive, h, w), **sc)
+        results.append(gpu[1])
+        alone = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, True, exact, g, (False, True, True, True, True))
+        if consecutive == "3":
+            for a, b in zip(alone[1][1][1:], results[0][1:]):
+                assert np.array_equal(a, b)
+    for r in results[:2]:
+        assert np.abs(r[0] - results[2][0]).max() <= 4e-6 * np.abs(results[2][0]).max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("h,w", [(24, 133), (33, 255), (25, 259), (40, 767), (24, 2046)])
+def test_grad_output_pass_of_odd_rows_half(hip, switches, h, w, dtype):
+    """The same with a 16-bit grad_output that starts on an odd element, and so on any 2-byte address in
+    every row, against its float32 copy: parameter gradients see the same float32 values in the same
+    order, grad_input is rounded once more."""
+    rng = np.random.default_rng(h + w)
+    planes, F = 3, 4
+    integ = hip.integral_image(dev(rng.standard_normal((1, planes, h, w)).astype(np.float32)))
+    flat = dev((rng.standard_normal(planes * F * h * w + 1) + 0.25).astype(np.float32)).to(dtype)
+    g = flat[1:].view(1, planes * F, h, w)
+    boxes = [dev(b) for b in make_boxes(rng, planes, F, h, w, "hanging", away_from_integers=0.05)]
+
+    def backward(grad):
+        return hip.box_convolution_backward(integ, *boxes, grad, None, 3.5 * h, 2.25 * w, True, True,
+                                            True, True, True, True, True)
+    switches("BOXCONV_GI_SNAPSHOTS", "2")
+    assert launches(hip, "grad_input_taps", lambda: backward(g)) == 1
+    a, b = backward(g), backward(g.float())
+    # half a unit in the last place of the 16-bit type, and of denormals of float16: the float32 sums
+    # are the same ones
+    unit, least = {torch.float16: (2.0 ** -11, 2.0 ** -25), torch.bfloat16: (2.0 ** -8, 0.0)}[dtype]
+    assert ((a[0].float() - b[0]).abs() <= unit * b[0].abs() + least).all()
+    for p, q in zip(a[1:], b[1:]):
+        assert torch.equal(p, q)
+
+
 @pytest.mark.parametrize("snapshots,planes,F,h,w", [
     (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
     # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
