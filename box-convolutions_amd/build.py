@@ -23,6 +23,8 @@ LIB_PATH = os.path.join(HERE, "box_convolution", "libboxconv_hip.so")
 # the backward kernels and is compiled once per element-type pair and part, so that they build in
 # parallel (one translation unit with all of them takes six minutes).
 def _inst(tag, t, tg, part, same):
+    if part == 7:
+        return ("narrow_rows.hip", "narrow_rows_%s.o" % tag, ["-DBOXCONV_INST_TG=" + tg])
     if part == 6:                                    # grad_input_taps.hip: a source of its own
         return ("grad_input_taps.hip", "grad_input_taps_%s.o" % tag, ["-DBOXCONV_INST_TG=" + tg])
     defs = ["-DBOXCONV_INST_T=" + t, "-DBOXCONV_INST_TG=" + tg, "-DBOXCONV_INST_PART=%d" % part]
@@ -36,7 +38,7 @@ SOURCES = [(s, s.replace(".hip", ".o"), []) for s in
             "boxconv_c_abi.hip")]
 for _tag, _t, _tg in (("f32", "float", "float"), ("f64", "double", "double"),
                       ("f16", "float", "f16_t"), ("bf16", "float", "bf16_t")):
-    for _part in (1, 2) + ((3, 4, 5, 6) if _t == "float" else ()):
+    for _part in (1, 2) + ((3, 4, 5, 6, 7) if _t == "float" else ()):
         SOURCES.append(_inst(_tag, _t, _tg, _part, _t == _tg))
 HEADERS = ["boxconv_device.hpp", "boxconv_host.hpp", "box_sampling_common.hpp", "box_sampling_impl.hpp",
            os.path.join("..", "..", "include", "boxconv.h")]

@@ -2,6 +2,7 @@
 // kernels themselves are templates in box_sampling_impl.hpp, instantiated by box_sampling_inst.hip.
 
 #include <atomic>
+#include <cmath>
 #include <mutex>
 
 #include "box_sampling_impl.hpp"   // stream_lds_bytes; the templates in it are not instantiated here
@@ -28,6 +29,9 @@ Switches read_switches() {
     e = text("BOXCONV_INTEGRAL_LOOKBACK");
     s.lookback = e == nullptr || std::atoi(e) != 0;
     s.lookback_any_shape = e != nullptr && std::atoi(e) == 2;
+    e = text("BOXCONV_NARROW");
+    s.narrow_rows = e == nullptr || e[0] != '0';
+    s.narrow_any_size = e != nullptr && std::atoi(e) == 2;
     s.plane_integral = flag_unless_zero("BOXCONV_INTEGRAL_PLANE");
     e = text("BOXCONV_INTEGRAL_PLANE");
     s.plane_integral_tall = e == nullptr || (e[0] != '0' && e[0] != '1');
@@ -112,7 +116,8 @@ hipError_t grad_params_begin(double* acc, int n_boxes, hipStream_t stream) {
     return hipGetLastError();
 }
 
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool sums_only) {
+StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t elem_size, bool sums_only) {
+    const int64_t planes_f = planes * F;
     StreamPlan sp{};
     const RowConfig rc = stream_row_config(std::max(w, 1), elem_size);
     sp.usable = row_kernels_apply(h, w, elem_size) &&
@@ -133,8 +138,30 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
     sp.R = std::max(R, 2);
     sp.nb = (h + sp.R - 1) / sp.R;
     sp.parts = (rc.nt == 1024 || stream_double_wide_split(w, elem_size)) ? 2 : 1;
+    if (sp.usable && sums_only && elem_size == 4 && narrow_rows_pay(planes, F, h, w)) {
+        // Several bands side by side in a wave: rows per band (a power of two of at least a group, so that groups
+        // of rows start with bands) for the least rounds of waves times row pairs of a band and what it takes to
+        // start and end one, about three pairs. A launch is short of waves or, with bands that end
+        // in the middle of a wave, wastes them: 671 x 37 planes of 72 x 107, the sums, bands of 16, 32 and 64
+        // rows 247, 298 and 295 us; 512 x 4 of 64 x 128 22, 19 and 29. No more bands than a box's column
+        // sums are quickly added up from (78 x 19 of 928 x 32, both kernels 156, 124 and 107).
+        const int lanes = w <= 32 ? 8 : w <= 64 ? 16 : 32, side = 64 / lanes;
+        double best = 0.0;
+        for (int R = 128; R >= 8; R /= 2) {
+            const int nb = (h + R - 1) / R, slots = (nb + side - 1) / side;
+            const double waves = static_cast<double>(planes_f) * slots, rounds = waves / (256 * 12);
+            const double cost = (rounds < 4 ? std::ceil(rounds) : rounds) * (std::min(R, h) / 2 + 3);
+            // (rows that the kernel with one row per wave takes, too: no more waves than that one may launch)
+            if (consecutive_rows(w) && planes_f * slots > std::max<int64_t>(2 * switches().stream_workgroups, planes_f)) break;
+            if (sp.lanes > 0 && (cost >= best || nb > 40)) continue;
+            best = cost;
+            sp.lanes = lanes; sp.R = R; sp.nb = nb;
+        }
+    }
     return sp;
 }
+
+namespace {
 
 // grad_input_taps_kernel walks through a plane's filters one after the other, 1.5 to 2.5 us each
 // however few the planes are, where grad_input_cols_kernel spreads filters and rows over more waves.
@@ -156,8 +183,8 @@ StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_s
 //  * three waves and more whose last one has a single lane in use keep the workspace (16 x 8 planes of
 //    512 x 514 128 us that way, 115 by snapshots, 162 before this kernel took such rows: what a launch of
 //    that size returns is fixed bit for bit).
-bool snapshots_pay(int64_t planes, int F, int h, int w) {
-    if (!switches().input_from_snapshots || F < 1 || !consecutive_rows(w)) return false;
+bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
+    if (!consecutive_rows(w)) return false;
     if (switches().snapshots_any_shape) return true;
     const int64_t pixels = planes * h * w;
     if (h < 24 || pixels < 180000 * static_cast<int64_t>(std::min(F, 8))) return false;
@@ -167,6 +194,43 @@ bool snapshots_pay(int64_t planes, int F, int h, int w) {
     if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) || (waves > 2 && (w + 3) / 4 % 64 == 1))) return false;
     const int64_t workgroups = planes * ((h + 7) / 8), resident = 256 * (waves == 1 ? 10 : 12 / waves);
     return workgroups <= (waves > 4 ? 256 : resident) || workgroups * F >= 4 * resident;
+}
+
+}  // namespace
+
+// Rows of at most 128 columns: the kernels that put several of them side by side in a wave (narrow_rows.hip)
+// against grad_output_stream_kernel and grad_input_cols_kernel, timed on 4300 shapes (1 to 2048 planes, 1 to
+// 40 filters, 16 to 1100 rows; float32 and bfloat16 with both gradients, float32 with the parameter sums alone):
+// 0.72, 0.75 and 0.69 of the time in the geometric mean by this rule, 0.59, 0.62 and 0.56 of the total, 33 of the
+// shapes more than 3 % slower (up to 1.15, one 1.40). Left to the others:
+//  * rows so few that bands of eight leave most of the wave empty (1629 x 2 planes of 12 x 20, the sums 12.5
+//    against 15.1 us; 1956 x 4 of 16 x 46 23.6 against 26.3);
+//  * fewer than 2^17 output pixels, where a step is bound by its launches, and few input pixels for the filters, which waves visit one after the other (25 planes of 24 x 16 with 40
+//    filters 22 against 32 us; 32 of 28 x 28 26 against 30);
+//  * tall planes that give too few waves: their bands are cut short, and a box spans many of them (15 x 4
+//    planes of 1086 x 23 30 against 37 us);
+//  * 96 to 124 columns in multiples of four where the wide kernels keep the column workspace: what such
+//    launches return is fixed bit for bit.
+bool narrow_rows_pay(int64_t planes, int F, int h, int w) {
+    const Switches& sw = switches();
+    if (!sw.narrow_rows || !sw.input_from_snapshots || F < 1 || w < 16 || w > 128 || h < 8 || h >= (1 << 22)) return false;
+    if (sw.narrow_any_size) return true;
+    if (sw.snapshots_any_shape) return false;
+    if (consecutive_rows(w)) return wide_snapshots_pay(planes, F, h, w);
+    const int64_t pixels = planes * h * w;
+    return h >= (w <= 32 ? 24 : w <= 64 ? 20 : 16) && pixels >= 1500 * static_cast<int64_t>(F) &&
+           pixels * F >= (h <= 400 ? 1 << 17 : 1 << 21);
+}
+
+int narrow_filter_sets(int64_t workgroups, int F) {
+    int sets = 1;
+    while (sets < 8 && 2 * sets <= F && workgroups * sets < 2048) sets *= 2;
+    return sets;
+}
+
+bool snapshots_pay(int64_t planes, int F, int h, int w) {
+    if (narrow_rows_pay(planes, F, h, w)) return true;
+    return switches().input_from_snapshots && F >= 1 && wide_snapshots_pay(planes, F, h, w);
 }
 
 }  // namespace boxconv

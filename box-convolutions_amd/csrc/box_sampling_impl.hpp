@@ -1586,7 +1586,10 @@ hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxPara
     a.src = integ; a.grad_out = reinterpret_cast<const T*>(grad_out); a.acc = acc; a.acc_slots = acc_slots;
     a.dst = column_workspace;
     a.mpitch = column_workspace_pitch(d.w);
-    if (acc_slots != 0 && acc_slots != sp.nb * sp.parts) return hipErrorInvalidValue;
+    if (acc_slots != 0 && acc_slots != sp.slots()) return hipErrorInvalidValue;
+    if constexpr (std::is_same<T, float>::value)
+        if (sp.lanes > 0)                              // (planned only where its loads are aligned)
+            return narrow_sums_launch<TG>(integ, grad_out, prm, acc, acc_slots, column_workspace, sp, snapshots, d, exact, stream);
     a.nb = sp.nb; a.R = sp.R;
     set_workspace_layout(a, d.h, sp.R);
     a.keep_tail = scan ? cached_tail_bytes() / kXcds : 0;

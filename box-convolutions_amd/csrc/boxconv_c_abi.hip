@@ -111,7 +111,9 @@ BackwardLayout backward_layout(int batch, int in_planes, int num_filters, int h,
     BackwardLayout L{};
     const int64_t planes = std::max<int64_t>(static_cast<int64_t>(batch) * in_planes, 1);
     const bool sums_only = need_params && (!need_input || boxconv::snapshots_pay(planes, num_filters, h, w));
-    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes * num_filters, h, w, elem_size, sums_only);
+    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(planes, num_filters, h, w, elem_size, sums_only);
+    // (what a grad_output that is not aligned takes)
+    const boxconv::StreamPlan any = boxconv::plan_grad_output_stream(planes, num_filters, h, w, elem_size, false);
     L.streaming = sp.usable;
     size_t off = 0;
     L.gint_off = off;
@@ -127,7 +129,7 @@ BackwardLayout backward_layout(int batch, int in_planes, int num_filters, int h,
         off += align_up(static_cast<size_t>(aux) * 8, 256);
     }
     L.acc_off = off;
-    L.acc_slots = (need_params && L.streaming) ? sp.nb * sp.parts : 0;
+    L.acc_slots = (need_params && L.streaming) ? std::max(sp.slots(), any.slots()) : 0;
     if (need_params)
         off += align_up(static_cast<size_t>(in_planes) * num_filters * 5 * 8 *
                         (L.acc_slots > 0 ? static_cast<size_t>(batch) * L.acc_slots : 1), 256);
@@ -384,9 +386,9 @@ int backward_impl(const T* integ, const T* x_min, const T* x_max, const T* y_min
     const boxconv::Dims d{in_planes, num_filters, h, w, planes, 0};
     const bool sums_only = need_params && boxconv::quads_aligned(grad_output, kSameType ? sizeof(T) : 2, w) &&
                            (!need_input || boxconv::snapshots_pay(planes, num_filters, h, w));
-    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(std::max<int64_t>(planes, 1) * num_filters, h, w,
+    const boxconv::StreamPlan sp = boxconv::plan_grad_output_stream(std::max<int64_t>(planes, 1), num_filters, h, w,
                                                                     sizeof(T), sums_only);
-    const int acc_slots = L.acc_slots > 0 ? sp.nb * sp.parts : 0;
+    const int acc_slots = L.acc_slots > 0 ? sp.slots() : 0;
     const int grad_dtype = std::is_same<TG, T>::value ? 0 : std::is_same<TG, boxconv::f16_t>::value ? 1 : 2;
     const boxconv::ParamFinish<T> finish{acc, batch, acc_slots, {gx_min, gx_max, gy_min, gy_max},
                                          n_boxes, reparam_h, reparam_w, normalize != 0, exact != 0,

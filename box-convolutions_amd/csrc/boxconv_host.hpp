@@ -128,11 +128,14 @@ struct StreamPlan {
     bool usable;             // false: width or LDS need outside what the streaming kernel covers
     int nb, R;               // bands per plane, rows per band (R even)
     int parts;               // workgroups that share a band for the parameter sums (1, or 2 for rows
-                             // wider than 2048 columns): accumulation slots per (plane, filter) = nb * parts
+                             // wider than 2048 columns)
+    int lanes;               // > 0: narrow_sums_kernel, 64 / lanes bands per wave (sums only, float)
+    // accumulation slots per (plane, filter)
+    int slots() const { return lanes > 0 ? (nb * lanes + 63) / 64 : nb * parts; }
 };
 // sums_only: the parameter sums are wanted and no column workspace (at most snapshots): the bands,
 // i.e. the slots per (plane, filter), depend on it, and are then at least as many as otherwise.
-StreamPlan plan_grad_output_stream(int64_t planes_f, int h, int w, size_t elem_size, bool sums_only);
+StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t elem_size, bool sums_only);
 // Whether a tensor with rows of w elements is aligned for the kernels whose lanes read 4 consecutive columns:
 // where rows are a multiple of that many columns they have to start on addresses that are, else on
 // whole elements.
@@ -149,6 +152,9 @@ struct SnapshotPlan {
 };
 // Whether that is the faster way for float sums of an image of this size (both gradients wanted).
 bool snapshots_pay(int64_t planes, int F, int h, int w);
+// Whether rows of this width take the kernels of narrow_rows.hip (they are then among those of
+// snapshots_pay), also for the parameter sums alone.
+bool narrow_rows_pay(int64_t planes, int F, int h, int w);
 template <class TG>
 SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d);
 template <class TG>
@@ -157,7 +163,20 @@ hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, co
                                   bool normalize, bool exact, hipStream_t stream,
                                   const ParamFinish<float>* finish, bool* finish_done);
 
-// acc may be null: no parameter sums. With acc_slots == sp.nb it is [all planes*F][nb][5] doubles
+// The two passes for rows of at most 128 columns (narrow_rows.hip), where the plan says so (sp.lanes).
+// plan: null for the parameter sums alone.
+template <class TG>
+hipError_t narrow_sums_launch(const float* integ, const TG* grad_out, BoxParams<float> prm, double* acc, int slots,
+                              float* snapshots, const StreamPlan& sp, const SnapshotPlan* plan, Dims d, bool exact,
+                              hipStream_t stream);
+template <class TG>
+hipError_t narrow_input_launch(const TG* grad_out, const float* snapshots, const SnapshotPlan& plan, const StreamPlan& sp,
+                               BoxParams<float> prm, TG* grad_in, Dims d, bool normalize, bool exact, hipStream_t stream,
+                               const ParamFinish<float>* finish, bool* finish_done);
+// Sets of threads of narrow_input_kernel that share the filters of a launch of `workgroups`.
+int narrow_filter_sets(int64_t workgroups, int F);
+
+// acc may be null: no parameter sums. With acc_slots == sp.slots() it is [all planes*F][slots][5] doubles
 // and every workgroup stores its five partial sums in its own slot (nothing to clear, no atomics,
 // results reproducible bit for bit); with acc_slots == 0 it is [C*F*5] doubles, cleared by
 // grad_params_begin, and workgroups add atomically. grad_params_finish takes the same two values.
@@ -228,6 +247,8 @@ struct Switches {
     bool stream_consecutive;  // BOXCONV_STREAM_CONSEC=0 clears it: no consecutive-column variant of the grad_output pass at all
     bool stream_consecutive_partial;  // BOXCONV_STREAM_CONSEC=1 clears it: that variant only for rows that fill its workgroup exactly
     bool stream_ragged;       // BOXCONV_STREAM_CONSEC=2 clears it: that variant only for rows of a multiple of four columns
+    bool narrow_rows;         // BOXCONV_NARROW=0 clears it: rows of at most 128 columns as all others
+    bool narrow_any_size;     // BOXCONV_NARROW=2: narrow_sums_kernel for every launch of such rows that it covers
     bool odd_rows_any_size;   // BOXCONV_STREAM_CONSEC=3: that variant for all other rows, too, in launches of any size
     bool stream_narrow_double;  // BOXCONV_STREAM_F64_NARROW=0 clears it: float64 rows with three or four columns per lane and one launch like float32
     bool interleave_workspace;  // BOXCONV_M_INTERLEAVE=0 clears it: rows of the column workspace in their natural order

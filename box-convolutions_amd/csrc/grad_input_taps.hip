@@ -333,7 +333,7 @@ SnapshotPlan plan_snapshots(const TG* grad_out, const StreamPlan& sp, Dims d) {
     SnapshotPlan plan{};
     // 16 rows per group where that still makes two waves per SIMD (measured above)
     const int64_t waves16 = d.planes * ((d.h + 15) / 16) * (consecutive_threads(d.w) / 64);
-    plan.shift = waves16 >= 2048 ? 4 : 3;
+    plan.shift = waves16 >= 2048 && sp.lanes == 0 ? 4 : 3;
     plan.groups = (d.h + (1 << plan.shift) - 1) >> plan.shift;
     // (the last condition: the snapshots fit where the column workspace would be)
     plan.use = snapshots_pay(d.planes, d.F, d.h, d.w) && sp.usable && sp.parts == 1 &&
@@ -348,6 +348,8 @@ hipError_t grad_input_taps_launch(const TG* grad_out, const float* snapshots, co
                                   const ParamFinish<float>* finish, bool* finish_done) {
     if (finish_done != nullptr) *finish_done = false;
     if (d.planes == 0 || d.hw() == 0) return hipSuccess;
+    if (sp.lanes > 0)
+        return narrow_input_launch<TG>(grad_out, snapshots, plan, sp, prm, grad_in, d, normalize, exact, stream, finish, finish_done);
     SampleArgs<float> a = base_args(prm, d);
     a.src = snapshots; a.grad_out = reinterpret_cast<const float*>(grad_out);
     a.dst = reinterpret_cast<float*>(grad_in);

@@ -692,6 +692,65 @@ def test_grad_output_pass_of_odd_rows_half(hip, switches, h, w, dtype):
         assert torch.equal(p, q)
 
 
+NARROW_SHAPES = [
+    # 8, 16 and 32 lanes per row, full, with idle lanes, and with a last lane that shares columns; one band,
+    # bands past the plane, several waves per plane; filters shared by 1, 2, 4 and 8 waves, evenly or not
+    (8, 16, 1), (28, 28, 9), (17, 17, 3), (33, 32, 2), (9, 31, 16), (130, 23, 5), (64, 33, 4), (40, 48, 3),
+    (200, 63, 1), (31, 64, 8), (64, 65, 2), (70, 95, 3), (129, 100, 2), (64, 128, 4), (300, 127, 1)]
+
+
+@pytest.mark.parametrize("exact,normalize", [(True, True), (False, True), (True, False)])
+@pytest.mark.parametrize("h,w,F", NARROW_SHAPES)
+def test_narrow_rows_side_by_side(hip, oracle, switches, h, w, F, exact, normalize):
+    """Rows of at most 128 columns with several bands (or groups of output rows) side by side in a wave
+    (BOXCONV_NARROW=2: launches of any size), against the oracle and against the kernels for wider
+    rows; the parameter sums alone are those of the full pass, bit for bit. The boxes hang over every edge."""
+    rng = np.random.default_rng(h * w + F)
+    B, C = 2, 3
+    x = rng.standard_normal((B, C, h, w)).astype(np.float32)
+    g = (rng.standard_normal((B, C * F, h, w)) + 0.25).astype(np.float32)
+    boxes = list(make_boxes(rng, C, F, h, w, "hanging", away_from_integers=0.05))
+    if not exact:
+        boxes[1] = np.maximum(boxes[1], np.ceil(boxes[0]) + 1).astype(np.float32)
+        boxes[3] = np.maximum(boxes[3], np.ceil(boxes[2]) + 1).astype(np.float32)
+    results = []
+    for variant in ("2", "0"):
+        switches("BOXCONV_NARROW", variant)
+        switches("BOXCONV_GI_SNAPSHOTS", None if variant == "2" else "0")
+        cpu, gpu, sc = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, normalize, exact, g)
+        assert_parity(cpu, gpu, np.float32, "narrow=%s %dx%d" % (variant, h, w), **sc)
+        results.append(gpu[1])
+    assert np.abs(results[0][0] - results[1][0]).max() <= 4e-6 * np.abs(results[1][0]).max()
+    switches("BOXCONV_NARROW", "2")
+    switches("BOXCONV_GI_SNAPSHOTS", None)
+    _, alone, _ = run_both(hip, oracle, x, tuple(boxes), 3.5 * h, 2.25 * w, normalize, exact, g, (False, True, True, True, True))
+    for a, b in zip(alone[1][1:], results[0][1:]):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("h,w,F", [(28, 28, 9), (41, 45, 3), (64, 128, 4), (33, 127, 2), (20, 18, 1)])
+def test_narrow_rows_half(hip, switches, h, w, F, dtype):
+    """The same with a 16-bit grad_output, for odd rows one that starts on any 2-byte address, against its
+    float32 copy: the same float32 sums, grad_input rounded once more."""
+    rng = np.random.default_rng(h + w)
+    planes = 5
+    switches("BOXCONV_NARROW", "2")
+    integ = hip.integral_image(dev(rng.standard_normal((1, planes, h, w)).astype(np.float32)))
+    flat = dev((rng.standard_normal(planes * F * h * w + 1) + 0.25).astype(np.float32)).to(dtype)
+    g = flat[1:].view(1, planes * F, h, w) if w % 4 else flat[:-1].view(1, planes * F, h, w)
+    boxes = [dev(b) for b in make_boxes(rng, planes, F, h, w, "hanging", away_from_integers=0.05)]
+
+    def backward(grad):
+        return hip.box_convolution_backward(integ, *boxes, grad, None, 3.5 * h, 2.25 * w, True, True,
+                                            True, True, True, True, True)
+    a, b = backward(g), backward(g.float())
+    unit, least = {torch.float16: (2.0 ** -11, 2.0 ** -25), torch.bfloat16: (2.0 ** -8, 0.0)}[dtype]
+    assert ((a[0].float() - b[0]).abs() <= unit * b[0].abs() + least).all()
+    for p, q in zip(a[1:], b[1:]):
+        assert torch.equal(p, q)
+
+
 @pytest.mark.parametrize("snapshots,planes,F,h,w", [
     (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
     # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
