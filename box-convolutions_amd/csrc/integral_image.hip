@@ -18,8 +18,9 @@
 // with a bounded wait; where all workgroups are resident (planes of at most 32 bands of 32 rows), and
 // for rows of a multiple of four columns also where there are several times as many (up to 64
 // bands; plan_integral has the rule). Planes of at most 192 rows
-// and 256 columns take plane_scan_kernel: the bands of a plane are the waves of one workgroup,
-// which hand their sums over through LDS.
+// and 256 columns, and taller ones of which there are enough (plane_scan_pays), take plane_scan_kernel:
+// the bands of a plane are the waves of one workgroup, or parts of them, which hand their sums over
+// through LDS.
 //
 // Arithmetic. All sums are carried in double and rounded once on store, so every stored value
 // is the correctly rounded exact sum (the CPU reference carries row sums in double as well but
@@ -626,23 +627,66 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
 }
 
 // ---- single pass, a whole plane per workgroup ---------------------------------------------------
-// Planes of at most 256 columns and 192 rows: wave b of the workgroup owns band b of the plane at
-// full width (a row is one wave, four columns per lane), so the bands of a plane meet in one
-// workgroup and hand their column sums over through LDS with one barrier: one launch, the input
-// read once, nothing in global memory besides input and output, no waiting between workgroups.
-// The arithmetic is that of band_scan_lookback_kernel with one wave per row: the band's rows in
-// registers, double column sums added in band order, rows scanned out of the registers.
-constexpr int kPlaneWaves = 8;        // bands per plane at most
+// Planes of at most 256 columns: a workgroup owns a plane, its waves hold bands of rows at full width,
+// four columns per lane, so the bands of a plane meet in one workgroup and hand their column sums
+// over through LDS with one barrier: one launch, the input read once, nothing in global memory
+// besides input and output, no waiting between workgroups. The arithmetic is that of
+// band_scan_lookback_kernel with one wave per row: the band's rows in registers, double column sums
+// added in band order, rows scanned out of the registers.
+// A wave takes 64 / L bands side by side, L lanes each, every lane walking down its own band's rows
+// (rows of at most 128 / 64 columns would otherwise leave half / three quarters of every wave idle).
+// VEC: rows of a multiple of four columns from an aligned address. Otherwise the last lane takes the
+// row's last four columns (loads of four elements may start anywhere) and drops those that the lane
+// in front of it holds.
+// TALL: planes of more rows than the workgroup holds at a time. It goes down the plane in chunks of
+// that many rows; a row's registers take the next chunk's row as soon as they are scanned out.
+// Measured against the kernels before it (two launches for the tall planes; for the others one row per wave or
+// rows of a multiple of four columns only), float32: 578 planes of 833 x 23 334 -> 70 us, 224 of 296 x 80 57 -> 13,
+// 384 of 360 x 224 117 -> 60, 671 of 72 x 107 18 -> 14, 128 of 135 x 240 20 -> 12 (16-bit elements and rows that
+// do not exist are now widened and dropped after all loads are under way), but 128 of 135 x 241 11.8 -> 13.0.
+// Bound by the chain load, sums, scan of a chunk where planes are few, else by memory.
+constexpr int kPlaneWaves = 8;        // waves per workgroup at most
 constexpr int kPlaneRows = 24;        // rows per band at most (registers: 4 x 24 floats per lane without spilling)
+constexpr int kPlaneTallRows = 16;    // the same where the next chunk's rows are in flight, too
 constexpr int kPlaneMaxRows = kPlaneWaves * kPlaneRows, kPlaneMaxCols = 256;
 
-template <class TI, int RMAX, bool VEC>
+// Four elements as one load, kept as they are in memory.
+template <bool ALIGNED, class TI>
+__device__ __forceinline__ Vec4<TI> load_raw_quad(const TI* p) {
+    if constexpr (sizeof(TI) == 4) {
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+        if constexpr (ALIGNED) return __builtin_bit_cast(Vec4<TI>, __builtin_nontemporal_load(reinterpret_cast<const f4*>(p)));
+        else return __builtin_bit_cast(Vec4<TI>, __builtin_nontemporal_load(reinterpret_cast<const f4_any*>(p)));
+    } else {
+        typedef unsigned u2 __attribute__((ext_vector_type(2)));
+        typedef unsigned u2_any __attribute__((ext_vector_type(2), aligned(2)));
+        if constexpr (ALIGNED) return __builtin_bit_cast(Vec4<TI>, __builtin_nontemporal_load(reinterpret_cast<const u2*>(p)));
+        else return __builtin_bit_cast(Vec4<TI>, __builtin_nontemporal_load(reinterpret_cast<const u2_any*>(p)));
+    }
+}
+
+// Inclusive prefix sum within segments of L consecutive lanes: the first steps of
+// wave_inclusive_scan. All lanes must be active.
+template <int L>
+__device__ __forceinline__ double segment_inclusive_scan(double x) {
+    static_assert(L == 16 || L == 32 || L == 64, "segments of one, two or four DPP rows");
+    x += dpp_move<0x111, 0xf>(x, x);
+    x += dpp_move<0x112, 0xf>(x, x);
+    x += dpp_move<0x114, 0xf>(x, x);
+    x += dpp_move<0x118, 0xf>(x, x);
+    if (L >= 32) x += dpp_move<0x142, 0xa>(0.0, x);   // lane 15 of rows 0,2 into rows 1,3
+    if (L == 64) x += dpp_move<0x143, 0xc>(0.0, x);   // lane 31 into rows 2,3
+    return x;
+}
+
+template <class TI, int RMAX, int L, bool VEC, bool TALL>
 __global__ void __launch_bounds__(kPlaneWaves * 64)
 plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int w, int R, int64_t planes,
                   int reverse, ClipArgs<float> clip, int clip_blocks) {
     using T = float;
-    constexpr int RB = 4;
-    __shared__ double sums[kPlaneWaves][4][64];
+    constexpr int RB = 4, S = 64 / L;
+    __shared__ double sums[TALL ? 2 : 1][kPlaneWaves * S * 4 * L];      // [band][4][L]
 
     // a clip job on the side (its first clip_blocks workgroups): what a training-mode forward does
     // before the integral image, in the same launch
@@ -654,189 +698,111 @@ plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int
     int64_t p = blockIdx.x - clip_blocks;
     if (reverse) p = planes - 1 - p;
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int band = __builtin_amdgcn_readfirstlane(tid >> 6);     // one wave per band
-    const int r0 = band * R;
-    const int r1 = min(h, r0 + R);                                  // (every wave of the launch has rows)
-    const int64_t W1 = static_cast<int64_t>(w) + 1;
-    const int c0 = 4 * lane;
-
-    const TI* src = in + p * static_cast<int64_t>(h) * w;
-    const Rows<const TI, false> irows(src, w, w, h);
-    T* dst = out + p * static_cast<int64_t>(h + 1) * W1;
-    const Rows<T, VEC> orows(dst, W1, w + 1, h + 1);
-    const int in_off = c0 * static_cast<int>(sizeof(TI));
-    const int out_off = (c0 + 1) * static_cast<int>(sizeof(T));
-    const bool lane_in = c0 < w;
-    const unsigned lane_col = lane_in ? static_cast<unsigned>(c0) : 0u;
-
-    // the whole band into registers, all loads in flight together (clamped addresses, values of
-    // rows and lanes that do not exist dropped afterwards)
-    T x[RMAX][4];
-#pragma unroll
-    for (int r = 0; r < RMAX; ++r) {
-        const int row = r0 + r;
-        const bool exists = r < R && row < r1;
-        if (VEC) {
-            load_quad(src + static_cast<int64_t>(min(row, h - 1)) * w + lane_col, x[r]);
-            if (!(exists && lane_in)) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[r][v] = T(0);
-            }
-        } else {
-            buffer_load_run_as<kCacheStream, TI>(x[r], irows.row(min(row, h - 1), exists), in_off);
-        }
-    }
-
-    if (band == 0)
-        for (int c = lane; c <= w; c += 64) dst[c] = T(0);
-
-    {
-        double own[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int r = 0; r < RMAX; ++r)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) own[v] += static_cast<double>(x[r][v]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sums[band][v][lane] = own[v];
-    }
-    __syncthreads();
-    double colacc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = 0; b < band; ++b)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) colacc[v] += sums[b][v][lane];
-
-#pragma unroll
-    for (int bi = 0; bi < RMAX / RB; ++bi) {
-        if (bi * RB >= R) break;
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const int row = r0 + bi * RB + rb;
-            double run = 0.0, pre[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                colacc[v] += static_cast<double>(x[bi * RB + rb][v]);
-                run += colacc[v];
-                pre[v] = run;
-            }
-            const double left = wave_inclusive_scan(run) - run;
-            T res[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) res[v] = static_cast<T>(left + pre[v]);
-            const RowRef orow = orows.row(min(row + 1, h), row < r1);
-            // (VEC: the rows are addressed by offset into one descriptor for the plane, without a
-            // bounds check of their own, so a lane past the row's end must not store)
-            if (!VEC || lane_in)
-                buffer_store_run<kCacheDefault, VEC>(res, orow, out_off, (w + 1) * static_cast<int>(sizeof(T)));
-            if (lane == 0 && row < r1) dst[static_cast<int64_t>(row + 1) * W1] = T(0);
-        }
-    }
-}
-
-// Inclusive prefix sum within segments of L consecutive lanes (L = 16 or 32): the first steps of
-// wave_inclusive_scan. All lanes must be active.
-template <int L>
-__device__ __forceinline__ double segment_inclusive_scan(double x) {
-    static_assert(L == 16 || L == 32, "segments of one or two DPP rows");
-    x += dpp_move<0x111, 0xf>(x, x);
-    x += dpp_move<0x112, 0xf>(x, x);
-    x += dpp_move<0x114, 0xf>(x, x);
-    x += dpp_move<0x118, 0xf>(x, x);
-    if (L == 32) x += dpp_move<0x142, 0xa>(0.0, x);   // lane 15 of rows 0,2 into rows 1,3
-    return x;
-}
-
-// The same for planes of at most 128 (L = 32) or 64 (L = 16) columns, which would leave half or
-// three quarters of every wave idle: a wave takes 64 / L bands side by side, L lanes each (band
-// v of the plane: wave v / (64/L), lanes (v % (64/L)) * L ..), every lane walking down its own
-// band's rows. Rows of a multiple of four columns from a 16-byte aligned address only.
-template <class TI, int RMAX, int L>
-__global__ void __launch_bounds__(kPlaneWaves * 64)
-plane_scan_packed_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int w, int R, int64_t planes,
-                         int reverse, ClipArgs<float> clip, int clip_blocks) {
-    using T = float;
-    constexpr int RB = 4, S = 64 / L;
-    __shared__ double sums[kPlaneWaves * S * 4 * L];      // [band][4][L]
-
-    if (static_cast<int>(blockIdx.x) < clip_blocks) {
-        const int i = blockIdx.x * blockDim.x + threadIdx.x;
-        if (i < clip.n) clip_box(clip, i);
-        return;
-    }
-    int64_t p = blockIdx.x - clip_blocks;
-    if (reverse) p = planes - 1 - p;
-    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     const int l = lane & (L - 1);
-    const int band = (tid >> 6) * S + lane / L;             // per lane; bands past the plane hold no rows
-    const int r0 = band * R;
-    const int r1 = min(h, r0 + R);
+    // (one band per wave: everything about rows is wave-uniform)
+    const int band = S == 1 ? wave : wave * S + lane / L;   // bands past the plane hold no rows
+    const int bands = static_cast<int>(blockDim.x >> 6) * S;
     const int64_t W1 = static_cast<int64_t>(w) + 1;
-    const int c0 = 4 * l;
-    const bool lane_in = c0 < w;
+    const bool lane_in = 4 * l < w;
+    const int c0 = VEC ? 4 * l : min(4 * l, w - 4);
+    const int twice = VEC || !lane_in ? 0 : 4 * l - c0;      // columns that the lane in front holds
+    const int rest = -w & 3;
+    const unsigned lane_col = lane_in ? static_cast<unsigned>(c0) : 0u;
 
     const TI* src = in + p * static_cast<int64_t>(h) * w;
     T* dst = out + p * static_cast<int64_t>(h + 1) * W1;
     const Rows<T, true> orows(dst, W1, w + 1, h + 1);
     const RowRef oplane = orows.row(0);                      // the plane as one buffer; rows by offset
-    const unsigned lane_col = lane_in ? static_cast<unsigned>(c0) : 0u;
+    const int out_off = (c0 + 1) * static_cast<int>(sizeof(T));
 
-    T x[RMAX][4];
+    // (clamped addresses; values of rows and lanes that do not exist are dropped when they are used, and
+    // 16-bit elements widened then: either of them at the load would make the wave wait for it there)
+    Vec4<TI> raw[RMAX];
+    auto load = [&](int row, Vec4<TI>& q) {
+        const TI* at = src + static_cast<int64_t>(min(row, h - 1)) * w;
+        q = load_raw_quad<VEC>(at + lane_col);
+    };
 #pragma unroll
-    for (int r = 0; r < RMAX; ++r) {
-        const int row = r0 + r;
-        const bool exists = r < R && row < r1 && lane_in;
-        load_quad(src + static_cast<int64_t>(min(row, h - 1)) * w + lane_col, x[r]);
-        if (!exists) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) x[r][v] = T(0);
-        }
-    }
+    for (int r = 0; r < RMAX; ++r) load(band * R + r, raw[r]);
 
     if (tid < 64)
         for (int c = tid; c <= w; c += 64) dst[c] = T(0);
 
-    {
+    double above[4] = {0.0, 0.0, 0.0, 0.0};                  // column sums of the chunks above
+    const int chunk = bands * R;
+    int flip = 0;
+    for (int base = 0;; base += chunk) {
+        const int r0 = base + band * R;
+        const int r1 = min(h, r0 + R);
+        const bool more = TALL && base + chunk < h;
         double own[4] = {0.0, 0.0, 0.0, 0.0};
+        T x[RMAX][4];
 #pragma unroll
-        for (int r = 0; r < RMAX; ++r)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) own[v] += static_cast<double>(x[r][v]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sums[(band * 4 + v) * L + l] = own[v];
-    }
-    __syncthreads();
-    double colacc[4] = {0.0, 0.0, 0.0, 0.0};
-    const int wave_last = ((tid >> 6) + 1) * S - 1;         // the wave's last band (wave-uniform)
-    for (int b = 0; b < wave_last; ++b)
-        if (b < band) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) colacc[v] += sums[(b * 4 + v) * L + l];
-        }
-
-#pragma unroll
-    for (int bi = 0; bi < RMAX / RB; ++bi) {
-        if (bi * RB >= R) break;
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const int row = r0 + bi * RB + rb;
-            double run = 0.0, pre[4];
+        for (int r = 0; r < RMAX; ++r) {
+            const bool exists = r < R && r0 + r < r1 && lane_in;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                colacc[v] += static_cast<double>(x[bi * RB + rb][v]);
-                run += colacc[v];
-                pre[v] = run;
-            }
-            const double left = segment_inclusive_scan<L>(run) - run;
-            T res[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) res[v] = static_cast<T>(left + pre[v]);
-            if (row < r1) {
-                const int off = static_cast<int>((static_cast<int64_t>(row + 1) * W1 + c0 + 1) * sizeof(T));
-                if (lane_in) buffer_store_run<kCacheDefault, true>(res, oplane, off, 0);
-                if (l == 0) dst[static_cast<int64_t>(row + 1) * W1] = T(0);
+                x[r][v] = !exists || (!VEC && v < 3 && v < twice) ? T(0) : widen(raw[r].v[v]);
+                own[v] += static_cast<double>(x[r][v]);
             }
         }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sums[flip][(band * 4 + v) * L + l] = own[v];
+        __syncthreads();
+        double colacc[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) colacc[v] = above[v];
+        const int wave_last = (wave + 1) * S - 1;             // the wave's last band (wave-uniform)
+        for (int b = 0; b < wave_last; ++b)
+            if (S == 1 || b < band) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) colacc[v] += sums[flip][(b * 4 + v) * L + l];
+            }
+        if (more)
+            for (int b = 0; b < bands; ++b)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) above[v] += sums[flip][(b * 4 + v) * L + l];
+
+#pragma unroll
+        for (int bi = 0; bi < RMAX / RB; ++bi) {
+            if (bi * RB >= R) break;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const int r = bi * RB + rb, row = r0 + r;
+                double run = 0.0, pre[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    colacc[v] += static_cast<double>(x[r][v]);
+                    run += colacc[v];
+                    pre[v] = run;
+                }
+                const double left = segment_inclusive_scan<L>(run) - run;
+                T res[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) res[v] = static_cast<T>(left + pre[v]);
+                // (the row by the scalar offset of a descriptor where it is the same for the whole wave, which
+                // drops the stores to one that does not exist; else by the lane's offset)
+                const RowRef orow = S == 1 ? orows.row(min(row + 1, h), row < r1) : oplane;
+                const int off = (S == 1 ? 0 : static_cast<int>((static_cast<int64_t>(row + 1) * W1) * sizeof(T))) + out_off;
+                if (S == 1 || row < r1) {
+                    if (lane_in && (VEC || twice == 0)) buffer_store_run<kCacheDefault, true>(res, orow, off, 0);
+                    if (!VEC && twice > 0) {                  // (rest: the same number, scalar: one store)
+                        if (rest == 1) buffer_store_wide<kCacheDefault>({res[1], res[2], res[3]}, orow, off + 4);
+                        else if (rest == 2) buffer_store_wide<kCacheDefault>({res[2], res[3]}, orow, off + 8);
+                        else buffer_store<kCacheDefault>(res[3], orow, off + 12);
+                    }
+                }
+                if (l == 0 && row < r1) dst[static_cast<int64_t>(row + 1) * W1] = T(0);
+            }
+            if (more) {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) load(r0 + chunk + bi * RB + rb, raw[bi * RB + rb]);
+            }
+        }
+        if (!more) break;
+        flip ^= 1;                                            // (two buffers: one barrier per chunk)
     }
 }
 
@@ -946,6 +912,7 @@ struct LookbackByWidth<float, TI> {
 // Bands of the plane-per-workgroup kernels: `slots` bands fit a workgroup (eight waves, times the
 // bands a wave takes side by side); rows per band: whole row batches, at least 8, so that all
 // rows fit those bands.
+inline int plane_row_lanes(int w) { return w <= 64 ? 16 : w <= 128 ? 32 : 64; }
 inline int plane_band_rows(int h, int slots) {
     return std::max(((h + slots - 1) / slots + 3) / 4 * 4, 8);
 }
@@ -957,26 +924,30 @@ hipError_t launch_plane_scan(const TI* in, float* out, int64_t planes, int h, in
     const int rev = reverse ? 1 : 0;
     const bool vec = aligned_for_vec4(in, w);
     // lanes per row: rows of at most 128 / 64 columns share a wave with one / three more bands
-    const int L = (vec && w <= 64) ? 16 : (vec && w <= 128) ? 32 : 64;
+    const int L = plane_row_lanes(w);
     const int S = 64 / L;
-    const int R = plane_band_rows(h, kPlaneWaves * S);
-    const int nb = (h + R - 1) / R;
+    const bool tall = h > kPlaneMaxRows * S;
+    const int most = kPlaneTallRows * kPlaneWaves * S, chunks = tall ? (h + most - 1) / most : 1;
+    const int R = plane_band_rows((h + chunks - 1) / chunks, kPlaneWaves * S);
+    const int nb = std::min((h + R - 1) / R, kPlaneWaves * S);
     const int waves = (nb + S - 1) / S;
     const int clip_blocks = (clip.n + waves * 64 - 1) / (waves * 64);
     const dim3 grid(static_cast<unsigned>(planes + clip_blocks)), block(waves * 64);
-#define LAUNCH_PLANE(RMAX)                                                                                \
-    if (L == 16)  BOXCONV_LAUNCH("band_scan", (plane_scan_packed_kernel<TI, RMAX, 16>), grid, block, 0, stream, \
-                                 in, out, h, w, R, planes, rev, clip, clip_blocks);                       \
-    else if (L == 32) BOXCONV_LAUNCH("band_scan", (plane_scan_packed_kernel<TI, RMAX, 32>), grid, block, 0, stream, \
-                                 in, out, h, w, R, planes, rev, clip, clip_blocks);                       \
-    else if (vec) BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, true>), grid, block, 0, stream, in, out, \
+#define LAUNCH_PLANE_L(RMAX, L_, TALL)                                                                    \
+    if (vec) BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, L_, true, TALL>), grid, block, 0, stream, in, out, \
                             h, w, R, planes, rev, clip, clip_blocks);                                     \
-    else     BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, false>), grid, block, 0, stream, in, out, \
+    else     BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, L_, false, TALL>), grid, block, 0, stream, in, out, \
                             h, w, R, planes, rev, clip, clip_blocks)
-    if (R <= 8)       { LAUNCH_PLANE(8); }
-    else if (R <= 16) { LAUNCH_PLANE(16); }
-    else              { LAUNCH_PLANE(kPlaneRows); }
+#define LAUNCH_PLANE(RMAX, TALL)                                                                          \
+    if (L == 16)      { LAUNCH_PLANE_L(RMAX, 16, TALL); }                                                 \
+    else if (L == 32) { LAUNCH_PLANE_L(RMAX, 32, TALL); }                                                 \
+    else              { LAUNCH_PLANE_L(RMAX, 64, TALL); }
+    if (tall)          { LAUNCH_PLANE(kPlaneTallRows, true) }
+    else if (R <= 8)   { LAUNCH_PLANE(8, false) }
+    else if (R <= 16)  { LAUNCH_PLANE(16, false) }
+    else               { LAUNCH_PLANE(kPlaneRows, false) }
 #undef LAUNCH_PLANE
+#undef LAUNCH_PLANE_L
     return hipGetLastError();
 }
 template <class T, class TI>
@@ -1009,6 +980,17 @@ inline bool scan_by_rows(int h, int w, size_t elem) {
     return w <= kMaxScanRowsWidth && plane_bytes < (1ull << 31);
 }
 
+bool plane_scan_pays(int64_t planes, int h, int w) {
+    if (w < 4 || w > kPlaneMaxCols || planes >= (1ll << 31) || !scan_by_rows(h, w, sizeof(float))) return false;
+    if (h <= kPlaneMaxRows) return true;
+    // Taller ones, as often as the workgroup has to start again. Time over that of the two launches, 3800 shapes of up to
+    // 1100 rows: from 128 planes on 0.11 to 0.65 (578 of 833 x 23 333 -> 94 us, 224 of 296 x 80 57 -> 13, 384
+    // of 360 x 224 117 -> 60); few planes leave the chip to a chain of chunks (2 of 1000 x 256 20 against 49 us,
+    // 3 of 872 x 200 24 against 44; but 36 of 492 x 22 25 -> 13).
+    const int rows = kPlaneTallRows * kPlaneWaves * (64 / plane_row_lanes(w)), chunks = (h + rows - 1) / rows;
+    return switches().plane_integral_tall && chunks <= (planes >= 128 ? 1 << 20 : planes >= 32 ? 3 : w <= 128 ? 2 : 0);
+}
+
 }  // namespace
 
 IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
@@ -1017,8 +999,7 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // (whole row batches) so that up to eight waves share the plane. The rest of the plan is what
     // the types that kernel is not built for take, and what the workspace is sized for.
     // (BOXCONV_INTEGRAL_LOOKBACK=2 asks for the look-back kernel wherever it applies, here too)
-    pl.plane_per_workgroup = switches().plane_integral && !lookback_any_shape() && h <= kPlaneMaxRows &&
-                             w <= kPlaneMaxCols && planes < (1ll << 31);
+    pl.plane_per_workgroup = switches().plane_integral && !lookback_any_shape() && plane_scan_pays(planes, h, w);
     // Enough workgroups to cover 256 CUs several times over, but bands no shorter than 32 rows
     // (the per-band column-sum vector is 8 B per column, i.e. 2/R of the input bytes) and no
     // taller than 256 (size of the per-row carry array in LDS).

@@ -808,3 +808,29 @@ def test_integral_image_switch_one_is_the_default(hip, switches):
     x = torch.randn(1, 16, 301, 767, device="cuda")
     switches("BOXCONV_INTEGRAL_LOOKBACK", "1")
     assert launches(hip, "fill_marker", lambda: hip.integral_image(x)) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("planes,h,w", [
+    # a workgroup per plane, rows of one, two and four lanes' groups of 16: last lanes that share one, two and three
+    # columns, whole rows, a single lane
+    (2, 50, 4), (2, 33, 7), (3, 29, 17), (2, 191, 62), (3, 130, 66), (2, 100, 127), (1, 192, 129), (2, 135, 241), (2, 40, 255),
+    # taller than the workgroup holds at a time: one more row, several chunks, rows of the last chunk missing
+    (2, 769, 33), (3, 1000, 64), (2, 850, 19), (2, 385, 127), (3, 512, 128), (130, 530, 100), (33, 193, 129), (40, 300, 256),
+    (128, 470, 203)])
+def test_integral_image_of_a_plane_per_workgroup(hip, switches, dtype, planes, h, w):
+    """Planes of at most 256 columns in one launch, against the two passes on the same planes, which add the
+    double sums in another order, and against a float64 cumulative sum."""
+    x = torch.randn(1, planes, h, w, generator=torch.Generator().manual_seed(h * w)).cuda().to(dtype)
+    switches("BOXCONV_INTEGRAL_PLANE", "0")
+    two = hip.integral_image(x).clone()
+    switches("BOXCONV_INTEGRAL_PLANE", None)
+    assert launches(hip, "band_colsum", lambda: hip.integral_image(x)) == 0
+    assert launches(hip, "band_scan", lambda: hip.integral_image(x)) == 1
+    one = hip.integral_image(x)
+    assert torch.allclose(one, two, rtol=2e-7, atol=0)
+    want = np.cumsum(np.cumsum(x.double().cpu().numpy(), axis=2), axis=3)
+    got = one.cpu().numpy()
+    assert not got[:, :, 0].any() and not got[..., 0].any()
+    # one rounding to float32, and that of double sums in another order
+    assert (np.abs(got[:, :, 1:, 1:] - want) <= 2.0 ** -24 * np.abs(want) * 1.001 + 1e-12 * np.abs(want).max()).all()
