@@ -40,7 +40,7 @@ PREWARM_MAX_S = 1.5 # upper bound on the untimed clock-up phase after --warmup
 RANKING_STEPS = 3   # untimed eager steps per kernel name while the per-kernel times are taken
 # every kernel a training step launches ("clip" is the parameter projection, which shares its
 # launch with the marking of the single-pass integral image's hand-over words)
-TIMED_KERNELS = ("grad_output_stream", "band_scan", "band_colsum", "forward_rows", "forward_quads", "grad_input_cols",
+TIMED_KERNELS = ("grad_output_stream", "band_scan", "band_colsum", "forward_rows", "forward_quads", "forward_narrow", "grad_input_cols",
                  "grad_input_taps", "clip")
 METRIC = "BoxConv2d fwd+bwd ms/iter + effective HBM GB/s (% peak) at 2x16ch 512x1024 fp32"
 
@@ -58,6 +58,7 @@ def kernel_algorithmic_bytes(ab, elem=4, from_snapshots=False):
         "band_colsum": elem * ab["n_in"],                        # pre-pass over the input
         "forward_rows": elem * (ab["n_int"] + ab["n_out"]),      # read integral, write output
         "forward_quads": elem * (ab["n_int"] + ab["n_out"]),     # the same
+        "forward_narrow": elem * (ab["n_int"] + ab["n_out"]),    # the same
         "grad_input_cols": elem * (ab["n_gint"] + ab["n_in"]),   # read integral of grad_output, write grad_input
         "grad_input_taps": elem * (ab["n_out"] + ab["n_in"]),    # read grad_output, write grad_input
     }

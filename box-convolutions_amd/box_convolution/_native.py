@@ -622,7 +622,7 @@ def training_forward(input, x_min, x_max, y_min, y_max, reparametrization_h, rep
     return integrated, output, real.unbind(0)
 
 
-KERNEL_NAMES = ("band_colsum", "band_prefix", "band_scan", "forward_rows", "forward_quads", "grad_output_stream",
+KERNEL_NAMES = ("band_colsum", "band_prefix", "band_scan", "forward_rows", "forward_quads", "forward_narrow", "grad_output_stream",
                 "grad_input_cols", "grad_input_taps", "param_grad_finalize", "fill_zero", "fill_marker", "clip",
                 "forward_gather", "grad_input_gather", "grad_params_gather", "int_row_prefix",
                 "int_col_prefix")

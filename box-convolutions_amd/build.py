@@ -23,6 +23,11 @@ LIB_PATH = os.path.join(HERE, "box_convolution", "libboxconv_hip.so")
 # the backward kernels and is compiled once per element-type pair and part, so that they build in
 # parallel (one translation unit with all of them takes six minutes).
 def _inst(tag, t, tg, part, same):
+    if part == 9:
+        defs = ["-DBOXCONV_INST_DOUBLE=1"] if t == "double" else ["-DBOXCONV_INST_TO=" + tg]
+        return ("box_forward.hip", "box_forward_%s.o" % tag, defs + (["-DBOXCONV_INST_SAME_TYPE=1"] if same else []))
+    if part == 8:
+        return ("narrow_forward.hip", "narrow_forward_%s.o" % tag, ["-DBOXCONV_INST_TO=" + tg])
     if part == 7:
         return ("narrow_rows.hip", "narrow_rows_%s.o" % tag, ["-DBOXCONV_INST_TG=" + tg])
     if part == 6:                                    # grad_input_taps.hip: a source of its own
@@ -34,13 +39,13 @@ def _inst(tag, t, tg, part, same):
 
 
 SOURCES = [(s, s.replace(".hip", ".o"), []) for s in
-           ("box_sampling.hip", "box_forward.hip", "integral_image.hip", "integral_image_int.hip", "box_misc.hip",
+           ("box_sampling.hip", "integral_image.hip", "integral_image_int.hip", "box_misc.hip",
             "boxconv_c_abi.hip")]
 for _tag, _t, _tg in (("f32", "float", "float"), ("f64", "double", "double"),
                       ("f16", "float", "f16_t"), ("bf16", "float", "bf16_t")):
-    for _part in (1, 2) + ((3, 4, 5, 6, 7) if _t == "float" else ()):
+    for _part in (1, 2, 9) + ((3, 4, 5, 6, 7, 8) if _t == "float" else ()):
         SOURCES.append(_inst(_tag, _t, _tg, _part, _t == _tg))
-HEADERS = ["boxconv_device.hpp", "boxconv_host.hpp", "box_sampling_common.hpp", "box_sampling_impl.hpp",
+HEADERS = ["boxconv_device.hpp", "boxconv_host.hpp", "box_sampling_common.hpp", "box_sampling_impl.hpp", "narrow_rows.hpp", "forward_tail.hpp",
            os.path.join("..", "..", "include", "boxconv.h")]
 
 ARCH = "gfx950"      # the only target: the kernels assume its 160 KiB of LDS per workgroup and its ISA

@@ -3,7 +3,7 @@
 // box_convolution_cuda_forward.cu:28-251). The math and the row-streaming scheme are described at
 // the top of box_sampling.hip.
 
-#include "box_sampling_common.hpp"
+#include "forward_tail.hpp"
 
 namespace boxconv {
 
@@ -13,21 +13,6 @@ namespace {
 // Forward. Work item = (plane p, filter f, band). blockDim = NT, K >= ceil(w / NT).
 // LDS: [2 buffers][w+3] RowPair<T>.
 //
-// TO: element type of the output (T, or a 16-bit type when T is float). TAIL: what happens to a
-// box sum S on its way out, fused into the store (inference only, there is no backward for it):
-//   y = S * channel_scale[c*F+f] + channel_shift[c*F+f]  (+ residual[same pixel])  (max(y, 0))
-// which is the tail of a block such as BoxConv -> BatchNorm (eval) -> residual add -> ReLU.
-// Absent pieces are neutral: a null scale/shift reads as 1/0, a null residual as zeros (its row
-// descriptors get size 0, so the loads return 0 without a branch).
-template <class TO>
-struct ForwardTail {
-    TO* dst;
-    const TO* residual;
-    const float* channel_scale;
-    const float* channel_shift;
-    int relu;
-};
-
 template <class T, class TO, int NT, int K, bool EXACT, bool FULL, bool TAIL>
 __global__ void __launch_bounds__(NT) forward_rows_kernel(SampleArgs<T> a, ForwardTail<TO> tl) {
     const unsigned vid = xcd_contiguous_id(a.per_xcd);
@@ -160,35 +145,21 @@ __global__ void __launch_bounds__(NT) forward_rows_kernel(SampleArgs<T> a, Forwa
     }
 }
 
-// The same for float rows of a multiple of four columns, up to 2048: a lane owns 4 CONSECUTIVE columns, for
-// the integral rows (one 16-byte load per row) as for the output (one 16- or 8-byte store per row), and
-// V sits in LDS by column modulo four (tap_run). The planes hold V[1..w]; the places in front of
-// them stay zero (V[0] = 0 and what clamps to it), those behind hold V[w].
+// The same for float rows of up to 2048 columns: a lane owns 4 CONSECUTIVE columns, for the integral rows
+// (one 16-byte load per row) as for the output (one 16- or 8-byte store per row), and V sits in LDS by
+// column modulo four (tap_run). The planes hold V[1..w]; the places in front of them stay zero (V[0] =
+// 0 and what clamps to it), those behind hold V[w]. Rows that are no multiple of four columns (FIT): the last
+// lane takes the row's last four columns (RowLane) and stores those it shares with its neighbour, too: the
+// same values.
 // The tail's residual: none, or loaded with the ordinary or the streaming cache policy.
 enum ResidualLoads { kNoResidual, kResidualCached, kResidualStreamed };
-template <bool STREAM, class TO>
-__device__ __forceinline__ Quad<TO> load_quad(const TO* p) {
-    typedef unsigned Words __attribute__((ext_vector_type(sizeof(Quad<TO>) / 4)));
-    Words v;
-    if constexpr (STREAM) v = __builtin_nontemporal_load(reinterpret_cast<const Words*>(p));
-    else v = *reinterpret_cast<const Words*>(p);     // (one expression for both would drop the policy)
-    return __builtin_bit_cast(Quad<TO>, v);
-}
-template <class TO>
-__device__ __forceinline__ void store_quad(TO* p, const Quad<TO>& q, bool stream) {
-    typedef unsigned Words __attribute__((ext_vector_type(sizeof(Quad<TO>) / 4)));
-    const Words v = __builtin_bit_cast(Words, q);
-    if (stream) __builtin_nontemporal_store(v, reinterpret_cast<Words*>(p));
-    else *reinterpret_cast<Words*>(p) = v;
-}
-
 // Without a residual nothing is loaded for it (loads of the output in its place, dropped, cost a read as
 // large as the output: 16 x 8 planes of 512 x 1024 in float16 153 -> 91 us, 256 x 4 of 128 x 256 in
 // bfloat16, output not in any cache, 42 -> 26). With one, the rows of the next pair are requested
 // with its integral rows: workgroups of few waves otherwise wait for memory right before the barrier
 // (residual not in any cache, 46 planes of 398 x 140 in float32 12.1 -> 10.0 us, 128 x 4 of 135 x 240
 // in bfloat16 27.7 -> 26.3); with two waves, and from five on, the registers cost more than that brings. Its cache policy: see forward_launch_any.
-template <class TO, int NT, bool EXACT, bool FULL, bool TAIL, int RESIDUAL>
+template <class TO, int NT, bool EXACT, int FIT, bool TAIL, int RESIDUAL>
 __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, ForwardTail<TO> tl) {
     using T = float;
     constexpr int K = 4, PLANE = quad_plane(NT), WAVES = NT / 64;
@@ -206,10 +177,11 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
     const int k_par = static_cast<int>(static_cast<unsigned>(a.plane0 + p) % static_cast<unsigned>(a.C)) * a.F + f;
     const int h = a.h, w = a.w, tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int quads = FULL ? NT : w / K;
-    const int c0 = K * tid;
-    const bool lane_in = FULL || tid < quads;
-    const unsigned cl = lane_in ? static_cast<unsigned>(c0) : 0u;    // idle lanes load the row's first columns and drop them
+    constexpr bool ALIGNED = FIT != kRowAny;
+    const RowLane<NT, FIT> ln(tid, w);
+    const int quads = ln.quads;
+    const bool lane_in = ln.in;
+    const unsigned cl = static_cast<unsigned>(ln.cl);
 
     const BoxOfWorkgroup<T> bx = load_box(a.prm, k_par);
     BoxSplit<T> s = split_forward(bx.xmin, bx.xmax, bx.ymin, bx.ymax);
@@ -233,7 +205,8 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
 
     if (tid < 2 * K * kQuadPad)
         vrow[tid / (K * kQuadPad)][tid / kQuadPad % K][tid % kQuadPad] = RowPair<T>{T(0), T(0)};
-    const TapRun er = tap_run<PLANE>(c0, s.yhi - 1, quads), el = tap_run<PLANE>(c0, s.ylo - 2, quads);
+    const TapRun er = tap_run<PLANE>(ln.c0, s.yhi - 1, quads), el = tap_run<PLANE>(ln.c0, s.ylo - 2, quads);
+    const QuadPlace<PLANE, FIT> place(ln);
     const int last = (quads - 1) & 63;               // lane of the last wave that owns column w
 
     const int i0 = band * a.R;
@@ -248,8 +221,8 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
     load_i(i0 + 2 + s.xhi, b2);
     auto load_residual = [&](int i, Quad<TO>& q0, Quad<TO>& q1) {
         const int64_t row = out0 + static_cast<int64_t>(i) * w;
-        q0 = load_quad<RESIDUAL == kResidualStreamed>(tl.residual + row + cl);
-        q1 = load_quad<RESIDUAL == kResidualStreamed>(tl.residual + (i + 1 < i1 ? row + w : row) + cl);
+        q0 = load_quad<RESIDUAL == kResidualStreamed, ALIGNED>(tl.residual + row + cl);
+        q1 = load_quad<RESIDUAL == kResidualStreamed, ALIGNED>(tl.residual + (i + 1 < i1 ? row + w : row) + cl);
     };
     Quad<TO> res0{}, res1{};
     if (EARLY) load_residual(i0, res0, res1);
@@ -275,14 +248,14 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
             v0[k] = blend<T, EXACT>(ta[k], t0[k], bc[k], b1[k], s.fxlo, s.fxhi);
             v1[k] = blend<T, EXACT>(t0[k], t1[k], b1[k], b2[k], s.fxlo, s.fxhi);
         }
-        if (lane_in) {
 #pragma unroll
-            for (int k = 0; k < K; ++k) vrow[FLIP][k][kQuadPad + tid] = RowPair<T>{v0[k], v1[k]};
-        }
+        for (int k = 0; k < K; ++k) *place.at(vrow[FLIP][0], k) = RowPair<T>{v0[k], v1[k]};
         if (wave == WAVES - 1) {                     // (scalar)
             const RowPair<T> end{read_lane(v0[K - 1], last), read_lane(v1[K - 1], last)};
             const int e = tid & 63;
             if (e < K * kQuadPad) vrow[FLIP][e / kQuadPad][kQuadPad + quads + e % kQuadPad] = end;
+            else if (FIT == kRowAny && e - K * kQuadPad < K && e - K * kQuadPad >= w % K)   // (the rest of the last quad)
+                vrow[FLIP][e - K * kQuadPad][kQuadPad + quads - 1] = end;
         }
         __syncthreads();
 
@@ -302,9 +275,9 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
             narrow(y0, z0.v[k]);
             narrow(y1, z1.v[k]);
         }
-        if (lane_in) {
-            store_quad(tl.dst + row0 + cl, z0, a.stream_out != 0);
-            if (second) store_quad(tl.dst + row1 + cl, z1, a.stream_out != 0);
+        if (FIT == kRowFull || lane_in) {
+            store_quad<ALIGNED>(tl.dst + row0 + cl, z0, a.stream_out != 0);
+            if (second) store_quad<ALIGNED>(tl.dst + row1 + cl, z1, a.stream_out != 0);
         }
         if (PREFETCH) {
 #pragma unroll
@@ -434,6 +407,8 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
     a.stream_out = ((static_cast<uint64_t>(d.w) * sizeof(TO)) % 64 == 0 || out_bytes > (256ull << 20)) ? 1 : 0;
     const dim3 grid(static_cast<unsigned>(a.per_xcd * kXcds));
     if constexpr (std::is_same<T, float>::value) {
+        if (narrow_forward_pays(d.planes, d.F, d.h, d.w, sizeof(TO), TAIL))
+            return narrow_forward_launch<TO>(a, tail, d, TAIL, exact, stream);
         // Four consecutive columns per lane: rows of one wave where one_wave_quads_pay says so, and
         // 16-bit outputs of wider rows, where the other kernel stores 2 bytes per lane. Measured, us, other
         // kernel -> this one: bfloat16 16 x 8 planes of 300 x 768 with the tail 74 -> 50, 1080 x 1920 380 -> 321;
@@ -447,8 +422,10 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
                                                               sizeof(TO), TAIL, tail.residual != nullptr);
         const bool wide_half = sizeof(TO) == 2 && cnt > 64 && (TAIL || (d.w <= 1280 && lanes * 8 >= cnt * 7));
         const size_t align = 4 * sizeof(TO);
-        if (switches().forward_quads && d.w % 4 == 0 && d.w <= 2048 && (one_wave || wide_half) &&
-            reinterpret_cast<uintptr_t>(tail.dst) % align == 0 && reinterpret_cast<uintptr_t>(tail.residual) % align == 0) {
+        const bool quads = d.w % 4 == 0 && (one_wave || wide_half) && reinterpret_cast<uintptr_t>(tail.dst) % align == 0 &&
+                           reinterpret_cast<uintptr_t>(tail.residual) % align == 0;
+        const bool odd = odd_forward_quads_pay(d.planes, d.F, d.h, d.w, sizeof(TO), TAIL);
+        if (switches().forward_quads && d.w <= 2048 && (quads || odd)) {
             // A residual that an earlier layer has just left in the memory-side cache is worth reading from
             // there (256 x 4 planes of 128 x 256 in bfloat16 30 us, 40 with the streaming policy); one that
             // does not fit it beside the output would only push that out (16-bit outputs, 16 x 8 planes of
@@ -469,8 +446,9 @@ hipError_t forward_launch_any(const T* integ, BoxParams<T> prm, ForwardTail<TO> 
     } while (0)
 #define LAUNCH_FQ(NT)                                                                                                  \
     case NT:                                                                                                           \
-        if (lanes == NT) { if (exact) LAUNCH_FQ_TAIL(NT, true, true); else LAUNCH_FQ_TAIL(NT, false, true); }          \
-        else             { if (exact) LAUNCH_FQ_TAIL(NT, true, false); else LAUNCH_FQ_TAIL(NT, false, false); }        \
+        if (odd) { if (exact) LAUNCH_FQ_TAIL(NT, true, kRowAny); else LAUNCH_FQ_TAIL(NT, false, kRowAny); }            \
+        else if (lanes == NT) { if (exact) LAUNCH_FQ_TAIL(NT, true, kRowFull); else LAUNCH_FQ_TAIL(NT, false, kRowFull); } \
+        else     { if (exact) LAUNCH_FQ_TAIL(NT, true, kRowQuads); else LAUNCH_FQ_TAIL(NT, false, kRowQuads); }        \
         break;
             switch (cnt) {
                 LAUNCH_FQ(64) LAUNCH_FQ(128) LAUNCH_FQ(192) LAUNCH_FQ(256)
@@ -507,14 +485,15 @@ hipError_t forward_fused_launch(const float* integ, BoxParams<float> prm, TO* ou
     return forward_launch_any<float, TO, true>(integ, prm, tail, d, normalize, exact, stream);
 }
 
-template hipError_t forward_launch<float>(const float*, BoxParams<float>, float*, Dims, bool, bool, hipStream_t);
+// Compiled once per element type of the output (BOXCONV_INST_TO).
+#ifdef BOXCONV_INST_DOUBLE
 template hipError_t forward_launch<double>(const double*, BoxParams<double>, double*, Dims, bool, bool, hipStream_t);
-#define BOXCONV_INSTANTIATE_FUSED(TO)                                                              \
-    template hipError_t forward_fused_launch<TO>(const float*, BoxParams<float>, TO*, const TO*,   \
-                                                 const float*, const float*, bool, Dims, bool,     \
-                                                 bool, hipStream_t);
-BOXCONV_INSTANTIATE_FUSED(float)
-BOXCONV_INSTANTIATE_FUSED(f16_t)
-BOXCONV_INSTANTIATE_FUSED(bf16_t)
+#else
+template hipError_t forward_fused_launch<BOXCONV_INST_TO>(const float*, BoxParams<float>, BOXCONV_INST_TO*, const BOXCONV_INST_TO*,
+                                                          const float*, const float*, bool, Dims, bool, bool, hipStream_t);
+#ifdef BOXCONV_INST_SAME_TYPE
+template hipError_t forward_launch<float>(const float*, BoxParams<float>, float*, Dims, bool, bool, hipStream_t);
+#endif
+#endif
 
 }  // namespace boxconv

@@ -46,6 +46,7 @@ Switches read_switches() {
     s.interleave_workspace = flag_unless_zero("BOXCONV_M_INTERLEAVE");
     s.forward_quads = flag_unless_zero("BOXCONV_FWD_QUADS");
     e = text("BOXCONV_FWD_QUADS");
+    s.odd_forward_quads = e == nullptr || std::atoi(e) != 1;
     s.quads_any_size = e != nullptr && std::atoi(e) == 2;
     s.input_from_snapshots = flag_unless_zero("BOXCONV_GI_SNAPSHOTS");
     e = text("BOXCONV_GI_SNAPSHOTS");
@@ -220,6 +221,40 @@ bool narrow_rows_pay(int64_t planes, int F, int h, int w) {
     const int64_t pixels = planes * h * w;
     return h >= (w <= 32 ? 24 : w <= 64 ? 20 : 16) && pixels >= 1500 * static_cast<int64_t>(F) &&
            pixels * F >= (h <= 400 ? 1 << 17 : 1 << 21);
+}
+
+// Output and integral images that no longer fit the memory-side cache together.
+static bool beyond_memory_side_cache(int64_t planes, int F, int h, int w, size_t elem_size) {
+    return planes * (static_cast<int64_t>(F) * h * w * static_cast<int64_t>(elem_size) + static_cast<int64_t>(h + 1) * (w + 1) * 4) >= (256ll << 20);
+}
+
+// Forward of rows of at most 128 columns with several of them side by side in a wave (narrow_forward.hip)
+// against forward_rows_kernel, timed on 7400 shapes (float32; bfloat16 with and without the tail and a residual): 0.71,
+// 0.68 and 0.70 of the time in the geometric mean, 3 shapes more than 3 % slower. Not for float32 rows of more
+// than 32 columns without a tail that the memory-side cache does not hold (0.9 to 1.8), nor where
+// one_wave_quads_pay decides.
+bool narrow_forward_pays(int64_t planes, int F, int h, int w, size_t elem_size, bool tail) {
+    const Switches& sw = switches();
+    if (!sw.forward_quads || !sw.narrow_rows || w < 16 || w > 128 || h >= (1 << 22)) return false;
+    if (sw.narrow_any_size) return true;
+    if (sw.quads_any_size || (w >= 96 && w < 128 && w % 4 == 0)) return false;
+    return w <= 32 || elem_size == 2 || tail || !beyond_memory_side_cache(planes, F, h, w, elem_size);
+}
+
+// forward_quads_kernel on rows that are no multiple of four columns, against forward_rows_kernel, timed on 9900
+// shapes: with a tail 0.83 of the time (0.56 to 1.09); without one, by this rule, 0.95 in float32 and 0.92 in bfloat16
+// (0.68 to 1.09). Left out: three or four columns per lane of one or two waves, which idle less in the other kernel
+// (129 to 191 columns 1.06 to 1.11 from 2^20 output pixels on, 257 to 384 columns 1.01 to 1.06 from 2^22), 769 to
+// 1024 columns below 2^20 (1.03), and wide float32 rows that the memory-side cache does not hold (1.03 to 1.2).
+bool odd_forward_quads_pay(int64_t planes, int F, int h, int w, size_t elem_size, bool tail) {
+    const Switches& sw = switches();
+    if (!sw.forward_quads || !sw.odd_forward_quads || w % 4 == 0 || w <= 128 || w > 2048) return false;
+    if (sw.quads_any_size || tail) return true;
+    const int64_t pixels = planes * F * h * w;
+    if (elem_size == 4 && beyond_memory_side_cache(planes, F, h, w, elem_size)) return w <= 256;
+    if (w < 192) return pixels < (1 << 20);
+    if (w > 256 && w <= 384) return pixels < (1 << 22);
+    return w <= 768 || w > 1024 || pixels >= (1 << 20);
 }
 
 int narrow_filter_sets(int64_t workgroups, int F) {

@@ -173,6 +173,10 @@ template <class TG>
 hipError_t narrow_input_launch(const TG* grad_out, const float* snapshots, const SnapshotPlan& plan, const StreamPlan& sp,
                                BoxParams<float> prm, TG* grad_in, Dims d, bool normalize, bool exact, hipStream_t stream,
                                const ParamFinish<float>* finish, bool* finish_done);
+// Which forward kernels take a launch with outputs of elem_size bytes: narrow_forward_kernel, forward_quads_kernel
+// for rows that are no multiple of four columns.
+bool narrow_forward_pays(int64_t planes, int F, int h, int w, size_t elem_size, bool tail);
+bool odd_forward_quads_pay(int64_t planes, int F, int h, int w, size_t elem_size, bool tail);
 // Sets of threads of narrow_input_kernel that share the filters of a launch of `workgroups`.
 int narrow_filter_sets(int64_t workgroups, int F);
 
@@ -256,6 +260,7 @@ struct Switches {
     bool snapshots_any_shape;   // BOXCONV_GI_SNAPSHOTS=2: from snapshots for every shape that way covers
     bool forward_quads;       // BOXCONV_FWD_QUADS=0 clears it: no forward kernel with four consecutive columns per lane
     bool quads_any_size;      // BOXCONV_FWD_QUADS=2: that kernel for rows of one wave in launches of any size
+    bool odd_forward_quads;   // BOXCONV_FWD_QUADS=1 clears it: that kernel only for rows of a multiple of four columns
     int stream_workgroups;    // BOXCONV_STREAM_WGS: workgroups the grad_output pass aims for when it cuts planes into bands (2048)
     int spin_limit;           // BOXCONV_INTEGRAL_SPIN: polls of a hand-over word before re-summing (64)
     int fwd_threads;          // BOXCONV_FWD_THREADS: 256 or 512 (512)

@@ -322,6 +322,54 @@ def test_forward_with_consecutive_columns(switches, dtype, h, w, tail, exact):
         assert ((a - b).abs() <= unit * b.abs() + 1e-6 * b.abs().max()).all()
 
 
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("tail", [False, True])
+@pytest.mark.parametrize("name,dtype,h,w", [
+    # several rows side by side in a wave: 8, 16 and 32 lanes per row, whole and with a last lane that shares columns
+    ("forward_narrow", torch.float32, 28, 28), ("forward_narrow", torch.float16, 9, 16), ("forward_narrow", torch.bfloat16, 130, 17),
+    ("forward_narrow", torch.float32, 3, 23), ("forward_narrow", torch.float32, 40, 33), ("forward_narrow", torch.float16, 64, 64),
+    ("forward_narrow", torch.bfloat16, 37, 63), ("forward_narrow", torch.float32, 65, 65), ("forward_narrow", torch.bfloat16, 70, 96),
+    ("forward_narrow", torch.float16, 21, 127), ("forward_narrow", torch.float32, 200, 128),
+    # rows of a wave and more that are no multiple of four columns
+    ("forward_quads", torch.float32, 17, 129), ("forward_quads", torch.bfloat16, 12, 255), ("forward_quads", torch.float16, 11, 257),
+    ("forward_quads", torch.float32, 9, 514), ("forward_quads", torch.bfloat16, 13, 767), ("forward_quads", torch.float32, 7, 1021),
+    ("forward_quads", torch.float16, 8, 2047)])
+def test_forward_of_narrow_and_odd_rows(switches, name, dtype, h, w, tail, exact):
+    """The forward kernels for rows of at most 128 columns (BOXCONV_NARROW=2) and for rows that are no multiple
+    of four columns (BOXCONV_FWD_QUADS=2) against the one with wave-strided columns (BOXCONV_FWD_QUADS=0): the
+    same expressions per pixel, so at most the contraction of a product and a sum differs, or one rounding to
+    16 bits. Boxes hang over every edge; the output's memory holds NaN beforehand."""
+    from box_convolution import _native as hip
+    gen = torch.Generator().manual_seed(h * w)
+    B, C, F = 2, 3, 2
+    x = torch.randn(B, C, h, w, generator=gen).cuda().to(dtype)
+    lo_x, lo_y = ((torch.rand(C, F, generator=gen) * 2 - 1.2) * n for n in (h, w))
+    boxes = [t.cuda() for t in (lo_x, lo_x + 2.2 + torch.rand(C, F, generator=gen) * h,
+                                lo_y, lo_y + 2.2 + torch.rand(C, F, generator=gen) * w)]
+    integ = hip.integral_image(x)
+    variants = [(None, None, None, False)]
+    if tail:
+        scale, shift = torch.rand(C * F, generator=gen).cuda(), torch.randn(C * F, generator=gen).cuda()
+        residual = torch.randn(B, C * F, h, w, generator=gen).cuda().to(dtype)
+        variants = [(scale, shift, residual, True), (scale, None, None, True)]
+    for args in variants:
+        results = []
+        for variant in ("2", "0"):
+            switches("BOXCONV_NARROW" if name == "forward_narrow" else "BOXCONV_FWD_QUADS", "2" if variant == "2" else None)
+            if variant == "0":
+                switches("BOXCONV_FWD_QUADS", "0")
+            filler = torch.full((B, C * F, h, w), float("nan"), device="cuda", dtype=dtype)
+            del filler                                   # (the allocator hands this block out next)
+            hip.profile_arm(name)
+            results.append(hip.box_convolution_forward_fused(integ, *boxes, True, exact, dtype, *args).float())
+            assert hip.profile_collect()[1] == (variant == "2")
+            switches("BOXCONV_FWD_QUADS", None)
+        a, b = results
+        assert torch.isfinite(a).all()
+        unit = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+        assert ((a - b).abs() <= unit * b.abs() + 1e-6 * b.abs().max()).all()
+
+
 def test_tail_without_residual_loads_none():
     """Scale, shift and ReLU alone move half the bytes of the same tail with a residual (a load of
     something else in its place, thrown away, would take as long). Kernel times at a size that no
