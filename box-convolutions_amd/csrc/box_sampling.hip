@@ -134,6 +134,19 @@ StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t e
     if (sums_only && elem_size == 4 && consecutive_rows(w) && consecutive_threads(w) == 64)
         nb = std::max(nb, static_cast<int>(std::min<int64_t>(2 * switches().stream_workgroups / std::max<int64_t>(planes_f, 1),
                                                              std::max(1, h / 32))));
+    // Rows of five, six and seven waves: a CU holds two such workgroups, a third would need its SIMDs to be
+    // shared more evenly than they are, so as many bands as make one round of two per CU, where that
+    // many come to 7/8 of it at least. Both backward kernels with snapshots / the sums alone: 16 x 8 planes of
+    // 720 x 1280 313 -> 270 / 151 -> 118 us, 8 x 8 of 900 x 1792 260 -> 223 / 114 -> 100, 32 x 4 of 400 x 1200
+    // 195 -> 172 / 89 -> 68; at 0.78 of it 0.94 to 1.02 of the time, and one band per plane, which cannot be cut
+    // to fit, 1.0 to 1.24. Four waves are worse off (16 x 8 of 512 x 1024 265 -> 287), as are eight
+    // (1024 x 2048 1455 -> 1615).
+    const int waves = consecutive_threads(w) / 64;
+    if (sums_only && elem_size == 4 && consecutive_rows(w) && waves >= 5 && waves <= 7) {
+        const int64_t one_round = switches().stream_workgroups / 4;
+        const int64_t bands = std::min<int64_t>(one_round / std::max<int64_t>(planes_f, 1), h / 32);
+        if (bands >= 2 && bands * planes_f * 8 >= one_round * 7) nb = static_cast<int>(bands);
+    }
     int R = (h + nb - 1) / nb;
     R += R & 1;                                        // rows are handled in pairs
     sp.R = std::max(R, 2);
@@ -181,9 +194,10 @@ namespace {
 // grad_output_stream_kernel (0.70 to 0.85 of its time from 2^24 output pixels on, 0.88 to 1.0 below); in addition
 //  * fewer than 40 rows (487 x 4 planes of 33 x 151 47 against 56 us, 90 x 8 of 34 x 506 46 against 54), or
 //    up to 192 columns and fewer than 2^24 output pixels (5 x 4 of 1055 x 171 45 against 51), are up to 1.2;
-//  * three waves and more whose last one has a single lane in use keep the workspace (16 x 8 planes of
+//  * three waves whose last one has a single lane in use keep the workspace (16 x 8 planes of
 //    512 x 514 128 us that way, 115 by snapshots, 162 before this kernel took such rows: what a launch of
-//    that size returns is fixed bit for bit).
+//    that size returns is fixed bit for bit). Of more waves that costs less than the workspace does (16 x 8 planes
+//    of 512 x 1025 321 -> 183 us, of 720 x 1281 466 -> 291).
 bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
     if (!consecutive_rows(w)) return false;
     if (switches().snapshots_any_shape) return true;
@@ -192,7 +206,7 @@ bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
     // resident: three waves per SIMD, ten workgroups of one wave by their LDS. Of two workgroups of five or
     // six waves on a CU the second slows the first by as much as it brings: they count as two rounds
     const int waves = consecutive_threads(w) / 64;
-    if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) || (waves > 2 && (w + 3) / 4 % 64 == 1))) return false;
+    if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) || (waves == 3 && (w + 3) / 4 % 64 == 1))) return false;
     const int64_t workgroups = planes * ((h + 7) / 8), resident = 256 * (waves == 1 ? 10 : 12 / waves);
     return workgroups <= (waves > 4 ? 256 : resident) || workgroups * F >= 4 * resident;
 }

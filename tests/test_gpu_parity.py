@@ -692,6 +692,33 @@ def test_grad_output_pass_of_odd_rows_half(hip, switches, h, w, dtype):
         assert torch.equal(p, q)
 
 
+@pytest.mark.parametrize("h,w", [(66, 1029), (65, 1281), (67, 1534), (64, 1536), (66, 1792)])
+def test_bands_that_make_one_round(hip, switches, h, w):
+    """Rows of five to seven waves of 256 planes and filters: two long bands each, 512 workgroups, with
+    snapshots and for the parameter sums alone, against the kernel with wave-strided columns (0). 1029 and 1281
+    columns end with a wave, 1281 with a single lane in use, 1536 and 1792 with a full one."""
+    rng = np.random.default_rng(h * w)
+    C, F = 32, 8
+    integ = hip.integral_image(dev(rng.standard_normal((1, C, h, w)).astype(np.float32)))
+    g = dev((rng.standard_normal((1, C * F, h, w)) + 0.25).astype(np.float32))
+    boxes = [dev(b) for b in make_boxes(rng, C, F, h, w, "hanging", away_from_integers=0.05)]
+
+    def backward(need_input):
+        return hip.box_convolution_backward(integ, *boxes, g, None, 3.5 * h, 2.25 * w, True, True,
+                                            need_input, True, True, True, True)
+    assert launches(hip, "grad_input_taps", lambda: backward(True)) == 1
+    full, alone = backward(True), backward(False)
+    switches("BOXCONV_STREAM_CONSEC", "0")
+    ref = backward(True)
+    assert (full[0] - ref[0]).abs().max() <= 4e-6 * ref[0].abs().max()
+    # as in assert_parity: the order of the float32 sums inside a row differs, each term a difference of
+    # integral-image entries that are known to half a unit in the last place, over h * w pixels
+    noise = 2.0 ** -23 * integ.abs().max() * g.abs().max() * 3.5 * (h * w) ** 0.5
+    for p, q, r, side in zip(full[1:], alone[1:], ref[1:], (h, h, w, w)):
+        assert torch.equal(p, q)
+        assert (p - r).abs().max() <= 1e-5 * r.abs().max() + noise * side
+
+
 NARROW_SHAPES = [
     # 8, 16 and 32 lanes per row, full, with idle lanes, and with a last lane that shares columns; one band,
     # bands past the plane, several waves per plane; filters shared by 1, 2, 4 and 8 waves, evenly or not
