@@ -43,11 +43,49 @@ namespace {
 template <class T>
 struct alignas(4 * sizeof(T)) Vec4 { T v[4]; };
 
+// How the kernels with four consecutive columns per lane read a row.
+enum RowLoads {
+    kElements,      // element by element (elements that are not aligned; rows of fewer than 4 columns)
+    kAlignedQuads,  // rows of a multiple of four columns, 16-byte (8-byte) aligned: one load per lane
+    kShiftedQuads,  // any other row: one load per lane from an address that is aligned to the element. The lane
+                    // whose four columns straddle the row's end reads the row's last four columns
+                    // and shifts them; nothing outside the row is touched
+};
+
+// Four consecutive elements from an address that is aligned to the element only, one load (16 or 8
+// bytes; a global load need not be aligned here).
+__device__ __forceinline__ void load_quad_unaligned(const float* p, float (&v)[4]) {
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    const f4 q = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+template <class H>
+__device__ __forceinline__ void load_quad_unaligned(const H* p, float (&v)[4]) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2), aligned(2)));
+    const u2 q = __builtin_nontemporal_load(reinterpret_cast<const u2*>(p));
+    f16_t raw[4];
+    unpack_quad(q.x, q.y, raw);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = widen(H{raw[k].bits});
+}
+
+// kShiftedQuads: four loaded elements, moved to the columns that the lane owns (it loaded `shift` columns
+// further to the left); zeros for those behind the row's end.
+__device__ __forceinline__ void shift_quad(float (&x)[4], int shift) {
+    const float q[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        x[v] = 0.0f;
+#pragma unroll
+        for (int u = v; u < 4; ++u) x[v] = shift == u - v ? q[u] : x[v];
+    }
+}
+
 // ---- pass 1 -----------------------------------------------------------------------------------
 // One workgroup per (plane, band, strip of 1024 columns); lane `tid` owns 4 consecutive columns
-// and keeps 8 row loads in flight. VEC: rows are 16-byte aligned and w is a multiple of 4.
+// and keeps 8 row loads in flight. LOADS: a RowLoads.
 // TI: element type of the input (T, or a 16-bit type widened to T = float on load).
-template <class T, class TI, bool VEC>
+template <class T, class TI, int LOADS>
 __global__ void __launch_bounds__(256)
 band_colsum_kernel(const TI* __restrict__ in, double* __restrict__ aux, int h, int w, int nb,
                    int R, int strips) {
@@ -64,17 +102,28 @@ band_colsum_kernel(const TI* __restrict__ in, double* __restrict__ aux, int h, i
     const Rows<const TI, false> irows(src, w, w, h);
     const int off = c0 * static_cast<int>(sizeof(TI));
 
+    const int lane_col = min(c0, w - 4), shift = c0 - lane_col;      // kShiftedQuads
+    const bool straddles = (c0 & ~255) + 256 > w;                    // (the wave of the row's end or behind it)
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int r = r0; r < r1; r += U) {
         T x[U][4];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (VEC) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[u][v] = T(0);
-                if (r + u < r1 && c0 < w) load_quad(src + static_cast<int64_t>(r + u) * w + c0, x[u]);
+            if constexpr (LOADS == kShiftedQuads) {
+                load_quad_unaligned(src + static_cast<int64_t>(min(r + u, r1 - 1)) * w + lane_col, x[u]);
+            } else if constexpr (LOADS == kAlignedQuads) {
+                load_quad(src + static_cast<int64_t>(min(r + u, r1 - 1)) * w + lane_col, x[u]);
             } else {
                 buffer_load_run_as<kCacheDefault, TI>(x[u], irows.row(min(r + u, h - 1), r + u < r1), off);
+            }
+        }
+        if constexpr (LOADS != kElements) {       // (unconditional loads, all in flight together)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if constexpr (LOADS == kShiftedQuads)
+                    if (__builtin_amdgcn_readfirstlane(straddles)) shift_quad(x[u], shift);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x[u][v] = r + u < r1 ? x[u][v] : T(0);
             }
         }
 #pragma unroll
@@ -248,8 +297,14 @@ band_scan_kernel(const T* __restrict__ in, T* __restrict__ out, const double* __
 // column sums (the sum over the bands above is formed here, no band_prefix pass); the loads of the
 // next RB rows are in flight while the current ones are scanned; there is one barrier per RB rows
 // (wave totals, double-buffered) and results are stored straight from registers, 4 consecutive
-// elements per lane. VEC: rows are 16-byte aligned and w is a multiple of 4. FULL: w == 4 * threads.
-template <class T, class TI, int WAVES, int RB, bool VEC, bool FULL>
+// elements per lane. As many waves as the row needs at 256 columns each, 16 above 2048. FULL: w == 4 * threads.
+// Bound by its stores and, where planes are cut into bands, by reading the input twice. LOADS (RowLoads): rows of no
+// multiple of four columns used to be read element by element, and the others' loads were behind branches that
+// made each row wait for the one before; with one unconditional load per lane and row, and
+// 5 to 7 waves instead of 8, this launch and band_colsum, float32: 806 planes of 128 x 1055 422 -> 258 us (205 in one
+// band each), 44 of 795 x 954 115 -> 79, 182 of 512 x 384 105 -> 78, 37 of 720 x 2038 194 -> 122; from float16 280 of
+// 400 x 300 149 -> 81, 450 of 160 x 300 88 -> 51.
+template <class T, class TI, int WAVES, int RB, int LOADS, bool FULL>
 __global__ void __launch_bounds__(WAVES * 64)
 band_scan_rows_kernel(const TI* __restrict__ in, T* __restrict__ out, const double* __restrict__ aux,
                       int h, int w, int nb, int R, int64_t total, int64_t per_xcd, int reverse) {
@@ -291,14 +346,16 @@ band_scan_rows_kernel(const TI* __restrict__ in, T* __restrict__ out, const doub
         }
     }
 
+    const int lane_col = min(c0, w - 4), shift = c0 - lane_col;      // kShiftedQuads
     auto load_batch = [&](int rbase, T (&x)[RB][4]) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const int row = rbase + rb;
-            if (VEC) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[rb][v] = T(0);
-                if (row < r1 && c0 < w) load_quad(src + static_cast<int64_t>(row) * w + c0, x[rb]);
+            if constexpr (LOADS != kElements) {
+                // (rows past the band: its last one again, whose sums go nowhere)
+                const TI* rowp = src + static_cast<int64_t>(min(row, r1 - 1)) * w + lane_col;
+                if constexpr (LOADS == kShiftedQuads) load_quad_unaligned(rowp, x[rb]);
+                else load_quad(rowp, x[rb]);
             } else {
                 buffer_load_run_as<kCacheStream, TI>(x[rb], irows.row(min(row, h - 1), row < r1), in_off);
             }
@@ -310,8 +367,14 @@ band_scan_rows_kernel(const TI* __restrict__ in, T* __restrict__ out, const doub
     int buf = 0;
     for (int rbase = r0; rbase < r1; rbase += RB) {
         T nx[RB][4];
-        load_batch(rbase + RB, nx);               // rows past the band come back as zeros, unread
+        load_batch(rbase + RB, nx);
 
+        if constexpr (LOADS == kShiftedQuads) {
+            if (wave * 256 + 256 > w) {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) shift_quad(x[rb], shift);
+            }
+        }
         double pre[RB][4], excl[RB];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
@@ -405,32 +468,6 @@ clip_and_fill_marker_kernel(ClipArgs<T> clip, int clip_blocks, unsigned long lon
     if (i < n) dst[i] = kNotPublished;
 }
 
-// How band_scan_lookback_kernel reads a row.
-enum RowLoads {
-    kElements,      // element by element (elements that are not aligned; rows of fewer than 4 columns)
-    kAlignedQuads,  // rows of a multiple of four columns, 16-byte (8-byte) aligned: one load per lane
-    kShiftedQuads,  // any other row: one load per lane from an address that is aligned to the element. The lane
-                    // whose four columns straddle the row's end reads the row's last four columns
-                    // and shifts them; nothing outside the row is touched
-};
-
-// Four consecutive elements from an address that is aligned to the element only, one load (16 or 8
-// bytes; a global load need not be aligned here).
-__device__ __forceinline__ void load_quad_unaligned(const float* p, float (&v)[4]) {
-    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
-    const f4 q = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-}
-template <class H>
-__device__ __forceinline__ void load_quad_unaligned(const H* p, float (&v)[4]) {
-    typedef unsigned u2 __attribute__((ext_vector_type(2), aligned(2)));
-    const u2 q = __builtin_nontemporal_load(reinterpret_cast<const u2*>(p));
-    f16_t raw[4];
-    unpack_quad(q.x, q.y, raw);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = widen(H{raw[k].bits});
-}
-
 template <class TI, int WAVES, int RB, int LOADS, bool FULL>
 __global__ void __launch_bounds__(WAVES * 64)
 band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, double* aux,
@@ -488,24 +525,13 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
             buffer_load_run_as<kCacheStream, TI>(x, irows.row(min(row, h - 1), exists), in_off);
         }
     };
-    // kShiftedQuads: what the last wave's lanes loaded, moved to the columns they own
-    auto shift_row = [&](T (&x)[4]) {
-        const T q[4] = {x[0], x[1], x[2], x[3]};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            x[v] = T(0);
-#pragma unroll
-            for (int u = v; u < 4; ++u) x[v] = shift == u - v ? q[u] : x[v];
-        }
-    };
-
     // -- the whole band into registers, its column sums published
     T x[RMAX][4];
 #pragma unroll
     for (int r = 0; r < RMAX; ++r) load_row(r0 + r, r < R && r0 + r < r1, x[r]);
     if (LOADS == kShiftedQuads && wave == WAVES - 1) {   // (scalar; the launch has no more waves than the row needs)
 #pragma unroll
-        for (int r = 0; r < RMAX; ++r) shift_row(x[r]);
+        for (int r = 0; r < RMAX; ++r) shift_quad(x[r], shift);
     }
 
     if (band == 0)
@@ -576,7 +602,7 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
                 for (int r = b * R; r < (b + 1) * R; ++r) {      // bands above are complete bands
                     T t[4];
                     load_row(r, true, t);
-                    if (LOADS == kShiftedQuads && wave == WAVES - 1) shift_row(t);
+                    if (LOADS == kShiftedQuads && wave == WAVES - 1) shift_quad(t, shift);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) part[v] += static_cast<double>(t[v]);
                 }
@@ -811,6 +837,11 @@ bool aligned_for_vec4(const T* p, int w) {
     return (w % 4 == 0) && (reinterpret_cast<uintptr_t>(p) % (4 * sizeof(T)) == 0);
 }
 
+template <class TI>
+bool shifted_quads_apply(const TI* p, int w) {
+    return w >= 4 && reinterpret_cast<uintptr_t>(p) % sizeof(TI) == 0;
+}
+
 template <class T, int WAVES, int M, int RB>
 hipError_t launch_scan(const T* in, T* out, const double* aux, int64_t planes, int h, int w,
                        int nb, int R, bool reverse, hipStream_t stream) {
@@ -837,12 +868,15 @@ hipError_t launch_scan_rows(const TI* in, T* out, const double* aux, int64_t pla
     const dim3 grid(static_cast<unsigned>(per_xcd * kXcds));
     const dim3 block(WAVES * 64);
     const bool vec = aligned_for_vec4(in, w), full = (w == WAVES * 256);
-#define LAUNCH_ROWS(VEC, FULL)                                                                     \
-    BOXCONV_LAUNCH("band_scan", (band_scan_rows_kernel<T, TI, WAVES, RB, VEC, FULL>), grid, block, 0,  \
+#define LAUNCH_ROWS(LOADS, FULL)                                                                   \
+    BOXCONV_LAUNCH("band_scan", (band_scan_rows_kernel<T, TI, WAVES, RB, LOADS, FULL>), grid, block, 0,  \
                    stream, in, out, aux, h, w, nb, R, total, per_xcd, rev)
-    if (vec && full) LAUNCH_ROWS(true, true);
-    else if (vec)    LAUNCH_ROWS(true, false);
-    else             LAUNCH_ROWS(false, false);
+    if (vec && full) { LAUNCH_ROWS(kAlignedQuads, true); }
+    else if (vec)    { LAUNCH_ROWS(kAlignedQuads, false); }
+    else if constexpr (std::is_same<T, float>::value) {
+        if (shifted_quads_apply(in, w)) { LAUNCH_ROWS(kShiftedQuads, false); }
+        else                            { LAUNCH_ROWS(kElements, false); }
+    } else               { LAUNCH_ROWS(kElements, false); }
 #undef LAUNCH_ROWS
     return hipGetLastError();
 }
@@ -879,7 +913,7 @@ hipError_t launch_lookback(const TI* in, float* out, double* aux, int64_t planes
     if (aligned_for_vec4(in, w)) {
         LAUNCH_LOOKBACK(kAlignedQuads, true);
     } else {
-        if (w >= 4 && reinterpret_cast<uintptr_t>(in) % sizeof(TI) == 0) LAUNCH_LOOKBACK(kShiftedQuads, false);
+        if (shifted_quads_apply(in, w)) LAUNCH_LOOKBACK(kShiftedQuads, false);
         else LAUNCH_LOOKBACK(kElements, false);
     }
 #undef LAUNCH_LOOKBACK
@@ -1042,9 +1076,14 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     const bool all_resident = groups <= resident && bands32 <= 32;
     const bool short_bands = min_rows == 16 && w <= 512 && planes * h * w < (3 << 19);
     const bool measured_faster = w >= 256 && (w % 4 == 0 ? all_resident || groups >= 4096 : all_resident && !short_bands);
+    // Enough planes for a workgroup each: no second pass over the input (it takes 0.63 to 0.97 of the time of the two
+    // from there on, down to 280 planes of four waves and more: 450 of 64 x 1024 64 -> 40 us, 640 of 250 x 1501 525 ->
+    // 415, 280 of 250 x 2048 in float16 86 -> 79; before that, 450 of 64 x 512 27 -> 32, 280 of 250 x 701 in float16 100 -> 111).
+    const bool one_band = w > 256 && w <= 2048 && planes >= 280 && planes * waves >= 1280;
     const bool single_pass = wanted >= 2 && h > kLookbackRows && w <= 2048 && scan_by_rows(h, w, sizeof(float)) &&
                              bands32 <= kLookbackBands && (lookback_any_shape() || measured_faster);
     if (single_pass) nb = (h + kLookbackRows - 1) / kLookbackRows;
+    if (!single_pass && one_band) nb = 1;
     nb = std::max(nb, (h + 255) / 256);
     nb = std::max(nb, 1);
     int R = (h + nb - 1) / nb;
@@ -1128,12 +1167,15 @@ hipError_t integral_image_any(const TI* in, T* out, int64_t planes, int h, int w
     if (nb > 1) {
         const int strips = (w + 1023) / 1024;
         const dim3 grid(static_cast<unsigned>(planes * (nb - 1) * strips));
-        if (aligned_for_vec4(in, w))
-            BOXCONV_LAUNCH("band_colsum", (band_colsum_kernel<T, TI, true>), grid, dim3(256), 0, stream,
-                           in, aux, h, w, nb, R, strips);
-        else
-            BOXCONV_LAUNCH("band_colsum", (band_colsum_kernel<T, TI, false>), grid, dim3(256), 0, stream,
-                           in, aux, h, w, nb, R, strips);
+#define LAUNCH_COLSUM(LOADS)                                                                       \
+        BOXCONV_LAUNCH("band_colsum", (band_colsum_kernel<T, TI, LOADS>), grid, dim3(256), 0, stream, \
+                       in, aux, h, w, nb, R, strips)
+        if (aligned_for_vec4(in, w)) { LAUNCH_COLSUM(kAlignedQuads); }
+        else if constexpr (std::is_same<T, float>::value) {
+            if (shifted_quads_apply(in, w)) { LAUNCH_COLSUM(kShiftedQuads); }
+            else                            { LAUNCH_COLSUM(kElements); }
+        } else { LAUNCH_COLSUM(kElements); }
+#undef LAUNCH_COLSUM
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -1146,11 +1188,17 @@ hipError_t integral_image_any(const TI* in, T* out, int64_t planes, int h, int w
         if (e != hipSuccess) return e;
     }
     if (by_rows) {
-        if (w <= 256)       return launch_scan_rows<T, TI, 1, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
-        else if (w <= 512)  return launch_scan_rows<T, TI, 2, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
-        else if (w <= 1024) return launch_scan_rows<T, TI, 4, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
-        else if (w <= 2048) return launch_scan_rows<T, TI, 8, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
-        else                return launch_scan_rows<T, TI, 16, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+        switch ((w + 255) / 256) {
+            case 1: return launch_scan_rows<T, TI, 1, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 2: return launch_scan_rows<T, TI, 2, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 3: return launch_scan_rows<T, TI, 3, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 4: return launch_scan_rows<T, TI, 4, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 5: return launch_scan_rows<T, TI, 5, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 6: return launch_scan_rows<T, TI, 6, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 7: return launch_scan_rows<T, TI, 7, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            case 8: return launch_scan_rows<T, TI, 8, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+            default: return launch_scan_rows<T, TI, 16, 4>(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
+        }
     }
     return TiledScan<T, TI>::run(in, out, aux, planes, h, w, nb, R, reverse_order, stream);
 }

@@ -861,3 +861,25 @@ def test_integral_image_of_a_plane_per_workgroup(hip, switches, dtype, planes, h
     assert not got[:, :, 0].any() and not got[..., 0].any()
     # one rounding to float32, and that of double sums in another order
     assert (np.abs(got[:, :, 1:, 1:] - want) <= 2.0 ** -24 * np.abs(want) * 1.001 + 1e-12 * np.abs(want).max()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("planes,h,w", [
+    # bands: every number of waves, rows that end on, just behind and just before a wave's end, last lanes that
+    # share one, two and three columns, last bands of a single row
+    (2, 97, 257), (3, 66, 511), (2, 70, 513), (2, 65, 767), (1, 129, 769), (2, 64, 1022), (2, 67, 1027), (1, 100, 1281),
+    (2, 66, 1535), (1, 75, 1538), (2, 64, 1793), (1, 97, 2047), (1, 64, 2049), (1, 70, 4095), (2, 300, 1036), (1, 520, 604),
+    # a workgroup per plane, one band of at most 256 rows
+    (280, 11, 1025), (320, 9, 1000), (430, 10, 514), (640, 7, 301), (280, 257, 1284), (641, 5, 512)])
+def test_integral_image_in_bands(hip, switches, dtype, planes, h, w):
+    """The launches with and without a column-sum pass (BOXCONV_INTEGRAL_LOOKBACK=0), from aligned addresses and from
+    an odd element on, against a float64 cumulative sum."""
+    flat = torch.randn(planes * h * w + 1, generator=torch.Generator().manual_seed(h * w)).cuda().to(dtype)
+    switches("BOXCONV_INTEGRAL_LOOKBACK", "0")
+    for x in (flat[:-1].view(1, planes, h, w), flat[1:].view(1, planes, h, w)):
+        got = hip.integral_image(x)
+        want = x.double().cumsum(2).cumsum(3)
+        assert not got[:, :, 0].any() and not got[..., 0].any()
+        # one rounding to the output type, and that of double sums in another order
+        unit = 2.0 ** -24 if got.dtype == torch.float32 else 0.0
+        assert ((got[:, :, 1:, 1:].double() - want).abs() <= unit * 1.001 * want.abs() + 1e-12 * want.abs().max()).all()
