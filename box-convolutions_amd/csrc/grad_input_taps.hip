@@ -26,7 +26,7 @@
 // It replaces the column workspace, which is written whole and read twice (grad_input_cols_kernel),
 // by a second read of grad_output and snapshots of 1/4 or 1/8 of that size (two rows per group of 8 or 16
 // output rows) and one row per band. Both backward kernels together, 16 x 8 planes: 512 x 1024 x 2 346 ->
-// 266 us, 720 x 1280 357 -> 304 us; 32 x 4 planes of 128 x 256 x 4 44 -> 41 us (x 8 in bfloat16 79 -> 57); 128 x 2
+// 266 us, 720 x 1280 357 -> 304 us (270 with its sums in one round of workgroups); 32 x 4 planes of 128 x 256 x 4 44 -> 41 us (x 8 in bfloat16 79 -> 57); 128 x 2
 // planes of 1024 x 2048 1632 -> 1520 us. Not every launch gains: snapshots_pay (box_sampling.hip).
 // Bound (512 x 1024, 131 us): latency and issue at 6.6 resident waves per CU; the vector ALU issues a third
 // of the time, the LDS pipe is busy for 15 % of it with no bank conflicts; 578 MB are fetched for 537 MB of
