@@ -1047,7 +1047,7 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     int nb = static_cast<int>(std::min<int64_t>(wanted, std::max(1, h / min_rows)));
     // Where planes get cut anyway and the single-pass kernel covers the width, cut them into
     // bands of at most 32 rows, which that kernel holds in registers.
-    // Measured against the three launches: 0.6-0.95 of their time when all workgroups are on the
+    // Measured against the launches as they then were (see below): 0.6-0.95 of their time when all workgroups are on the
     // chip at once (they then read, hand over and write in step, so the bands above are never
     // late) or when there are several times more than fit (they fall out of step and reads overlap
     // writes); 1.05-1.3 in between, for rows that do not fill the workgroup exactly, and for
@@ -1058,15 +1058,15 @@ IntegralPlan plan_integral(int64_t planes, int h, int w, int64_t want) {
     // workgroups of five waves and more, of which only one would fit, get three per SIMD
     const int waves = std::max(1, (w + 255) / 256);
     const int64_t resident = 256 * (waves <= 4 ? 8 / waves : 12 / waves);
-    // (rows of a multiple of four columns: every lane holds four columns or none. Measured on
-    // 16 x 8 or 32 x 8 planes, single pass against two: 720 x 1280 43 against 59 us, 512 x 768 27
-    // against 44, 256 x 1536 26 against 37, 512 x 1000 40 against 50, 480 x 640 35 against 41;
-    // but 540 x 960, one workgroup in sixteen too many to be resident, 63 against 51, and
-    // 1080 x 1920, 34 bands per plane, 117 against 80.)
+    // (rows of a multiple of four columns: every lane holds four columns or none. Measured on 16 or 32 planes, the marker
+    // fill, which a training or inference forward has in its clip's launch, left out: single pass against two launches
+    // 512 x 1024 30 against 39 us, 512 x 768 26 against 32, 256 x 1536 25 against 35; even by now
+    // at 720 x 1280, 44 against 45, and 512 x 1000, 39 against 40, and behind at 480 x 640, 34 against 32, where it is ahead from
+    // 16-bit elements, 23 against 31; not resident 540 x 960, 63 against 42, and 1080 x 1920, 34 bands per plane, 114 against 81.)
     // Rows of other widths (kShiftedQuads), only where all workgroups are resident, which also bounds
-    // the workspace: 64 planes of 270 x 481 39 -> 25 us, 16 of 301 x 767 33 -> 20, 16 of 500 x 1001
+    // the workspace, against the two launches with element loads: 64 planes of 270 x 481 39 -> 25 us, 16 of 301 x 767 33 -> 20, 16 of 500 x 1001
     // 38 -> 27, 8 of 1000 x 2001 65 -> 41, 12 of 700 x 1401 57 -> 49; in bfloat16 35 -> 25, 27 -> 21, 34 -> 26,
-    // 56 -> 37, 50 -> 49 (28, 21, 27, 43 and 56 with element loads). Not below 3 << 19 pixels for images of 64 to
+    // 56 -> 37, 50 -> 49 (28, 21, 27, 43 and 56 with element loads); the two launches take 29, 25, 33, 48 and 42 by now. Not below 3 << 19 pixels for images of 64 to
     // 256 rows and up to 512 columns, which the two passes cut into bands of 16 rows (single pass
     // against two, alone and in a training forward, where the clip's launch also marks the hand-over
     // words: 6 planes of 64 x 505 in bfloat16 14.6 against 11.3 and 20.3 against 18.5 us, 4 of 144 x 402 in
