@@ -150,7 +150,8 @@ __global__ void __launch_bounds__(NT) forward_rows_kernel(SampleArgs<T> a, Forwa
 // column modulo four (tap_run). The planes hold V[1..w]; the places in front of them stay zero (V[0] =
 // 0 and what clamps to it), those behind hold V[w]. Rows that are no multiple of four columns (FIT): the last
 // lane takes the row's last four columns (RowLane) and stores those it shares with its neighbour, too: the
-// same values.
+// same values. Not where the residual is the output itself: the neighbour may be in another wave, and what
+// this lane stored early would be added a second time there.
 // The tail's residual: none, or loaded with the ordinary or the streaming cache policy.
 enum ResidualLoads { kNoResidual, kResidualCached, kResidualStreamed };
 // Without a residual nothing is loaded for it (loads of the output in its place, dropped, cost a read as
@@ -202,6 +203,7 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
         if (tl.channel_shift != nullptr) ch_shift = tl.channel_shift[k_par];
     }
     const bool relu = TAIL && tl.relu != 0;
+    const bool in_place = RESIDUAL != kNoResidual && FIT == kRowAny && tl.residual == tl.dst;
 
     if (tid < 2 * K * kQuadPad)
         vrow[tid / (K * kQuadPad)][tid / kQuadPad % K][tid % kQuadPad] = RowPair<T>{T(0), T(0)};
@@ -275,7 +277,14 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
             narrow(y0, z0.v[k]);
             narrow(y1, z1.v[k]);
         }
-        if (FIT == kRowFull || lane_in) {
+        if (in_place) {                              // (scalar)
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (ln.owns(k)) {
+                    tl.dst[row0 + cl + k] = z0.v[k];
+                    if (second) tl.dst[row1 + cl + k] = z1.v[k];
+                }
+        } else if (FIT == kRowFull || lane_in) {
             store_quad<ALIGNED>(tl.dst + row0 + cl, z0, a.stream_out != 0);
             if (second) store_quad<ALIGNED>(tl.dst + row1 + cl, z1, a.stream_out != 0);
         }

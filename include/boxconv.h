@@ -233,8 +233,9 @@ int boxconv_training_forward_half_f32(const void* input, int io_dtype, float* x_
  * point at elements of that type, [batch, in_planes*num_filters, h, w]. channel_scale and
  * channel_shift are float [in_planes*num_filters] (an eval-mode BatchNorm folds to
  * scale = gamma / sqrt(var + eps), shift = beta - mean * scale). residual, channel_scale and
- * channel_shift may each be NULL (no residual, scale 1, shift 0). There is no backward for
- * this entry point. */
+ * channel_shift may each be NULL (no residual, scale 1, shift 0). residual may be the output itself
+ * (the sum is then formed in place); in any other way the two must not overlap. There is no
+ * backward for this entry point. */
 int boxconv_forward_fused_f32(const float* input_integrated, const float* x_min,
                               const float* x_max, const float* y_min, const float* y_max,
                               void* output, int output_dtype, const void* residual,

@@ -460,3 +460,32 @@ def test_residual_at_any_offset(switches, dtype, h, w):
     assert hip.profile_collect()[1] == 1
     switches("BOXCONV_FWD_QUADS", "0")
     assert torch.equal(got, forward(aligned))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("h,w", [
+    # rows that are no multiple of four columns: a last wave with a single lane in use, whose neighbour is in another
+    # wave (257 to 259, 513, 770, 1025 columns), and with more; several rows in a wave; whole quads; one element per lane
+    (37, 257), (38, 258), (41, 259), (33, 513), (30, 770), (29, 1025), (36, 301), (70, 129), (33, 31), (24, 127), (40, 64),
+    (30, 256), (21, 512), (20, 2100)])
+def test_residual_in_the_memory_of_the_output(dtype, h, w):
+    """The C entry point adds a residual in place: every pixel is read and written by one lane. The result is that of
+    a residual elsewhere, bit for bit."""
+    from box_convolution import _native as hip
+    B, C, F = 2, 6, 3
+    gen = torch.Generator().manual_seed(h * w)
+    integ = hip.integral_image(torch.randn(B, C, h, w, generator=gen).cuda())
+    lo_x, lo_y = ((torch.rand(C, F, generator=gen) * 2 - 1.2) * n for n in (h, w))
+    boxes = [t.cuda() for t in (lo_x, lo_x + 2.2 + torch.rand(C, F, generator=gen) * h,
+                                lo_y, lo_y + 2.2 + torch.rand(C, F, generator=gen) * w)]
+    scale, shift = torch.rand(C * F, generator=gen).cuda(), torch.randn(C * F, generator=gen).cuda()
+    residual = torch.randn(B, C * F, h, w, generator=gen).cuda().to(dtype)
+    want = hip.box_convolution_forward_fused(integ, *boxes, True, True, dtype, scale, shift, residual, True)
+    lib = hip.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    for _ in range(5):
+        both = residual.clone()
+        assert lib.boxconv_forward_fused_f32(
+            integ.data_ptr(), *[b.data_ptr() for b in boxes], both.data_ptr(), hip._FUSED_OUTPUT[dtype], both.data_ptr(),
+            scale.data_ptr(), shift.data_ptr(), 1, B, C, F, h, w, 1, 1, stream) == 0
+        assert torch.equal(both, want)
