@@ -622,8 +622,8 @@ def training_forward(input, x_min, x_max, y_min, y_max, reparametrization_h, rep
     return integrated, output, real.unbind(0)
 
 
-KERNEL_NAMES = ("band_colsum", "band_prefix", "band_scan", "forward_rows", "forward_quads", "forward_narrow", "grad_output_stream",
-                "grad_input_cols", "grad_input_taps", "param_grad_finalize", "fill_zero", "fill_marker", "clip",
+KERNEL_NAMES = ("band_colsum", "band_prefix", "band_scan", "forward_rows", "forward_quads", "forward_narrow", "forward_narrow_unaligned",
+                "grad_output_stream", "grad_input_cols", "grad_input_taps", "param_grad_finalize", "fill_zero", "fill_marker", "clip",
                 "forward_gather", "grad_input_gather", "grad_params_gather", "int_row_prefix",
                 "int_col_prefix")
 

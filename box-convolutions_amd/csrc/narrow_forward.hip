@@ -170,12 +170,14 @@ hipError_t narrow_forward_launch(SampleArgs<float> a, ForwardTail<TO> tail, Dims
     }
     finish_args(a, planes_f * a.acc_slots);
     const dim3 grid(static_cast<unsigned>(a.per_xcd * kXcds));
-    const bool quads = d.w % 4 == 0;
+    // whole quads only from addresses that are aligned to them; else loads and stores that need elements to be (the same for odd rows)
+    const bool quads = d.w % 4 == 0 && quads_aligned(tail.dst, sizeof(TO), d.w) && quads_aligned(tail.residual, sizeof(TO), d.w);
+    const char* const name = d.w % 4 == 0 && !quads ? "forward_narrow_unaligned" : "forward_narrow";
 #define LAUNCH_NF_TAIL(L, EX, QUADS)                                                                                    \
     do {                                                                                                                \
-        if (!has_tail) BOXCONV_LAUNCH("forward_narrow", (narrow_forward_kernel<TO, L, EX, QUADS, false, false>), grid, dim3(64), 0, stream, a, tail); \
-        else if (tail.residual == nullptr) BOXCONV_LAUNCH("forward_narrow", (narrow_forward_kernel<TO, L, EX, QUADS, true, false>), grid, dim3(64), 0, stream, a, tail); \
-        else BOXCONV_LAUNCH("forward_narrow", (narrow_forward_kernel<TO, L, EX, QUADS, true, true>), grid, dim3(64), 0, stream, a, tail); \
+        if (!has_tail) BOXCONV_LAUNCH(name, (narrow_forward_kernel<TO, L, EX, QUADS, false, false>), grid, dim3(64), 0, stream, a, tail); \
+        else if (tail.residual == nullptr) BOXCONV_LAUNCH(name, (narrow_forward_kernel<TO, L, EX, QUADS, true, false>), grid, dim3(64), 0, stream, a, tail); \
+        else BOXCONV_LAUNCH(name, (narrow_forward_kernel<TO, L, EX, QUADS, true, true>), grid, dim3(64), 0, stream, a, tail); \
     } while (0)
 #define LAUNCH_NF(L)                                                                                                    \
     if (quads) { if (exact) LAUNCH_NF_TAIL(L, true, true); else LAUNCH_NF_TAIL(L, false, true); }                       \

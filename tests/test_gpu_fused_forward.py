@@ -462,6 +462,38 @@ def test_residual_at_any_offset(switches, dtype, h, w):
     assert torch.equal(got, forward(aligned))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("h,w", [(40, 28), (64, 64), (33, 128)])
+def test_narrow_rows_with_a_residual_at_any_offset(dtype, h, w):
+    """Rows of at most 128 columns in a multiple of four whose residual or (through the C entry point) output does not
+    start on four elements: accesses that need aligned elements only, the same result bit for bit."""
+    from box_convolution import _native as hip
+    B, C, F = 4, 16, 3
+    integ = hip.integral_image(torch.randn(B, C, h, w, device="cuda"))
+    lo = torch.full((C, F), -3.25, device="cuda")
+    residual = torch.randn(B, C * F, h, w, device="cuda").to(dtype)
+    lib = hip.load()
+
+    def at_odd_element(t):
+        return torch.empty(t.numel() + 1, device="cuda", dtype=dtype)[1:].view_as(t).copy_(t)
+
+    def forward(res, out, name):
+        hip.profile_arm(name)
+        assert lib.boxconv_forward_fused_f32(
+            integ.data_ptr(), lo.data_ptr(), (-lo).data_ptr(), lo.data_ptr(), (-lo).data_ptr(), out.data_ptr(),
+            hip._FUSED_OUTPUT[dtype], None if res is None else res.data_ptr(), None, None, 1, B, C, F, h, w, 1, 1,
+            torch.cuda.current_stream().cuda_stream) == 0
+        assert hip.profile_collect()[1] == 1
+        return out
+
+    for res in (residual, None):
+        want = forward(res, torch.empty_like(residual), "forward_narrow")
+        shifted = at_odd_element(residual)
+        if res is not None:
+            assert torch.equal(forward(shifted, torch.empty_like(residual), "forward_narrow_unaligned"), want)
+        assert torch.equal(forward(res, at_odd_element(residual), "forward_narrow_unaligned"), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("h,w", [
     # rows that are no multiple of four columns: a last wave with a single lane in use, whose neighbour is in another
