@@ -87,17 +87,20 @@ narrow_sums_kernel(SampleArgs<float> a) {
     const T* iplane = a.src + p * static_cast<int64_t>(h + 1) * (w + 1) + 1;
     const TG* gplane = reinterpret_cast<const TG*>(a.grad_out) + pf * static_cast<int64_t>(h) * w;
     const unsigned i_bytes = 4u * static_cast<unsigned>(w + 1), g_bytes = static_cast<unsigned>(sizeof(TG)) * static_cast<unsigned>(w);
-    auto load_i = [&](int r, T (&dst)[K]) {
-        load4_dword_aligned(at_bytes(iplane, row_offset(confine(r, h), i_bytes, 4u * ln.cl)), dst);
+    // The upper rows end at those of the plane's last output row, and so do the lower ones: a row behind it, of
+    // which bands past the plane have many, adds V times zero, and what only it would read may be infinite.
+    const int top_last = uniform(min(max(h - 1 + s.xlo, 0), h)), bottom_last = uniform(min(max(h + s.xhi, 0), h));
+    auto load_i = [&](int r, int last, T (&dst)[K]) {
+        load4_dword_aligned(at_bytes(iplane, row_offset(confine(r, last), i_bytes, 4u * ln.cl)), dst);
     };
     auto load_g = [&](int i, RawQuad<TG>& q) {
         q.template load<QUADS>(at_bytes(gplane, row_offset(min(i, h - 1), g_bytes, static_cast<unsigned>(sizeof(TG)) * ln.cl)));
     };
     auto load_window = [&](int i, T (&t0)[K], T (&t1)[K], T (&b1)[K], T (&b2)[K]) {
-        load_i(i + s.xlo, t0);
-        load_i(i + 1 + s.xlo, t1);
-        load_i(i + 1 + s.xhi, b1);
-        load_i(i + 2 + s.xhi, b2);
+        load_i(i + s.xlo, top_last, t0);
+        load_i(i + 1 + s.xlo, top_last, t1);
+        load_i(i + 1 + s.xhi, bottom_last, b1);
+        load_i(i + 2 + s.xhi, bottom_last, b2);
     };
     RawQuad<TG> r0, r1;
     load_g(i0, r0);
@@ -133,8 +136,8 @@ narrow_sums_kernel(SampleArgs<float> a) {
     double total[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     T colacc[K] = {T(0), T(0), T(0), T(0)};
     T ta[K], bc[K], t0[K], t1[K], b1[K], b2[K];
-    load_i(i0 + s.xlo - 1, ta);
-    load_i(i0 + s.xhi, bc);
+    load_i(i0 + s.xlo - 1, top_last, ta);
+    load_i(i0 + s.xhi, bottom_last, bc);
     load_window(i0, t0, t1, b1, b2);
 
     const int mask = (1 << a.snap_shift) - 1;

@@ -778,6 +778,48 @@ def test_narrow_rows_half(hip, switches, h, w, F, dtype):
         assert torch.equal(p, q)
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("h,w,F", [
+    # several rows side by side in a wave, bands past the plane among them; rows that are no multiple of four columns;
+    # rows of five waves
+    (33, 32, 2), (28, 28, 9), (17, 17, 3), (70, 60, 3), (45, 100, 2), (50, 127, 4), (41, 128, 2), (40, 129, 3), (36, 301, 2),
+    (34, 767, 2), (40, 1281, 2)])
+def test_infinities_and_nan_stay_where_they_act(hip, switches, h, w, F, bad):
+    """An input pixel that no box reaches has no effect on the parameter gradients, whatever its value; a value of
+    grad_output makes what depends on it infinite or NaN, and changes no bit of other planes' and other boxes' gradients."""
+    switches("BOXCONV_NARROW", "2")
+    switches("BOXCONV_GI_SNAPSHOTS", "2" if w > 128 else None)
+    switches("BOXCONV_STREAM_CONSEC", "3")
+    C = 3
+    gen = torch.Generator().manual_seed(h * w)
+    x = torch.randn(1, C, h, w, generator=gen)
+    g = torch.randn(1, C * F, h, w, generator=gen).cuda()
+    y_lo = -2.3 - 3 * torch.rand(C, F, generator=gen).cuda()
+
+    def backward(x, boxes, g):
+        return hip.box_convolution_backward(hip.integral_image(x.cuda()), *boxes, g, None, 1.0, 1.0, True, True,
+                                            True, True, True, True, True)
+    # boxes that end 2.6 rows and more above the image's last row for every output pixel
+    x_hi = -3.6 - torch.rand(C, F, generator=gen).cuda()
+    above = (x_hi - 2.2 - 3 * torch.rand(C, F, generator=gen).cuda(), x_hi, y_lo, -y_lo)
+    spoiled, clean = x.clone(), x.clone()
+    spoiled[..., -1, w // 3], clean[..., -1, :] = bad, 0.0
+    spoiled[..., -1, 1] = -bad
+    for a, b in zip(backward(spoiled, above, g)[1:], backward(clean, above, g)[1:]):
+        assert torch.equal(a, b)
+    # boxes around the pixel, far enough inside the image to be whole
+    boxes = (y_lo - 0.1, -y_lo, y_lo, 0.2 - y_lo)
+    i, j = h // 2, w // 2
+    spoiled = g.clone()
+    spoiled[0, 0, i, j] = bad
+    got, want = backward(x, boxes, spoiled), backward(x, boxes, g)
+    assert torch.equal(got[0][:, 1:], want[0][:, 1:])
+    assert not torch.isfinite(got[0][0, 0, i - 2:i + 3, j - 2:j + 3]).any()
+    for a, b in zip(got[1:], want[1:]):
+        assert not torch.isfinite(a[0, 0])
+        assert torch.equal(a.flatten()[1:], b.flatten()[1:])
+
+
 @pytest.mark.parametrize("snapshots,planes,F,h,w", [
     (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
     # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
