@@ -52,7 +52,7 @@ __device__ __forceinline__ A row_scan(A x, int l) {
 // SNAP: snapshots for narrow_input_kernel, else the parameter sums alone. QUADS: rows of a multiple of
 // four columns, aligned to four elements.
 template <class TG, int L, bool EXACT, bool QUADS, bool SNAP>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 4)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SNAP ? 3 : 4, 4)))
 narrow_sums_kernel(SampleArgs<float> a) {
     using T = float;
     using Lane = NarrowLane<L>;
@@ -215,14 +215,30 @@ narrow_sums_kernel(SampleArgs<float> a) {
             xw[0][threadIdx.x] = LastColumn{v0[K - 1], t0[K - 1] - ta[K - 1], b1[K - 1] - bc[K - 1], T(0)};
             xw[1][threadIdx.x] = LastColumn{v1[K - 1], t1[K - 1] - t0[K - 1], b2[K - 1] - b1[K - 1], T(0)};
             wave_lds_order();
+            // The row pair's share of a column goes to double at once (two products, as in the kernel for wider rows
+            // at one column per lane). finish_here: left alone the compiler holds all the sums back and spills.
+            auto add = [&](const T (&sum)[5]) {
+#pragma unroll
+                for (int n = 0; n < 5; ++n) {
+                    T part = sum[n];
+                    finish_here(part);
+                    total[n] += static_cast<double>(part);
+                    finish_here(total[n]);
+                }
+            };
+            {
+                const LastColumn x0 = xw[0][owner], x1 = xw[1][owner];
+                const RowPair<T> gmax = G[at_ymax], gmin = G[at_ymin];
+                const T sum[5] = {-(x0.dt * tl0 + x1.dt * tl1), x0.db * tl0 + x1.db * tl1, -(x0.v * gmin.r0 + x1.v * gmin.r1),
+                                  x0.v * gmax.r0 + x1.v * gmax.r1, x0.v * tl0 + x1.v * tl1};
+                add(sum);
+            }
             RowPair<T> R[K + 1], Lt[K + 1];
             read_taps(G, er, R);
             read_taps(G, el, Lt);
-            const LastColumn x0 = xw[0][owner], x1 = xw[1][owner];
-            const RowPair<T> gmax = G[at_ymax], gmin = G[at_ymin];
-            T sum[5] = {T(0), T(0), T(0), T(0), T(0)};
 #pragma unroll
             for (int k = 0; k < K; ++k) {
+                T sum[5] = {T(0), T(0), T(0), T(0), T(0)};
                 const RowPair<T> grA = R[k], gr = R[k + 1], gl = Lt[k], glA = Lt[k + 1];
                 const T dr0 = grA.r0 - gr.r0, dl0 = gl.r0 - glA.r0;
                 const T dr1 = grA.r1 - gr.r1, dl1 = gl.r1 - glA.r1;
@@ -242,16 +258,8 @@ narrow_sums_kernel(SampleArgs<float> a) {
                 sum[0] -= (t1[k] - t0[k]) * w1;
                 sum[3] += v1[k] * dr1;
                 sum[2] -= v1[k] * dl1;
+                add(sum);
             }
-            sum[4] += x0.v * tl0 + x1.v * tl1;
-            sum[1] += x0.db * tl0 + x1.db * tl1;
-            sum[0] -= x0.dt * tl0 + x1.dt * tl1;
-            sum[3] += x0.v * gmax.r0 + x1.v * gmax.r1;
-            sum[2] -= x0.v * gmin.r0 + x1.v * gmin.r1;
-#pragma unroll
-            for (int n = 0; n < 5; ++n) finish_here(sum[n]);
-#pragma unroll
-            for (int n = 0; n < 5; ++n) total[n] += static_cast<double>(sum[n]);
         }
         if (PREFETCH) {
             BOXCONV_PUBLISH_NARROW(FLIP ^ 1, lr + 2, m0, m1, tl0, tl1)

@@ -9,7 +9,8 @@ namespace boxconv {
 namespace {
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ void finish_here(float& v) { asm volatile("" : "+v"(v)); }
+template <class V>
+__device__ __forceinline__ void finish_here(V& v) { asm volatile("" : "+v"(v)); }
 
 // Row r confined to [0, last], and the byte offset of a row: one instruction each (the compiler makes two
 // of the first, and a product of four times the cost of the second; rows and their bytes are below 2^24).

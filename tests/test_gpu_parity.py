@@ -820,6 +820,27 @@ def test_infinities_and_nan_stay_where_they_act(hip, switches, h, w, F, bad):
         assert torch.equal(a.flatten()[1:], b.flatten()[1:])
 
 
+@pytest.mark.parametrize("need_input", [True, False])
+@pytest.mark.parametrize("h,w", [(40, 31), (33, 64), (50, 100), (64, 128)])
+def test_narrow_rows_add_few_products_in_float(hip, switches, h, w, need_input):
+    """Neighbouring columns whose contributions to a parameter gradient cancel, 2^26, 1, -2^26, 1, and again: no more than a
+    row pair's products of one column may meet in a float sum, where the ones would be lost."""
+    switches("BOXCONV_NARROW", "2")
+    x = torch.zeros(1, 2, h, w, device="cuda")
+    x[..., 0] = 1.0                                     # (the same V in every column)
+    g = torch.tensor([2.0 ** 26, 1.0, -2.0 ** 26, 1.0], device="cuda").repeat(w)[:w].expand(1, 2, h, w).contiguous()
+    if w % 4:
+        g[..., w // 4 * 4:] = 1.0
+    whole = torch.ones(2, 1, device="cuda")
+    boxes = (-2.5 * whole, 2.5 * whole, -3.0 * w * whole, 0.0 * whole)
+    got = hip.box_convolution_backward(hip.integral_image(x), *boxes, g, None, 1.0, 1.0, False, True, need_input,
+                                       True, True, True, True)
+    # the border row of output row i is i - 3 and i + 3: a sum of grad_output over the rows that have one
+    want = g[0, 0, 3:].double().sum().item()
+    assert torch.equal(got[1].double().cpu(), torch.full((2, 1), -want, dtype=torch.float64))
+    assert torch.equal(got[2].double().cpu(), torch.full((2, 1), want, dtype=torch.float64))
+
+
 @pytest.mark.parametrize("snapshots,planes,F,h,w", [
     (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
     # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
