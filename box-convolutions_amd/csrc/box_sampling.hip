@@ -117,6 +117,37 @@ hipError_t grad_params_begin(double* acc, int n_boxes, hipStream_t stream) {
     return hipGetLastError();
 }
 
+namespace {
+
+// Several bands side by side in a wave: rows per band (a power of two of at least a group, so that groups
+// of rows start with bands) for the least rounds of waves times row pairs of a band and what it takes to
+// start and end one, about three pairs. A launch is short of waves or, with bands that end
+// in the middle of a wave, wastes them: 671 x 37 planes of 72 x 107, the sums, bands of 16, 32 and 64
+// rows 247, 298 and 295 us; 512 x 4 of 64 x 128 22, 19 and 29. No more bands than a box's column
+// sums are quickly added up from (78 x 19 of 928 x 32, both kernels 156, 124 and 107).
+struct NarrowBands {
+    int lanes, R, nb;       // lanes == 0: none
+    double used;            // how much of what the waves hold are the plane's rows
+};
+NarrowBands narrow_bands(int64_t planes_f, int h, int w) {
+    NarrowBands b{};
+    const int lanes = w <= 32 ? 8 : w <= 64 ? 16 : 32, side = 64 / lanes;
+    double best = 0.0;
+    for (int R = 128; R >= 8; R /= 2) {
+        const int nb = (h + R - 1) / R, slots = (nb + side - 1) / side;
+        const double waves = static_cast<double>(planes_f) * slots, rounds = waves / (256 * 12);
+        const double cost = (rounds < 4 ? std::ceil(rounds) : rounds) * (std::min(R, h) / 2 + 3);
+        // (rows that the kernel with one row per wave takes, too: no more waves than that one may launch)
+        if (consecutive_rows(w) && planes_f * slots > std::max<int64_t>(2 * switches().stream_workgroups, planes_f)) break;
+        if (b.lanes > 0 && (cost >= best || nb > 40)) continue;
+        best = cost;
+        b = {lanes, R, nb, static_cast<double>(h) / (static_cast<double>(slots) * side * R)};
+    }
+    return b;
+}
+
+}  // namespace
+
 StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t elem_size, bool sums_only) {
     const int64_t planes_f = planes * F;
     StreamPlan sp{};
@@ -153,24 +184,8 @@ StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t e
     sp.nb = (h + sp.R - 1) / sp.R;
     sp.parts = (rc.nt == 1024 || stream_double_wide_split(w, elem_size)) ? 2 : 1;
     if (sp.usable && sums_only && elem_size == 4 && narrow_rows_pay(planes, F, h, w)) {
-        // Several bands side by side in a wave: rows per band (a power of two of at least a group, so that groups
-        // of rows start with bands) for the least rounds of waves times row pairs of a band and what it takes to
-        // start and end one, about three pairs. A launch is short of waves or, with bands that end
-        // in the middle of a wave, wastes them: 671 x 37 planes of 72 x 107, the sums, bands of 16, 32 and 64
-        // rows 247, 298 and 295 us; 512 x 4 of 64 x 128 22, 19 and 29. No more bands than a box's column
-        // sums are quickly added up from (78 x 19 of 928 x 32, both kernels 156, 124 and 107).
-        const int lanes = w <= 32 ? 8 : w <= 64 ? 16 : 32, side = 64 / lanes;
-        double best = 0.0;
-        for (int R = 128; R >= 8; R /= 2) {
-            const int nb = (h + R - 1) / R, slots = (nb + side - 1) / side;
-            const double waves = static_cast<double>(planes_f) * slots, rounds = waves / (256 * 12);
-            const double cost = (rounds < 4 ? std::ceil(rounds) : rounds) * (std::min(R, h) / 2 + 3);
-            // (rows that the kernel with one row per wave takes, too: no more waves than that one may launch)
-            if (consecutive_rows(w) && planes_f * slots > std::max<int64_t>(2 * switches().stream_workgroups, planes_f)) break;
-            if (sp.lanes > 0 && (cost >= best || nb > 40)) continue;
-            best = cost;
-            sp.lanes = lanes; sp.R = R; sp.nb = nb;
-        }
+        const NarrowBands b = narrow_bands(planes_f, h, w);
+        sp.lanes = b.lanes; sp.R = b.R; sp.nb = b.nb;
     }
     return sp;
 }
@@ -214,27 +229,28 @@ bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
 }  // namespace
 
 // Rows of at most 128 columns: the kernels that put several of them side by side in a wave (narrow_rows.hip)
-// against grad_output_stream_kernel and grad_input_cols_kernel, timed on 4300 shapes (1 to 2048 planes, 1 to
-// 40 filters, 16 to 1100 rows; float32 and bfloat16 with both gradients, float32 with the parameter sums alone):
-// 0.72, 0.75 and 0.69 of the time in the geometric mean by this rule, 0.59, 0.62 and 0.56 of the total, 33 of the
-// shapes more than 3 % slower (up to 1.15, one 1.40). Left to the others:
-//  * rows so few that bands of eight leave most of the wave empty (1629 x 2 planes of 12 x 20, the sums 12.5
-//    against 15.1 us; 1956 x 4 of 16 x 46 23.6 against 26.3);
-//  * fewer than 2^17 output pixels, where a step is bound by its launches, and few input pixels for the filters, which waves visit one after the other (25 planes of 24 x 16 with 40
-//    filters 22 against 32 us; 32 of 28 x 28 26 against 30);
+// against those for wider rows (column workspace, or snapshots where wide_snapshots_pay), timed on 31000 shapes (1 to 2048
+// planes, 1 to 40 filters, 16 to 1100 rows; float32 and bfloat16 with both gradients, float32 with the parameter sums
+// alone): by this rule 0.66, 0.68 and 0.63 of the time in the geometric mean, 44 of the 11800 shapes it takes (and none
+// of the 6500 with 96 to 124 columns in a multiple of four) more than 3 % slower, up to 1.14 (293 x 27 planes of
+// 37 x 45 77 -> 87 us). Left to the others:
+//  * fewer than 28 rows (nine shapes in ten of 16 to 23 rows 0.73 to 1.30 of the time, of 24 to 27 rows 0.64 to 1.12;
+//    51 x 23 planes of 20 x 36 20.7 against 26.8 us);
+//  * bands that leave nearly half of the waves' lanes without rows (0.61 to 1.09; 185 x 12 planes of 33 x 110, the
+//    sums, 22.7 against 27.7 us); for 96 to 124 columns in a multiple of four, of which the kernels for wider rows
+//    leave few lanes idle, a quarter (0.65 to 1.08; 554 x 3 of 135 x 96, the sums, 48.7 against 58.9);
+//  * fewer than 2^17 output pixels, where a step is bound by its launches, and few input pixels for the filters, which
+//    waves visit one after the other (25 planes of 24 x 16 with 40 filters 22 against 32 us; 32 of 28 x 28 26 against 30);
 //  * tall planes that give too few waves: their bands are cut short, and a box spans many of them (15 x 4
-//    planes of 1086 x 23 30 against 37 us);
-//  * 96 to 124 columns in multiples of four where the wide kernels keep the column workspace: what such
-//    launches return is fixed bit for bit.
+//    planes of 1086 x 23 30 against 37 us; the sums alone of 4 x 8 of 754 x 90 13.3 against 17.0).
 bool narrow_rows_pay(int64_t planes, int F, int h, int w) {
     const Switches& sw = switches();
     if (!sw.narrow_rows || !sw.input_from_snapshots || F < 1 || w < 16 || w > 128 || h < 8 || h >= (1 << 22)) return false;
     if (sw.narrow_any_size) return true;
     if (sw.snapshots_any_shape) return false;
-    if (consecutive_rows(w)) return wide_snapshots_pay(planes, F, h, w);
     const int64_t pixels = planes * h * w;
-    return h >= (w <= 32 ? 24 : w <= 64 ? 20 : 16) && pixels >= 1500 * static_cast<int64_t>(F) &&
-           pixels * F >= (h <= 400 ? 1 << 17 : 1 << 21);
+    return h >= 28 && pixels >= 3000 * static_cast<int64_t>(F) && pixels * F >= (h <= 400 ? 1 << 17 : 1 << 22) &&
+           narrow_bands(planes * F, h, w).used >= (w % 4 == 0 && w >= 96 && w < 128 ? 0.75 : 0.55);
 }
 
 // Output and integral images that no longer fit the memory-side cache together.

@@ -820,6 +820,32 @@ def test_infinities_and_nan_stay_where_they_act(hip, switches, h, w, F, bad):
         assert torch.equal(a.flatten()[1:], b.flatten()[1:])
 
 
+@pytest.mark.parametrize("narrow,planes,F,h,w", [
+    # from 28 rows on; bands that leave up to a quarter (96 to 124 columns in a multiple of four) or 0.45 of the
+    # lanes without rows; enough pixels for the filters, from 400 rows on more of them
+    (True, 64, 4, 28, 60), (False, 64, 4, 27, 60), (False, 51, 23, 20, 36), (False, 185, 12, 33, 110), (True, 185, 12, 64, 110),
+    (False, 554, 3, 135, 96), (True, 554, 3, 128, 96), (True, 512, 4, 64, 128), (False, 479, 2, 69, 100), (False, 32, 40, 28, 28),
+    (True, 64, 4, 500, 40), (False, 4, 8, 754, 90)])
+def test_narrow_rows_only_where_they_pay(hip, switches, narrow, planes, F, h, w):
+    """The launches for which several rows side by side in a wave are the slower way return what BOXCONV_NARROW=0
+    returns, bit for bit; the others what BOXCONV_NARROW=2 does, and that differs."""
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    g = torch.randn(1, planes * F, h, w, device="cuda")
+    boxes = [dev(b) for b in make_boxes(np.random.default_rng(h + w), planes, F, h, w, "inside")]
+
+    def backward(need_input):
+        return hip.box_convolution_backward(integ, *boxes, g, None, 1.0, 1.0, True, True, need_input, True, True, True, True)
+    for need_input in (True, False):
+        got = backward(need_input)
+        results = {}
+        for variant in ("0", "2"):
+            switches("BOXCONV_NARROW", variant)
+            results[variant] = [torch.equal(a, b) for a, b in zip(got, backward(need_input)) if a is not None]
+            switches("BOXCONV_NARROW", None)
+        assert all(results["2" if narrow else "0"])
+        assert not all(results["0" if narrow else "2"])
+
+
 @pytest.mark.parametrize("need_input", [True, False])
 @pytest.mark.parametrize("h,w", [(40, 31), (33, 64), (50, 100), (64, 128)])
 def test_narrow_rows_add_few_products_in_float(hip, switches, h, w, need_input):
