@@ -253,22 +253,30 @@ bool narrow_rows_pay(int64_t planes, int F, int h, int w) {
            narrow_bands(planes * F, h, w).used >= (w % 4 == 0 && w >= 96 && w < 128 ? 0.75 : 0.55);
 }
 
-// Output and integral images that no longer fit the memory-side cache together.
+// Output and integral images together; the memory-side cache holds 256 MB.
+static int64_t forward_bytes(int64_t planes, int F, int h, int w, size_t elem_size) {
+    return planes * (static_cast<int64_t>(F) * h * w * static_cast<int64_t>(elem_size) + static_cast<int64_t>(h + 1) * (w + 1) * 4);
+}
 static bool beyond_memory_side_cache(int64_t planes, int F, int h, int w, size_t elem_size) {
-    return planes * (static_cast<int64_t>(F) * h * w * static_cast<int64_t>(elem_size) + static_cast<int64_t>(h + 1) * (w + 1) * 4) >= (256ll << 20);
+    return forward_bytes(planes, F, h, w, elem_size) >= (256ll << 20);
 }
 
 // Forward of rows of at most 128 columns with several of them side by side in a wave (narrow_forward.hip)
 // against forward_rows_kernel, timed on 7400 shapes (float32; bfloat16 with and without the tail and a residual): 0.71,
 // 0.68 and 0.70 of the time in the geometric mean, 3 shapes more than 3 % slower. Not for float32 rows of more
-// than 32 columns without a tail that the memory-side cache does not hold (0.9 to 1.8), nor where
-// one_wave_quads_pay decides.
+// than 32 columns without a tail that the memory-side cache does not hold (0.9 to 1.8).
+// 96 to 124 columns in a multiple of four, against whichever of forward_rows_kernel and forward_quads_kernel
+// one_wave_quads_pay has them, on 13000 shapes: 16-bit outputs 0.75 to 0.79 (4 of 6800 more than 3 % slower);
+// float32 without a tail 0.78 (2 of 2044) up to 256 MB, 0.73 to 1.7 beyond; with a tail 0.80, with a residual,
+// too, 0.83 (24 of 1856, up to 1.15) up to 128 MB, 0.57 to 1.5 beyond.
 bool narrow_forward_pays(int64_t planes, int F, int h, int w, size_t elem_size, bool tail) {
     const Switches& sw = switches();
     if (!sw.forward_quads || !sw.narrow_rows || w < 16 || w > 128 || h >= (1 << 22)) return false;
     if (sw.narrow_any_size) return true;
-    if (sw.quads_any_size || (w >= 96 && w < 128 && w % 4 == 0)) return false;
-    return w <= 32 || elem_size == 2 || tail || !beyond_memory_side_cache(planes, F, h, w, elem_size);
+    if (sw.quads_any_size) return false;
+    if (w <= 32 || elem_size == 2) return true;
+    if (w >= 96 && w < 128 && w % 4 == 0 && tail) return forward_bytes(planes, F, h, w, elem_size) < (128ll << 20);
+    return tail || !beyond_memory_side_cache(planes, F, h, w, elem_size);
 }
 
 // forward_quads_kernel on rows that are no multiple of four columns, against forward_rows_kernel, timed on 9900

@@ -415,8 +415,10 @@ def test_large_residual(switches, dtype, planes, F, h, w):
 
 
 @pytest.mark.parametrize("quads,dtype,planes,h,w,tail", [
-    # 96 to 127 columns from 2^21 pixels on, never 128; 129 to 192 below 2^22; above with a residual
-    (False, torch.float32, 19, 59, 96, None), (True, torch.float32, 219, 100, 96, None),
+    # 96 to 127 columns from 2^21 pixels on where narrow_forward_kernel does not take them, never 128; 129 to 192 below
+    # 2^22; above with a residual
+    (False, torch.float32, 19, 59, 96, None), (False, torch.float32, 219, 100, 96, None),
+    (True, torch.float32, 160, 1000, 112, "relu"), (True, torch.float32, 310, 1000, 112, "residual"),
     (False, torch.float32, 219, 100, 128, None), (True, torch.float32, 100, 200, 192, None),
     (False, torch.float32, 150, 200, 160, None), (True, torch.float32, 150, 200, 160, "residual"),
     (False, torch.bfloat16, 150, 200, 160, None),
@@ -436,6 +438,25 @@ def test_consecutive_columns_only_where_they_pay(quads, dtype, planes, h, w, tai
     hip.profile_arm("forward_quads")
     hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, dtype, None, None, residual, tail == "relu")
     assert hip.profile_collect()[1] == quads
+
+
+@pytest.mark.parametrize("narrow,dtype,planes,h,w,tail", [
+    # up to 32 columns and 16-bit outputs always; float32 while output and integral images fit the memory-side cache,
+    # with a tail always; 96 to 124 columns in a multiple of four with a tail while they take less than half of it
+    (False, torch.float32, 64, 100, 15, None), (True, torch.float32, 2100, 600, 28, None), (True, torch.float32, 300, 100, 60, None),
+    (False, torch.float32, 1400, 400, 60, None), (True, torch.float32, 1400, 400, 60, "relu"), (True, torch.bfloat16, 1400, 400, 64, None),
+    (True, torch.float32, 219, 100, 96, None), (False, torch.float32, 310, 1000, 112, None), (True, torch.float32, 120, 1000, 112, "relu"),
+    (False, torch.float32, 160, 1000, 112, "relu"), (False, torch.float32, 160, 1000, 112, "residual"),
+    (True, torch.float32, 160, 1000, 111, "relu"), (True, torch.bfloat16, 500, 1000, 112, "residual"), (False, torch.bfloat16, 8, 100, 129, None)])
+def test_narrow_forward_only_where_it_pays(narrow, dtype, planes, h, w, tail):
+    """Rows of at most 128 columns: which launches take the kernel with several of them in a wave."""
+    from box_convolution import _native as hip
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    lo = torch.full((planes, 1), -3.25, device="cuda")
+    residual = torch.randn(1, planes, h, w, device="cuda").to(dtype) if tail == "residual" else None
+    hip.profile_arm("forward_narrow")
+    hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, dtype, None, None, residual, tail == "relu")
+    assert hip.profile_collect()[1] == narrow
 
 
 @pytest.mark.parametrize("dtype,h,w", [(torch.float32, 130, 252), (torch.bfloat16, 40, 512)])
