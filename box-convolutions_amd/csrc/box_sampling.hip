@@ -283,13 +283,16 @@ bool narrow_forward_pays(int64_t planes, int F, int h, int w, size_t elem_size, 
 // shapes: with a tail 0.83 of the time (0.56 to 1.09); without one, by this rule, 0.95 in float32 and 0.92 in bfloat16
 // (0.68 to 1.09). Left out: three or four columns per lane of one or two waves, which idle less in the other kernel
 // (129 to 191 columns 1.06 to 1.11 from 2^20 output pixels on, 257 to 384 columns 1.01 to 1.06 from 2^22), 769 to
-// 1024 columns below 2^20 (1.03), and wide float32 rows that the memory-side cache does not hold (1.03 to 1.2).
+// 1024 columns below 2^20 (1.03), and float32 rows of more than 256 columns that the memory-side cache does not hold:
+// 6500 of these 0.55 to 1.6, without a bound that parts them but the filters, which share a plane's integral rows; from
+// 16 of them and 100 rows on 0.78 (5 of 844 shapes more than 3 % slower, up to 1.11; 64 planes of 270 x 481 with 16
+// filters 189 -> 136 us), below that 1.04.
 bool odd_forward_quads_pay(int64_t planes, int F, int h, int w, size_t elem_size, bool tail) {
     const Switches& sw = switches();
     if (!sw.forward_quads || !sw.odd_forward_quads || w % 4 == 0 || w <= 128 || w > 2048) return false;
     if (sw.quads_any_size || tail) return true;
     const int64_t pixels = planes * F * h * w;
-    if (elem_size == 4 && beyond_memory_side_cache(planes, F, h, w, elem_size)) return w <= 256;
+    if (elem_size == 4 && beyond_memory_side_cache(planes, F, h, w, elem_size)) return w <= 256 || (F >= 16 && h >= 100);
     if (w < 192) return pixels < (1 << 20);
     if (w > 256 && w <= 384) return pixels < (1 << 22);
     return w <= 768 || w > 1024 || pixels >= (1 << 20);

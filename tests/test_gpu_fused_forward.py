@@ -459,6 +459,20 @@ def test_narrow_forward_only_where_it_pays(narrow, dtype, planes, h, w, tail):
     assert hip.profile_collect()[1] == narrow
 
 
+@pytest.mark.parametrize("quads,C,F,h,w", [
+    (True, 64, 16, 270, 481), (False, 64, 15, 270, 481), (True, 190, 16, 100, 301), (False, 200, 16, 99, 301),
+    (True, 300, 4, 350, 255), (True, 16, 4, 270, 481)])
+def test_large_odd_forward_by_filters(quads, C, F, h, w):
+    """float32 rows of more than 256 columns that the memory-side cache does not hold: four consecutive columns per
+    lane where many filters read the same integral rows."""
+    from box_convolution import _native as hip
+    integ = hip.integral_image(torch.randn(1, C, h, w, device="cuda"))
+    lo = torch.full((C, F), -3.25, device="cuda")
+    hip.profile_arm("forward_quads")
+    hip.box_convolution_forward_fused(integ, lo, -lo, lo, -lo, True, True, torch.float32, None, None, None, False)
+    assert hip.profile_collect()[1] == quads
+
+
 @pytest.mark.parametrize("dtype,h,w", [(torch.float32, 130, 252), (torch.bfloat16, 40, 512)])
 def test_residual_at_any_offset(switches, dtype, h, w):
     """A residual that does not start on four elements takes the kernel with wave-strided columns and
