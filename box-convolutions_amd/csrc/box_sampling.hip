@@ -209,10 +209,11 @@ namespace {
 // grad_output_stream_kernel (0.70 to 0.85 of its time from 2^24 output pixels on, 0.88 to 1.0 below); in addition
 //  * fewer than 40 rows (487 x 4 planes of 33 x 151 47 against 56 us, 90 x 8 of 34 x 506 46 against 54), or
 //    up to 192 columns and fewer than 2^24 output pixels (5 x 4 of 1055 x 171 45 against 51), are up to 1.2;
-//  * three waves whose last one has a single lane in use keep the workspace (16 x 8 planes of
-//    512 x 514 128 us that way, 115 by snapshots, 162 before this kernel took such rows: what a launch of
-//    that size returns is fixed bit for bit). Of more waves that costs less than the workspace does (16 x 8 planes
-//    of 512 x 1025 321 -> 183 us, of 720 x 1281 466 -> 291).
+//  * three waves whose last one has a single lane in use (513 to 515 columns, 1754 shapes) against the workspace, written
+//    by the same kernel: 0.95 of the time below 2^22 output pixels, 0.97 (up to 1.13, one shape in four more than 3 %
+//    slower: 53 x 10 planes of 55 x 514 68 against 77 us) from there to 2^25, 0.90 above (16 x 8 of 512 x 514 130 -> 114 us).
+//    Of more waves the lane costs less than the workspace does (16 x 8 planes of 512 x 1025 321 -> 183 us, of
+//    720 x 1281 466 -> 291).
 bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
     if (!consecutive_rows(w)) return false;
     if (switches().snapshots_any_shape) return true;
@@ -221,7 +222,8 @@ bool wide_snapshots_pay(int64_t planes, int F, int h, int w) {
     // resident: three waves per SIMD, ten workgroups of one wave by their LDS. Of two workgroups of five or
     // six waves on a CU the second slows the first by as much as it brings: they count as two rounds
     const int waves = consecutive_threads(w) / 64;
-    if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) || (waves == 3 && (w + 3) / 4 % 64 == 1))) return false;
+    if (w % 4 != 0 && (h < 40 || (w <= 192 && pixels * F < (1 << 24)) ||
+                       (waves == 3 && (w + 3) / 4 % 64 == 1 && pixels * F >= (1 << 22) && pixels * F < (1 << 25)))) return false;
     const int64_t workgroups = planes * ((h + 7) / 8), resident = 256 * (waves == 1 ? 10 : 12 / waves);
     return workgroups <= (waves > 4 ? 256 : resident) || workgroups * F >= 4 * resident;
 }

@@ -871,7 +871,9 @@ def test_narrow_rows_add_few_products_in_float(hip, switches, h, w, need_input):
     (True, 128, 4, 128, 256), (True, 32, 8, 128, 512), (True, 16, 1, 256, 512), (True, 2, 2, 512, 1024),
     # few input pixels for the filters, fewer than 24 rows, a second round with hardly anything in it
     (False, 8, 40, 17, 100), (False, 1, 8, 96, 256), (False, 16, 8, 200, 252), (False, 2, 1, 64, 1024),
-    (False, 86, 8, 17, 1212), (False, 15, 1, 552, 1124), (False, 479, 2, 69, 100), (False, 16, 8, 512, 514)])
+    (False, 86, 8, 17, 1212), (False, 15, 1, 552, 1124), (False, 479, 2, 69, 100),
+    # a third wave with a single lane in use, from 2^22 to 2^25 output pixels
+    (False, 53, 10, 55, 514), (True, 16, 8, 512, 514), (True, 6, 2, 500, 513)])
 def test_snapshots_only_where_they_pay(hip, switches, snapshots, planes, F, h, w):
     """The launches for which snapshots are the slower way keep the column workspace, and then
     return what BOXCONV_GI_SNAPSHOTS=0 returns, bit for bit."""
