@@ -663,13 +663,17 @@ band_scan_lookback_kernel(const TI* __restrict__ in, float* __restrict__ out, do
 // (rows of at most 128 / 64 columns would otherwise leave half / three quarters of every wave idle).
 // VEC: rows of a multiple of four columns from an aligned address. Otherwise the last lane takes the
 // row's last four columns (loads of four elements may start anywhere) and drops those that the lane
-// in front of it holds.
-// TALL: planes of more rows than the workgroup holds at a time. It goes down the plane in chunks of
+// in front of it holds. Float rows of one wave are instead read and written through descriptors of their size
+// (ROW_BOUNDS), which give zeros behind a row and drop what is stored there: the selects and the last lane's own stores
+// cost a chain of 8 to 24 rows 1.04 to 1.25 of the time (16 planes of 135 x 131 8.1 -> 10.1 us, 512 9.6 -> 11.0; from 16-bit
+// elements, which descriptors would read two bytes at a time, the loads of four save more: 0.87 to 0.93).
+// R: rows per band, known at compile time (a row that may or may not be one of the band's costs selects or branches: with them 16
+// planes of 192 x 256 take 9.8 us instead of 9.0). TALL: planes of more rows than the workgroup holds at a time. It goes down the plane in chunks of
 // that many rows; a row's registers take the next chunk's row as soon as they are scanned out.
 // Measured against the kernels before it (two launches for the tall planes; for the others one row per wave or
 // rows of a multiple of four columns only), float32: 578 planes of 833 x 23 334 -> 70 us, 224 of 296 x 80 57 -> 13,
 // 384 of 360 x 224 117 -> 60, 671 of 72 x 107 18 -> 14, 128 of 135 x 240 20 -> 12 (16-bit elements and rows that
-// do not exist are now widened and dropped after all loads are under way), but 128 of 135 x 241 11.8 -> 13.0.
+// do not exist are now widened and dropped after all loads are under way).
 // Bound by the chain load, sums, scan of a chunk where planes are few, else by memory.
 constexpr int kPlaneWaves = 8;        // waves per workgroup at most
 constexpr int kPlaneRows = 24;        // rows per band at most (registers: 4 x 24 floats per lane without spilling)
@@ -706,12 +710,13 @@ __device__ __forceinline__ double segment_inclusive_scan(double x) {
     return x;
 }
 
-template <class TI, int RMAX, int L, bool VEC, bool TALL>
+template <class TI, int R, int L, bool VEC, bool TALL>
 __global__ void __launch_bounds__(kPlaneWaves * 64)
-plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int w, int R, int64_t planes,
+plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int w, int64_t planes,
                   int reverse, ClipArgs<float> clip, int clip_blocks) {
     using T = float;
     constexpr int RB = 4, S = 64 / L;
+    constexpr bool ROW_BOUNDS = !VEC && S == 1 && std::is_same<TI, float>::value;
     __shared__ double sums[TALL ? 2 : 1][kPlaneWaves * S * 4 * L];      // [band][4][L]
 
     // a clip job on the side (its first clip_blocks workgroups): what a training-mode forward does
@@ -732,26 +737,30 @@ plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int
     const int bands = static_cast<int>(blockDim.x >> 6) * S;
     const int64_t W1 = static_cast<int64_t>(w) + 1;
     const bool lane_in = 4 * l < w;
-    const int c0 = VEC ? 4 * l : min(4 * l, w - 4);
-    const int twice = VEC || !lane_in ? 0 : 4 * l - c0;      // columns that the lane in front holds
+    const int c0 = VEC || ROW_BOUNDS ? 4 * l : min(4 * l, w - 4);
+    const int twice = VEC || ROW_BOUNDS || !lane_in ? 0 : 4 * l - c0;      // columns that the lane in front holds
     const int rest = -w & 3;
     const unsigned lane_col = lane_in ? static_cast<unsigned>(c0) : 0u;
 
     const TI* src = in + p * static_cast<int64_t>(h) * w;
     T* dst = out + p * static_cast<int64_t>(h + 1) * W1;
-    const Rows<T, true> orows(dst, W1, w + 1, h + 1);
+    const Rows<const TI, false> irows(src, w, w, h);
+    const Rows<T, !ROW_BOUNDS> orows(dst, W1, w + 1, h + 1);
     const RowRef oplane = orows.row(0);                      // the plane as one buffer; rows by offset
     const int out_off = (c0 + 1) * static_cast<int>(sizeof(T));
 
-    // (clamped addresses; values of rows and lanes that do not exist are dropped when they are used, and
-    // 16-bit elements widened then: either of them at the load would make the wave wait for it there)
-    Vec4<TI> raw[RMAX];
+    // (clamped addresses; 16-bit elements are widened when they are used: at the load that would make the wave wait for it there)
+    Vec4<TI> raw[R];
     auto load = [&](int row, Vec4<TI>& q) {
-        const TI* at = src + static_cast<int64_t>(min(row, h - 1)) * w;
-        q = load_raw_quad<VEC>(at + lane_col);
+        if constexpr (ROW_BOUNDS) {
+            buffer_load_run_as<kCacheStream, TI>(q.v, irows.row(min(row, h - 1), row < h), 4 * l * static_cast<int>(sizeof(TI)));
+        } else {
+            const TI* at = src + static_cast<int64_t>(min(row, h - 1)) * w;
+            q = load_raw_quad<VEC>(at + lane_col);
+        }
     };
 #pragma unroll
-    for (int r = 0; r < RMAX; ++r) load(band * R + r, raw[r]);
+    for (int r = 0; r < R; ++r) load(band * R + r, raw[r]);
 
     if (tid < 64)
         for (int c = tid; c <= w; c += 64) dst[c] = T(0);
@@ -764,16 +773,16 @@ plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int
         const int r1 = min(h, r0 + R);
         const bool more = TALL && base + chunk < h;
         double own[4] = {0.0, 0.0, 0.0, 0.0};
-        T x[RMAX][4];
+        T x[R][4];
+        // (lanes behind a row and rows behind the plane keep what they loaded: it reaches only lanes and rows
+        // further behind, and nothing of either is stored)
 #pragma unroll
-        for (int r = 0; r < RMAX; ++r) {
-            const bool exists = r < R && r0 + r < r1 && lane_in;
+        for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                x[r][v] = !exists || (!VEC && v < 3 && v < twice) ? T(0) : widen(raw[r].v[v]);
+                x[r][v] = !VEC && v < 3 && v < twice ? T(0) : widen(raw[r].v[v]);
                 own[v] += static_cast<double>(x[r][v]);
             }
-        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) sums[flip][(band * 4 + v) * L + l] = own[v];
         __syncthreads();
@@ -792,8 +801,7 @@ plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int
                 for (int v = 0; v < 4; ++v) above[v] += sums[flip][(b * 4 + v) * L + l];
 
 #pragma unroll
-        for (int bi = 0; bi < RMAX / RB; ++bi) {
-            if (bi * RB >= R) break;
+        for (int bi = 0; bi < R / RB; ++bi) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const int r = bi * RB + rb, row = r0 + r;
@@ -812,7 +820,9 @@ plane_scan_kernel(const TI* __restrict__ in, float* __restrict__ out, int h, int
                 // drops the stores to one that does not exist; else by the lane's offset)
                 const RowRef orow = S == 1 ? orows.row(min(row + 1, h), row < r1) : oplane;
                 const int off = (S == 1 ? 0 : static_cast<int>((static_cast<int64_t>(row + 1) * W1) * sizeof(T))) + out_off;
-                if (S == 1 || row < r1) {
+                if constexpr (ROW_BOUNDS) {
+                    buffer_store_run<kCacheDefault, false>(res, orow, off, (w + 1) * static_cast<int>(sizeof(T)));
+                } else if (S == 1 || row < r1) {
                     if (lane_in && (VEC || twice == 0)) buffer_store_run<kCacheDefault, true>(res, orow, off, 0);
                     if (!VEC && twice > 0) {                  // (rest: the same number, scalar: one store)
                         if (rest == 1) buffer_store_wide<kCacheDefault>({res[1], res[2], res[3]}, orow, off + 4);
@@ -957,8 +967,12 @@ hipError_t launch_plane_scan(const TI* in, float* out, int64_t planes, int h, in
     const ClipArgs<float> clip = clip_job != nullptr ? *clip_job : ClipArgs<float>{};
     const int rev = reverse ? 1 : 0;
     const bool vec = aligned_for_vec4(in, w);
-    // lanes per row: rows of at most 128 / 64 columns share a wave with one / three more bands
-    const int L = plane_row_lanes(w);
+    // lanes per row: rows of at most 128 / 64 columns share a wave with one / three more bands. But not odd float rows of
+    // planes so low and so few that the chip holds a wave per band anyway, which then are the faster ones (ROW_BOUNDS; side by
+    // side 16 to 512 planes of 16 to 40 rows 1.04 to 1.19 of the time, 64 of 28 x 127 3.9 -> 4.5 us; up to 48 rows 0.97 to
+    // 1.04, 2048 waves 0.59 to 1.07)
+    const bool few = !vec && std::is_same<TI, float>::value && h <= 48 && planes * ((h + 7) / 8) <= 1536;
+    const int L = few ? 64 : plane_row_lanes(w);
     const int S = 64 / L;
     const bool tall = h > kPlaneMaxRows * S;
     const int most = kPlaneTallRows * kPlaneWaves * S, chunks = tall ? (h + most - 1) / most : 1;
@@ -967,19 +981,26 @@ hipError_t launch_plane_scan(const TI* in, float* out, int64_t planes, int h, in
     const int waves = (nb + S - 1) / S;
     const int clip_blocks = (clip.n + waves * 64 - 1) / (waves * 64);
     const dim3 grid(static_cast<unsigned>(planes + clip_blocks)), block(waves * 64);
-#define LAUNCH_PLANE_L(RMAX, L_, TALL)                                                                    \
-    if (vec) BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, L_, true, TALL>), grid, block, 0, stream, in, out, \
-                            h, w, R, planes, rev, clip, clip_blocks);                                     \
-    else     BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, RMAX, L_, false, TALL>), grid, block, 0, stream, in, out, \
-                            h, w, R, planes, rev, clip, clip_blocks)
-#define LAUNCH_PLANE(RMAX, TALL)                                                                          \
-    if (L == 16)      { LAUNCH_PLANE_L(RMAX, 16, TALL); }                                                 \
-    else if (L == 32) { LAUNCH_PLANE_L(RMAX, 32, TALL); }                                                 \
-    else              { LAUNCH_PLANE_L(RMAX, 64, TALL); }
-    if (tall)          { LAUNCH_PLANE(kPlaneTallRows, true) }
-    else if (R <= 8)   { LAUNCH_PLANE(8, false) }
-    else if (R <= 16)  { LAUNCH_PLANE(16, false) }
-    else               { LAUNCH_PLANE(kPlaneRows, false) }
+#define LAUNCH_PLANE_L(R_, L_, TALL)                                                                      \
+    if (vec) BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, R_, L_, true, TALL>), grid, block, 0, stream, in, out, \
+                            h, w, planes, rev, clip, clip_blocks);                                        \
+    else     BOXCONV_LAUNCH("band_scan", (plane_scan_kernel<TI, R_, L_, false, TALL>), grid, block, 0, stream, in, out, \
+                            h, w, planes, rev, clip, clip_blocks)
+#define LAUNCH_PLANE(R_, TALL)                                                                            \
+    case R_:                                                                                              \
+        if (L == 16)      { LAUNCH_PLANE_L(R_, 16, TALL); }                                               \
+        else if (L == 32) { LAUNCH_PLANE_L(R_, 32, TALL); }                                               \
+        else              { LAUNCH_PLANE_L(R_, 64, TALL); }                                               \
+        break;
+    static_assert(kPlaneRows == 24 && kPlaneTallRows == 16, "the bands below");
+    if (tall) {
+        switch (R) { LAUNCH_PLANE(12, true) LAUNCH_PLANE(16, true) default: return hipErrorInvalidValue; }
+    } else {
+        switch (R) {
+            LAUNCH_PLANE(8, false) LAUNCH_PLANE(12, false) LAUNCH_PLANE(16, false) LAUNCH_PLANE(20, false) LAUNCH_PLANE(24, false)
+            default: return hipErrorInvalidValue;
+        }
+    }
 #undef LAUNCH_PLANE
 #undef LAUNCH_PLANE_L
     return hipGetLastError();

@@ -935,7 +935,9 @@ def test_integral_image_switch_one_is_the_default(hip, switches):
     (2, 50, 4), (2, 33, 7), (3, 29, 17), (2, 191, 62), (3, 130, 66), (2, 100, 127), (1, 192, 129), (2, 135, 241), (2, 40, 255),
     # taller than the workgroup holds at a time: one more row, several chunks, rows of the last chunk missing
     (2, 769, 33), (3, 1000, 64), (2, 850, 19), (2, 385, 127), (3, 512, 128), (130, 530, 100), (33, 193, 129), (40, 300, 256),
-    (128, 470, 203)])
+    (128, 470, 203),
+    # 8 to 24 rows per band and wave; low float planes with a wave per row, and with several rows in a wave: more rows, more planes
+    (2, 65, 140), (2, 100, 131), (3, 160, 202), (2, 190, 40), (3, 40, 61), (200, 48, 60), (3, 49, 99), (257, 48, 99)])
 def test_integral_image_of_a_plane_per_workgroup(hip, switches, dtype, planes, h, w):
     """Planes of at most 256 columns in one launch, against the two passes on the same planes, which add the
     double sums in another order, and against a float64 cumulative sum."""
@@ -952,6 +954,22 @@ def test_integral_image_of_a_plane_per_workgroup(hip, switches, dtype, planes, h
     assert not got[:, :, 0].any() and not got[..., 0].any()
     # one rounding to float32, and that of double sums in another order
     assert (np.abs(got[:, :, 1:, 1:] - want) <= 2.0 ** -24 * np.abs(want) * 1.001 + 1e-12 * np.abs(want).max()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("planes,h,w", [(3, 28, 28), (2, 61, 51), (2, 100, 96), (3, 33, 130), (2, 190, 241), (2, 100, 256), (128, 470, 203)])
+def test_integral_image_of_infinities_and_nan(hip, dtype, planes, h, w):
+    """Lanes behind a row and bands behind the plane load pixels of the plane: an infinite one in its first column and last
+    row, a NaN in its last column, reach the entries that they are part of and no others."""
+    x = torch.randn(planes, h, w, device="cuda").to(dtype)
+    clean = hip.integral_image(x)
+    for i, j, bad in ((h - 1, 0, float("inf")), (h // 2, 0, float("inf")), (h // 2, w - 1, float("nan"))):
+        y = x.clone()
+        y[1, i, j] = bad
+        got = hip.integral_image(y)
+        assert not got[1, i + 1:, j + 1:].isfinite().any()
+        got[1, i + 1:, j + 1:] = clean[1, i + 1:, j + 1:]
+        assert torch.equal(got, clean)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64])
