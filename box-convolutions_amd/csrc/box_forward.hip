@@ -159,9 +159,11 @@ enum ResidualLoads { kNoResidual, kResidualCached, kResidualStreamed };
 // bfloat16, output not in any cache, 42 -> 26). With one, the rows of the next pair are requested
 // with its integral rows: workgroups of few waves otherwise wait for memory right before the barrier
 // (residual not in any cache, 46 planes of 398 x 140 in float32 12.1 -> 10.0 us, 128 x 4 of 135 x 240
-// in bfloat16 27.7 -> 26.3); with two waves, and from five on, the registers cost more than that brings. Its cache policy: see forward_launch_any.
+// in bfloat16 27.7 -> 26.3); with two waves, and from five on, the registers cost more than that brings. From five on they have to
+// fit six waves per SIMD: at five, which three registers more are enough for, 46 x 18 planes of 64 x 1164 in bfloat16 take 73.8 us instead
+// of 67.4, 1 x 20 of 326 x 1608 17.1 instead of 14.4. Its cache policy: see forward_launch_any.
 template <class TO, int NT, bool EXACT, int FIT, bool TAIL, int RESIDUAL>
-__global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, ForwardTail<TO> tl) {
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(RESIDUAL != kNoResidual && NT > 256 && FIT != kRowAny ? 6 : 1))) forward_quads_kernel(SampleArgs<float> a, ForwardTail<TO> tl) {
     using T = float;
     constexpr int K = 4, PLANE = quad_plane(NT), WAVES = NT / 64;
     constexpr bool EARLY = RESIDUAL != kNoResidual && WAVES <= 4 && WAVES != 2;   // residual rows a pair ahead
@@ -215,19 +217,22 @@ __global__ void __launch_bounds__(NT) forward_quads_kernel(SampleArgs<float> a, 
     const int i1 = min(h, i0 + a.R);
     T ta[K], bc[K];                       // I[t(i-1)], I[b(i)]
     T t0[K], t1[K], b1[K], b2[K];         // I[t(i)], I[t(i+1)], I[b(i+1)], I[b(i+2)]
-    load_i(i0 + s.xlo - 1, ta);
-    load_i(i0 + s.xhi, bc);
-    load_i(i0 + s.xlo, t0);
-    load_i(i0 + 1 + s.xlo, t1);
-    load_i(i0 + 1 + s.xhi, b1);
-    load_i(i0 + 2 + s.xhi, b2);
     auto load_residual = [&](int i, Quad<TO>& q0, Quad<TO>& q1) {
         const int64_t row = out0 + static_cast<int64_t>(i) * w;
         q0 = load_quad<RESIDUAL == kResidualStreamed, ALIGNED>(tl.residual + row + cl);
         q1 = load_quad<RESIDUAL == kResidualStreamed, ALIGNED>(tl.residual + (i + 1 < i1 ? row + w : row) + cl);
     };
     Quad<TO> res0{}, res1{};
-    if (EARLY) load_residual(i0, res0, res1);
+    if (EARLY) {                          // in front of the integral rows: they mostly come from the L2, the residual from memory
+        load_residual(i0, res0, res1);    // (behind them 256 x 4 planes of 128 x 256 in bfloat16 41.2 -> 41.6 us)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    load_i(i0 + s.xlo - 1, ta);
+    load_i(i0 + s.xhi, bc);
+    load_i(i0 + s.xlo, t0);
+    load_i(i0 + 1 + s.xlo, t1);
+    load_i(i0 + 1 + s.xhi, b1);
+    load_i(i0 + 2 + s.xhi, b2);
 
     auto row_pair = [&](int i, auto prefetch_tag, auto flip_tag) {
         constexpr bool PREFETCH = decltype(prefetch_tag)::value;
