@@ -171,7 +171,8 @@ StreamPlan plan_grad_output_stream(int64_t planes, int F, int h, int w, size_t e
     // 720 x 1280 313 -> 270 / 151 -> 118 us, 8 x 8 of 900 x 1792 260 -> 223 / 114 -> 100, 32 x 4 of 400 x 1200
     // 195 -> 172 / 89 -> 68; at 0.78 of it 0.94 to 1.02 of the time, and one band per plane, which cannot be cut
     // to fit, 1.0 to 1.24. Four waves are worse off (16 x 8 of 512 x 1024 265 -> 287), as are eight
-    // (1024 x 2048 1455 -> 1615).
+    // (1024 x 2048 1455 -> 1615). Bands get up to h / 2 rows long by this; what the snapshots' float column sums would lose over
+    // so many rows, kSumRows (box_sampling_impl.hpp) keeps.
     const int waves = consecutive_threads(w) / 64;
     if (sums_only && elem_size == 4 && consecutive_rows(w) && waves >= 5 && waves <= 7) {
         const int64_t one_round = switches().stream_workgroups / 4;

@@ -940,6 +940,10 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     constexpr int WAVES = NT / 64;
     constexpr bool MERGED = !SCAN || NT <= 256;
     static_assert(MERGED || !SNAP, "the running sums are taken where the merged pass publishes its rows");
+    // Five to seven waves, whose bands may have any number of rows (plan_grad_output_stream): the float column sums
+    // behind the snapshots are added to ones in double every so many rows, since over a long band they would lose
+    // bits (180 rows at 720 x 1280, 46 to 64 in bands of other widths).
+    constexpr int kSumRows = SNAP && NT > 256 && NT < 512 ? 32 : 0;
     struct alignas(16) WaveSums { T tot0, tot1, tail0, tail1; };
     struct alignas(16) LastColumn { T v, dt, db, unused; };      // V, DT, DB at column w
     __shared__ __align__(16) RowPair<T> grow[2][K][PLANE];
@@ -947,6 +951,7 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     __shared__ WaveSums wsum[2][WAVES];
     __shared__ LastColumn xw[2][2];
     __shared__ double red[5 * WAVES];
+    __shared__ double above[kSumRows > 0 ? K * NT : 1];          // (each lane's own)
 
     const unsigned vid = xcd_contiguous_id(a.per_xcd);
     if (vid >= a.total) return;                      // whole workgroup leaves together
@@ -1022,8 +1027,12 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     const int snap_lo = __builtin_amdgcn_readfirstlane(sm.xlo), snap_hi = __builtin_amdgcn_readfirstlane(sm.xhi);
     // the sum of the band's rows above integral row r, where grad_input_taps_kernel will want it
     auto keep_snapshot = [&](int r, const T (&sum)[K]) {
-        const Quad<T> q{{sum[0], sum[1], sum[2], sum[3]}};
         const int mask = (1 << a.snap_shift) - 1, ut = r - snap_lo, ub = r - snap_hi;
+        if (kSumRows > 0 && (ut & mask) != 0 && (ub & mask) != 0 && r != i1) return;
+        Quad<T> q{{sum[0], sum[1], sum[2], sum[3]}};
+        if (kSumRows > 0)
+#pragma unroll
+            for (int k = 0; k < K; ++k) q.v[k] = static_cast<T>(above[k * NT + tid] + static_cast<double>(sum[k]));
         if ((ut & mask) == 0 && ut >= 0 && (ut >> a.snap_shift) < a.snap_groups)
             store_row_quad<FIT != kRowAny>(at_bytes(snap + static_cast<int64_t>(ut >> a.snap_shift) * spitch, 4u * cl), q);
         if ((ub & mask) == 0 && ub >= 0 && (ub >> a.snap_shift) < a.snap_groups)
@@ -1062,7 +1071,10 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
     double total[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     T colacc[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) colacc[k] = T(0);
+    for (int k = 0; k < K; ++k) {
+        colacc[k] = T(0);
+        if (kSumRows > 0) above[k * NT + tid] = 0.0;
+    }
 
     T ta[K], bc[K], t0[K], t1[K], b1[K], b2[K];
     load_i(clampi(i0 + s.xlo - 1, 0, h), ta);
@@ -1111,6 +1123,12 @@ grad_output_stream_consec_kernel(SampleArgs<float> a) {
             for (int k = 0; k < K; ++k) colacc[k] += gb[k];
             keep_snapshot(i + 2, colacc);
         }
+        if (kSumRows > 0 && ((i + 2 - i0) & (kSumRows - 1)) == 0)    // (scalar; i - i0 is even)
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                above[k * NT + tid] += static_cast<double>(colacc[k]);
+                colacc[k] = T(0);
+            }
     };
 
     T tl0 = T(0), tl1 = T(0);

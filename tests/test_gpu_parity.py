@@ -692,7 +692,7 @@ def test_grad_output_pass_of_odd_rows_half(hip, switches, h, w, dtype):
         assert torch.equal(p, q)
 
 
-@pytest.mark.parametrize("h,w", [(66, 1029), (65, 1281), (67, 1534), (64, 1536), (66, 1792)])
+@pytest.mark.parametrize("h,w", [(272, 1029), (285, 1281), (271, 1534), (272, 1536), (287, 1792)])
 def test_bands_that_make_one_round(hip, switches, h, w):
     """Rows of five to seven waves of 256 planes and filters: two long bands each, 512 workgroups, with
     snapshots and for the parameter sums alone, against the kernel with wave-strided columns (0). 1029 and 1281
@@ -700,7 +700,7 @@ def test_bands_that_make_one_round(hip, switches, h, w):
     rng = np.random.default_rng(h * w)
     C, F = 32, 8
     integ = hip.integral_image(dev(rng.standard_normal((1, C, h, w)).astype(np.float32)))
-    g = dev((rng.standard_normal((1, C * F, h, w)) + 0.25).astype(np.float32))
+    g = torch.randn(1, C * F, h, w, device="cuda", generator=torch.Generator("cuda").manual_seed(h * w)).add_(0.25)
     boxes = [dev(b) for b in make_boxes(rng, C, F, h, w, "hanging", away_from_integers=0.05)]
 
     def backward(need_input):
@@ -708,6 +708,17 @@ def test_bands_that_make_one_round(hip, switches, h, w):
                                             need_input, True, True, True, True)
     assert launches(hip, "grad_input_taps", lambda: backward(True)) == 1
     full, alone = backward(True), backward(False)
+
+    def bands():                       # sums that a call leaves per plane and filter: all that its scratch memory holds
+        hip.release_workspaces()
+        backward(False)
+        (scratch,) = hip._workspaces.values()
+        scratch.fill_(255)             # (a NaN in float64)
+        backward(False)
+        n = int(scratch.view(torch.float64).isfinite().sum())
+        assert n % (5 * C * F) == 0
+        return n // (5 * C * F)
+    assert bands() == 2
     switches("BOXCONV_STREAM_CONSEC", "0")
     ref = backward(True)
     assert (full[0] - ref[0]).abs().max() <= 4e-6 * ref[0].abs().max()
@@ -717,6 +728,28 @@ def test_bands_that_make_one_round(hip, switches, h, w):
     for p, q, r, side in zip(full[1:], alone[1:], ref[1:], (h, h, w, w)):
         assert torch.equal(p, q)
         assert (p - r).abs().max() <= 1e-5 * r.abs().max() + noise * side
+
+
+@pytest.mark.parametrize("h,w", [(272, 1029), (285, 1281), (272, 1536), (287, 1792)])
+def test_long_bands_lose_no_bits(hip, h, w):
+    """The column sums that the first backward kernel leaves for the second, over bands of up to 144 rows. Rows of
+    grad_output are multiples of 2**-18 from 1 to 1.5, so that float32 holds the sums of 32 of them exactly, but not
+    of all: a band's sum, added up in double from there on, is rounded once."""
+    rng = np.random.default_rng(h + w)
+    C, F = 32, 8
+    g = 1 + torch.randint(0, 1 << 17, (1, C * F, h, w), device="cuda").float() * 2.0 ** -18
+    boxes = [dev(b) for b in make_boxes(rng, C, F, h, w, "inside")]
+    integ = hip.integral_image(torch.randn(1, C, h, w, device="cuda"))
+    hip.release_workspaces()
+    assert launches(hip, "grad_input_taps", lambda: hip.box_convolution_backward(
+        integ, *boxes, g, None, 1.0, 1.0, True, True, True, True, True, True, True)) == 1
+    # rows of the scratch memory: zeros; per plane and filter two snapshots per group of 16 output rows, a sum per band
+    (scratch,) = hip._workspaces.values()
+    pitch, groups = (w + 3) // 4 * 4, (h + 15) // 16
+    bands = scratch.view(torch.float32)[pitch:][:C * F * (2 * groups + 2) * pitch].view(C * F, 2 * groups + 2, pitch)[:, -2:, :w]
+    first = (h + 1) // 2 + (h + 1) // 2 % 2
+    exact = torch.stack([g[0, :, :first].double().sum(1), g[0, :, first:].double().sum(1)], 1)
+    assert torch.equal(bands, exact.float())
 
 
 NARROW_SHAPES = [
