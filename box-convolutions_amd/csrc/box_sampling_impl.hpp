@@ -1551,12 +1551,15 @@ inline bool consecutive_rows(int w) {
 // grad_output_stream_kernel, both backward kernels with the column workspace / the parameter sums alone:
 //  * 129 to 192 columns 1.03 to 1.06 / 0.85 to 0.99; from 193 on 0.79 to 1.01 / 0.75 to 1.0;
 //  * but 1281 to 1536 columns, three columns per lane there, 1.0 to 1.03 with the workspace;
+//  * the sums alone of 129 to 192 columns below 2^23 output pixels, 257 to 384 below 2^22 and 513 to 640 below 2^21: 0.87 to
+//    1.09, one shape in six more than 3 % slower (9 x 10 planes of 116 x 161 in bfloat16 17.9 -> 19.4 us, 24 x 9 of 80 x 173 16.6 -> 17.8);
 //  * the sums alone of more than 1024 columns: 1.06 to 1.20 while every CU has one workgroup at most, 0.70 to
 //    0.93 with more of them (12 planes of 700 x 1279, 252 workgroups, 21.6 -> 24.6 us; 32 of 300, 288, 34.6 -> 26.7).
-inline bool odd_rows_pay(int w, int64_t workgroups, bool workspace) {
+inline bool odd_rows_pay(int w, int64_t pixels, int64_t workgroups, bool workspace) {
     if (switches().odd_rows_any_size) return true;
     if (workspace) return w > 192 && (w <= 1280 || w > 1536);
-    return w <= 1024 || workgroups > 256;
+    if (w > 1024) return workgroups > 256;
+    return pixels >= (w <= 192 ? 1 << 23 : w > 256 && w <= 384 ? 1 << 22 : w > 512 && w <= 640 ? 1 << 21 : 0);
 }
 
 // The launches of grad_output_stream_consec_kernel (workgroups of `cnt`; MODE: a StreamMode). Its instantiations are translation units of their own (BOXCONV_INST_PART 3 to
@@ -1666,7 +1669,7 @@ hipError_t grad_output_stream_launch(const T* integ, const TG* grad_out, BoxPara
     if constexpr (std::is_same<T, float>::value) {
         const int cnt = consecutive_threads(d.w);
         if (params && acc_slots > 0 && consecutive_rows(d.w) && quads_aligned(grad_out, sizeof(TG), d.w) &&
-            (d.w % 4 == 0 || snapshots != nullptr || odd_rows_pay(d.w, planes_f * sp.nb, scan))) {
+            (d.w % 4 == 0 || snapshots != nullptr || odd_rows_pay(d.w, planes_f * d.hw(), planes_f * sp.nb, scan))) {
             if (snapshots != nullptr) {
                 a.snap_shift = snapshots->shift; a.snap_groups = snapshots->groups; a.snap_bands = sp.nb;
                 return grad_output_stream_consec_launch<TG, kStreamSnapshots>(a, cnt, exact, grid, stream);

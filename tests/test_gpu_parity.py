@@ -853,6 +853,31 @@ def test_infinities_and_nan_stay_where_they_act(hip, switches, h, w, F, bad):
         assert torch.equal(a.flatten()[1:], b.flatten()[1:])
 
 
+@pytest.mark.parametrize("consecutive,planes,F,h,w", [
+    # 129 to 192 columns from 2^23 output pixels on, 257 to 384 from 2^22, 513 to 640 from 2^21, between them always; more
+    # than 1024 columns with more than 256 workgroups
+    (False, 9, 10, 116, 161), (False, 64, 10, 70, 187), (True, 64, 10, 71, 187), (True, 9, 10, 116, 193), (True, 2, 4, 100, 255),
+    (False, 8, 5, 300, 331), (True, 32, 5, 100, 331), (True, 2, 4, 100, 385), (False, 2, 2, 900, 534), (True, 8, 4, 125, 525),
+    (True, 2, 4, 100, 641), (False, 12, 1, 700, 1279), (True, 32, 1, 300, 1279)])
+def test_parameter_sums_of_odd_rows_only_where_they_pay(hip, switches, consecutive, planes, F, h, w):
+    """The launches for which consecutive columns per lane are the slower way return what BOXCONV_STREAM_CONSEC=2 returns, bit
+    for bit; the others what =3 does, and that differs."""
+    integ = hip.integral_image(torch.randn(1, planes, h, w, device="cuda"))
+    g = torch.randn(1, planes * F, h, w, device="cuda")
+    boxes = [dev(b) for b in make_boxes(np.random.default_rng(h + w), planes, F, h, w, "inside")]
+
+    def same(variant):
+        got = sums()
+        switches("BOXCONV_STREAM_CONSEC", variant)
+        result = all(torch.equal(a, b) for a, b in zip(got, sums()))
+        switches("BOXCONV_STREAM_CONSEC", None)
+        return result
+
+    def sums():
+        return hip.box_convolution_backward(integ, *boxes, g, None, 1.0, 1.0, True, True, False, True, True, True, True)[1:]
+    assert same("3" if consecutive else "2") and not same("2" if consecutive else "3")
+
+
 @pytest.mark.parametrize("narrow,planes,F,h,w", [
     # from 28 rows on; bands that leave up to a quarter (96 to 124 columns in a multiple of four) or 0.45 of the
     # lanes without rows; enough pixels for the filters, from 400 rows on more of them
@@ -992,11 +1017,11 @@ def test_integral_image_of_a_plane_per_workgroup(hip, switches, dtype, planes, h
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("planes,h,w", [(3, 28, 28), (2, 61, 51), (2, 100, 96), (3, 33, 130), (2, 190, 241), (2, 100, 256), (128, 470, 203)])
 def test_integral_image_of_infinities_and_nan(hip, dtype, planes, h, w):
-    """Lanes behind a row and bands behind the plane load pixels of the plane: an infinite one in its first column and last
-    row, a NaN in its last column, reach the entries that they are part of and no others."""
+    """Lanes behind a row and bands behind the plane load pixels of the plane: an infinite one in the first column of its last
+    row, or a NaN in the middle of that column, reaches the entries that it is part of and no others."""
     x = torch.randn(planes, h, w, device="cuda").to(dtype)
     clean = hip.integral_image(x)
-    for i, j, bad in ((h - 1, 0, float("inf")), (h // 2, 0, float("inf")), (h // 2, w - 1, float("nan"))):
+    for i, j, bad in ((h - 1, 0, float("inf")), (h // 2, 0, float("nan"))):
         y = x.clone()
         y[1, i, j] = bad
         got = hip.integral_image(y)
